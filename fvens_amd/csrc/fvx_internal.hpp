@@ -196,6 +196,23 @@ struct fvx_matrix_s {
 	void* raw() const { return prec == FVX_PREC_F32 ? (void*)v32.p : (void*)v64.p; }
 };
 
+namespace fvx {
+/// Overlapping patches of the cell graph for several symmetric Gauss-Seidel sweeps per launch
+/// (sgs_patch.hip), made when a multicolour SGS preconditioner has been applied a few times.
+struct SgsPatch {
+	int most = 0;                          // sweeps per launch the tables were chosen up to
+	double spent = 0;                      // us of applications that had no such tables
+	bool failed = false;                   // no room for the tables or the scratch vector
+	int cycles = 0;                        // sweeps one launch performs at most (0: no tables)
+	int slots = 0, npatch = 0, nhalo = 0;
+	DBuf<uint4> d_rec;
+	DBuf<int> d_halo;
+	DBuf<double> scratch;                  // [ninst][ncell][4] iterate between launches
+	hipStream_t owner = nullptr;           // stream the scratch serves since the last set-up
+	bool claimed = false;
+};
+}
+
 /// Preconditioner: factors in the matrix layout with slot 0 holding the inverted diagonal
 /// block; multicolour ordering (colour per cell, cells listed by colour, lower-colour mask).
 struct fvx_pc_s {
@@ -231,6 +248,7 @@ struct fvx_pc_s {
 	fvx::DBuf<float> v32;
 	fvx::DBuf<fvx::bf16> v16;
 	fvx::Krylov* kry = nullptr;            // FGMRES workspace of fvx_linear_solve, first use
+	mutable fvx::SgsPatch patch;
 	double* f64() const { return v64.p; }
 	float* f32() const { return v32.p; }
 	fvx::bf16* fb16() const { return v16.p; }
@@ -286,6 +304,11 @@ void launch_pseudotime(fvx_matrix_s& A, const double* dt, double cfl, double* dt
 void launch_pc_setup(fvx_pc_s& p, const fvx_matrix_s& A, const Inst& L, hipStream_t s);
 void launch_pc_apply(const fvx_pc_s& p, const double* r, long sr, double* z, long sz,
                      const Inst& L, hipStream_t s);
+/// z = M^-1 r of multicolour SGS on the patches; false where they do not apply (the caller then
+/// sweeps colour by colour, with the same bits).
+template <class VTF>
+bool sgs_patch_apply(const fvx_pc_s& p, const VTF* fac, const double* r, long sr, double* z,
+                     long sz, const Inst& L, hipStream_t s);
 int reduction_blocks();
 int max_dots();
 long partial_stride();

@@ -10,77 +10,17 @@
  * the preconditioner sweeps colour by colour. Within a colour every row depends only on rows of
  * other colours, so one launch processes a whole colour; the result equals the sequential
  * sweep over the cells sorted by (colour, index). lowmask[cell] bit k marks neighbour slot k as
- * belonging to a lower colour.
+ * belonging to a lower colour. Multicolour symmetric Gauss-Seidel runs several sweeps per launch
+ * where it can (sgs_patch.hip), with the same bits as the colour passes here.
  *
  * Reductions (dot products, norms) are deterministic: fixed grid, fixed per-thread order, fixed
  * tree within the block, then one block sums the per-block partials in order.
  */
 #include "fvx_internal.hpp"
 #include "wave.hpp"
+#include "blocks.hpp"
 
 namespace fvx {
-
-/* ----------------------------------------------------------------- block helpers ------- */
-
-template <class VT> __device__ __forceinline__ void load_row(const VT* p, double* v);
-template <> __device__ __forceinline__ void load_row<double>(const double* p, double* v)
-{
-	const double2 a = reinterpret_cast<const double2*>(p)[0];
-	const double2 b = reinterpret_cast<const double2*>(p)[1];
-	v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-}
-template <> __device__ __forceinline__ void load_row<float>(const float* p, double* v)
-{
-	const float4 a = *reinterpret_cast<const float4*>(p);
-	v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-}
-/// bfloat16 rows: 4 x 2 bytes (8-byte aligned: rows start at multiples of 4 values)
-__device__ __forceinline__ double bf16_value(unsigned int h)
-{
-	return (double)__uint_as_float(h << 16);
-}
-template <> __device__ __forceinline__ void load_row<bf16>(const bf16* p, double* v)
-{
-	const uint2 w = *reinterpret_cast<const uint2*>(p);
-	v[0] = bf16_value(w.x & 0xffffu); v[1] = bf16_value(w.x >> 16);
-	v[2] = bf16_value(w.y & 0xffffu); v[3] = bf16_value(w.y >> 16);
-}
-/// FP64 -> FP32 (rounded) -> bfloat16, rounded to nearest even; NaN stays NaN
-__device__ __forceinline__ unsigned int bf16_bits(double x)
-{
-	const unsigned int u = __float_as_uint((float)x);
-	if((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
-	return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-}
-template <class VT> __device__ __forceinline__ void put_row(VT* p, const double* v);
-template <> __device__ __forceinline__ void put_row<bf16>(bf16* p, const double* v)
-{
-	*reinterpret_cast<uint2*>(p) = make_uint2(bf16_bits(v[0]) | (bf16_bits(v[1]) << 16),
-	                                          bf16_bits(v[2]) | (bf16_bits(v[3]) << 16));
-}
-template <> __device__ __forceinline__ void put_row<double>(double* p, const double* v)
-{
-	reinterpret_cast<double2*>(p)[0] = make_double2(v[0], v[1]);
-	reinterpret_cast<double2*>(p)[1] = make_double2(v[2], v[3]);
-}
-template <> __device__ __forceinline__ void put_row<float>(float* p, const double* v)
-{
-	*reinterpret_cast<float4*>(p) = make_float4((float)v[0], (float)v[1], (float)v[2],
-	                                            (float)v[3]);
-}
-template <class VT> __device__ __forceinline__ void load_block(const VT* p, double* b)
-{
-	for(int r = 0; r < 4; r++) load_row<VT>(p + 4*r, b + 4*r);
-}
-template <class VT> __device__ __forceinline__ void put_block(VT* p, const double* b)
-{
-	for(int r = 0; r < 4; r++) put_row<VT>(p + 4*r, b + 4*r);
-}
-
-__device__ __forceinline__ double dot4(const double* a, const double* x)
-{
-	return a[0]*x[0] + a[1]*x[1] + a[2]*x[2] + a[3]*x[3];
-}
 
 /// C = A B for 4x4 row-major blocks.
 __device__ __forceinline__ void gemm4(const double* A, const double* B, double* C)
@@ -120,12 +60,6 @@ __device__ __forceinline__ void invert4(const double* a, double* inv)
 	}
 	for(int i = 0; i < 4; i++)
 		for(int j = 0; j < 4; j++) inv[i*4+j] = m[i][j+4];
-}
-
-/// Value of lane k of the quad, on every lane of the quad.
-template <int K> __device__ __forceinline__ double quad_bcast(double v)
-{
-	return dpp_d<K*0x55>(v);
 }
 
 __device__ __forceinline__ int4 load_nbr(const int* nbr, int c)
@@ -942,6 +876,7 @@ static void pc_setup_t(fvx_pc_s& p, const VTA* vals, VTF* fac, const Inst& L, hi
 		hipLaunchKernelGGL((k_invert_diag<VTA, VTF>), dim3(thread_blocks(n), L.nact), dim3(BLOCK),
 		                   0, s, n, L.list, vals, fac, sa, pc_sgs(p.type) ? 1 : 0);
 		FVX_HIP(hipGetLastError());
+		p.patch.claimed = false;
 	} else if(p.type == FVX_PC_LINE) {
 		hipLaunchKernelGGL((k_line_factor<VTA, VTF>), dim3(thread_blocks(p.nvert), L.nact),
 		                   dim3(BLOCK), 0, s, p.nvert, p.d_vptr.p, p.d_vcells.p, p.d_lineinfo.p,
@@ -1105,7 +1040,8 @@ static void pc_apply_t(const fvx_pc_s& p, const VTF* fac, const double* r, long 
                        long sz, const Inst& L, hipStream_t s)
 {
 	if(pc_sgs(p.type)) {
-		sgs_passes(p, fac, r, sr, z, sz, p.sweeps, L, s);
+		if(!sgs_patch_apply(p, fac, r, sr, z, sz, L, s))
+			sgs_passes(p, fac, r, sr, z, sz, p.sweeps, L, s);
 		return;
 	}
 	if(p.type == FVX_PC_LINE) {
