@@ -13,11 +13,21 @@
 
 namespace fvx {
 
+/// A value without derivatives beside duals: its zero derivatives cost nothing, and its quotients
+/// round like a dual's (numerator times rounded reciprocal), so that an expression has the
+/// same value whichever of its arguments carry derivatives.
+struct Val {
+	double v;
+	__host__ __device__ Val() : v(0) {}
+	__host__ __device__ Val(double x) : v(x) {}
+};
+
 template <int N> struct Dual {
 	double v;
 	double d[N];
 	__host__ __device__ Dual() : v(0) { for(int i = 0; i < N; i++) d[i] = 0; }
 	__host__ __device__ Dual(double x) : v(x) { for(int i = 0; i < N; i++) d[i] = 0; }
+	__host__ __device__ Dual(Val x) : v(x.v) { for(int i = 0; i < N; i++) d[i] = 0; }
 };
 
 #define FVX_DD template <int N> __host__ __device__ __forceinline__
@@ -82,6 +92,44 @@ FVX_DD Dual<N> pow(const Dual<N>& a, double e)
 	return r;
 }
 
+
+// Val with Val, with double and with Dual
+#define FVX_V __host__ __device__ __forceinline__
+FVX_V Val operator+(Val a, Val b) { return Val(a.v + b.v); }
+FVX_V Val operator-(Val a, Val b) { return Val(a.v - b.v); }
+FVX_V Val operator-(Val a) { return Val(-a.v); }
+FVX_V Val operator*(Val a, Val b) { return Val(a.v*b.v); }
+FVX_V Val operator/(Val a, Val b) { const double ib = 1.0/b.v; return Val(a.v*ib); }
+FVX_V Val operator+(Val a, double b) { return Val(a.v + b); }
+FVX_V Val operator+(double b, Val a) { return Val(a.v + b); }
+FVX_V Val operator-(Val a, double b) { return Val(a.v - b); }
+FVX_V Val operator-(double b, Val a) { return Val(-a.v + b); }
+FVX_V Val operator*(Val a, double b) { return Val(a.v*b); }
+FVX_V Val operator*(double b, Val a) { return Val(a.v*b); }
+FVX_V Val operator/(Val a, double b) { return Val(a.v*(1.0/b)); }
+FVX_V Val operator/(double a, Val b) { const double ib = 1.0/b.v; return Val(a*ib); }
+FVX_V Val& operator+=(Val& a, Val b) { a.v = a.v + b.v; return a; }
+FVX_V Val& operator-=(Val& a, Val b) { a.v = a.v - b.v; return a; }
+FVX_V bool operator<(Val a, Val b) { return a.v < b.v; }
+FVX_V bool operator>(Val a, Val b) { return a.v > b.v; }
+FVX_V bool operator<=(Val a, Val b) { return a.v <= b.v; }
+FVX_V bool operator>=(Val a, Val b) { return a.v >= b.v; }
+FVX_V bool operator<(Val a, double b) { return a.v < b; }
+FVX_V bool operator>(Val a, double b) { return a.v > b; }
+FVX_V bool operator<=(Val a, double b) { return a.v <= b; }
+FVX_V bool operator>=(Val a, double b) { return a.v >= b; }
+FVX_V Val sqrt(Val a) { return Val(::sqrt(a.v)); }
+FVX_V Val pow(Val a, double e) { return Val(::pow(a.v, e)); }
+#undef FVX_V
+FVX_DD Dual<N> operator+(const Dual<N>& a, Val b) { return a + b.v; }
+FVX_DD Dual<N> operator+(Val b, const Dual<N>& a) { return a + b.v; }
+FVX_DD Dual<N> operator-(const Dual<N>& a, Val b) { return a - b.v; }
+FVX_DD Dual<N> operator-(Val b, const Dual<N>& a) { return b.v - a; }
+FVX_DD Dual<N> operator*(const Dual<N>& a, Val b) { return a*b.v; }
+FVX_DD Dual<N> operator*(Val b, const Dual<N>& a) { return a*b.v; }
+FVX_DD Dual<N> operator/(const Dual<N>& a, Val b) { return a/b.v; }
+FVX_DD Dual<N> operator/(Val a, const Dual<N>& b) { return a.v/b; }
+
 #undef FVX_DD
 
 // keep the scalar overloads visible next to the dual ones inside this namespace
@@ -91,6 +139,7 @@ using ::pow;
 /// Scalar value of a double or a dual.
 __host__ __device__ __forceinline__ double value(double a) { return a; }
 template <int N> __host__ __device__ __forceinline__ double value(const Dual<N>& a) { return a.v; }
+__host__ __device__ __forceinline__ double value(Val a) { return a.v; }
 
 }
 #endif

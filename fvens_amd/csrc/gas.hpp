@@ -106,9 +106,13 @@ template <class T> FVX_HD T tsqrt(const T& a) { using std::sqrt; return sqrt(a);
 /// Roe averages (anumericalflux.hpp:175-189).
 template <class T> struct RoeAvg { T rho, v[2], vn, v2, H, c; };
 
-template <class T> FVX_HD RoeAvg<T> roe_avg(const GasParams& gp, const T* ul, const T* ur,
-                                            const double* n, const SideVars<T>& a,
-                                            const SideVars<T>& b)
+/// Scalar of a face quantity formed from both sides: double, or the dual type of the side that
+/// carries derivatives (either side may be plain double, which spares its zero derivatives).
+template <class TA, class TB> using FaceScalar = decltype(TA()*TB());
+
+template <class TA, class TB, class T = FaceScalar<TA, TB>>
+FVX_HD RoeAvg<T> roe_avg(const GasParams& gp, const TA* ul, const TB* ur, const double* n,
+                         const SideVars<TA>& a, const SideVars<TB>& b)
 {
 	RoeAvg<T> r;
 	const T R = tsqrt(ur[0]/ul[0]);
@@ -124,10 +128,11 @@ template <class T> FVX_HD RoeAvg<T> roe_avg(const GasParams& gp, const T* ul, co
 }
 
 /// Roe flux with Harten's entropy fix, delta = 1e-4 c (anumericalflux.cpp:664,667-732).
-template <class T> FVX_HD void flux_roe(const GasParams& gp, const T* ul, const T* ur,
-                                        const double* n, T* f)
+template <class TA, class TB, class T = FaceScalar<TA, TB>>
+FVX_HD void flux_roe(const GasParams& gp, const TA* ul, const TB* ur, const double* n, T* f)
 {
-	const SideVars<T> a = side_vars(gp, ul, n), b = side_vars(gp, ur, n);
+	const SideVars<TA> a = side_vars(gp, ul, n);
+	const SideVars<TB> b = side_vars(gp, ur, n);
 	const RoeAvg<T> m = roe_avg(gp, ul, ur, n, a, b);
 	T l0 = tabs(m.vn - m.c), l1 = tabs(m.vn), l3 = tabs(m.vn + m.c);
 	const T delta = 1.0e-4*m.c;
@@ -149,15 +154,17 @@ template <class T> FVX_HD void flux_roe(const GasParams& gp, const T* ul, const 
 	ad[2] = a0*(m.v[1] - m.c*n[1]) + a1*m.v[1] + a2*(dvy - dvn*n[1]) + a3*(m.v[1] + m.c*n[1]);
 	ad[3] = a0*(m.H - m.c*m.vn) + a1*m.v2*0.5 + a2*(m.v[0]*dvx + m.v[1]*dvy - m.vn*dvn)
 	        + a3*(m.H + m.c*m.vn);
-	T fa[4], fb[4];
+	TA fa[4];
+	TB fb[4];
 	phys_flux(ul, n, a.vn, a.p, fa);
 	phys_flux(ur, n, b.vn, b.p, fb);
 	for(int k = 0; k < 4; k++) f[k] = 0.5*(fa[k] + fb[k] - ad[k]);
 }
 
 /// Einfeldt signal speeds shared by HLL and HLLC (anumericalflux.cpp:990-996, 1191-1197).
-template <class T> FVX_HD void einfeldt(const T& vna, const T& ca, const T& vnb, const T& cb,
-                                        const RoeAvg<T>& m, T& sl, T& sr)
+template <class TA, class TB, class T>
+FVX_HD void einfeldt(const TA& vna, const TA& ca, const TB& vnb, const TB& cb,
+                     const RoeAvg<T>& m, T& sl, T& sr)
 {
 	sl = vna - ca;
 	if(sl > m.vn - m.c) sl = m.vn - m.c;
@@ -166,11 +173,13 @@ template <class T> FVX_HD void einfeldt(const T& vna, const T& ca, const T& vnb,
 }
 
 /// HLLC (Batten et al.) (anumericalflux.cpp:1069-1081, 1175-1228).
-template <class T> FVX_HD void flux_hllc(const GasParams& gp, const T* ul, const T* ur,
-                                         const double* n, T* f)
+template <class TA, class TB, class T = FaceScalar<TA, TB>>
+FVX_HD void flux_hllc(const GasParams& gp, const TA* ul, const TB* ur, const double* n, T* f)
 {
-	const SideVars<T> a = side_vars(gp, ul, n), b = side_vars(gp, ur, n);
-	const T ca = tsqrt(gp.g*a.p/ul[0]), cb = tsqrt(gp.g*b.p/ur[0]);
+	const SideVars<TA> a = side_vars(gp, ul, n);
+	const SideVars<TB> b = side_vars(gp, ur, n);
+	const TA ca = tsqrt(gp.g*a.p/ul[0]);
+	const TB cb = tsqrt(gp.g*b.p/ur[0]);
 	const RoeAvg<T> m = roe_avg(gp, ul, ur, n, a, b);
 	T sl, sr;
 	einfeldt(a.vn, ca, b.vn, cb, m, sl, sr);
@@ -182,20 +191,24 @@ template <class T> FVX_HD void flux_hllc(const GasParams& gp, const T* ul, const
 	else if(sl <= 0.0 && sm > 0.0) { left = true; star = true; }
 	else if(sm <= 0.0 && sr >= 0.0) { left = false; star = true; }
 	else { left = false; star = false; }
-	const T* u = left ? ul : ur;
-	const SideVars<T>& s = left ? a : b;
 	const T ss = left ? sl : sr;
-	phys_flux(u, n, s.vn, s.p, f);
-	if(star) {
-		const T pstar = u[0]*(s.vn - ss)*(s.vn - sm) + s.p;
-		const T idn = 1.0/(ss - sm);
-		T us[4];
-		us[0] = u[0]*(ss - s.vn)*idn;
-		us[1] = ((ss - s.vn)*u[1] + (pstar - s.p)*n[0])*idn;
-		us[2] = ((ss - s.vn)*u[2] + (pstar - s.p)*n[1])*idn;
-		us[3] = ((ss - s.vn)*u[3] - s.p*s.vn + pstar*sm)*idn;
-		for(int k = 0; k < 4; k++) f[k] += ss*(us[k] - u[k]);
-	}
+	// the flux of one side, in its own scalar, and what its star state adds
+	auto side = [&](const auto* u, const auto& s, auto* fs) {
+		phys_flux(u, n, s.vn, s.p, fs);
+		for(int k = 0; k < 4; k++) f[k] = fs[k];
+		if(star) {
+			const T pstar = u[0]*(s.vn - ss)*(s.vn - sm) + s.p;
+			const T idn = 1.0/(ss - sm);
+			T us[4];
+			us[0] = u[0]*(ss - s.vn)*idn;
+			us[1] = ((ss - s.vn)*u[1] + (pstar - s.p)*n[0])*idn;
+			us[2] = ((ss - s.vn)*u[2] + (pstar - s.p)*n[1])*idn;
+			us[3] = ((ss - s.vn)*u[3] - s.p*s.vn + pstar*sm)*idn;
+			for(int k = 0; k < 4; k++) f[k] += ss*(us[k] - u[k]);
+		}
+	};
+	if(left) { TA fa[4]; side(ul, a, fa); }
+	else { TB fb[4]; side(ur, b, fb); }
 }
 
 /// HLL with Einfeldt speeds (anumericalflux.cpp:973-1007).
@@ -236,13 +249,17 @@ template <class T> FVX_HD void flux_llf(const GasParams& gp, const T* ul, const 
 }
 
 /// Liou-Steffen AUSM (anumericalflux.cpp:264-315).
-template <class T> FVX_HD void flux_ausm(const GasParams& gp, const T* ul, const T* ur,
-                                         const double* n, T* f)
+template <class TA, class TB, class T = FaceScalar<TA, TB>>
+FVX_HD void flux_ausm(const GasParams& gp, const TA* ul, const TB* ur, const double* n, T* f)
 {
-	const SideVars<T> a = side_vars(gp, ul, n), b = side_vars(gp, ur, n);
-	const T ca = tsqrt(gp.g*a.p/ul[0]), cb = tsqrt(gp.g*b.p/ur[0]);
-	const T Ma = a.vn/ca, Mb = b.vn/cb;
-	T ML, MR, pL, pR;
+	const SideVars<TA> a = side_vars(gp, ul, n);
+	const SideVars<TB> b = side_vars(gp, ur, n);
+	const TA ca = tsqrt(gp.g*a.p/ul[0]);
+	const TB cb = tsqrt(gp.g*b.p/ur[0]);
+	const TA Ma = a.vn/ca;
+	const TB Mb = b.vn/cb;
+	TA ML, pL;
+	TB MR, pR;
 	if(tabs(Ma) <= 1.0) { ML = 0.25*(Ma + 1.0)*(Ma + 1.0); pL = ML*a.p*(2.0 - Ma); }
 	else if(Ma < -1.0) { ML = 0.0; pL = 0.0; }
 	else { ML = Ma; pL = a.p; }
@@ -329,8 +346,8 @@ template <class T> FVX_HD void flux_vanleer(const GasParams& gp, const T* ul, co
 	for(int k = 0; k < 4; k++) f[k] = fp[k] + fm[k];
 }
 
-template <int FLUX, class T> FVX_HD void num_flux(const GasParams& gp, const T* ul, const T* ur,
-                                                  const double* n, T* f)
+template <int FLUX, class TA, class TB, class T = FaceScalar<TA, TB>>
+FVX_HD void num_flux(const GasParams& gp, const TA* ul, const TB* ur, const double* n, T* f)
 {
 	if constexpr(FLUX == 0) flux_roe(gp, ul, ur, n, f);
 	else if constexpr(FLUX == 1) flux_hllc(gp, ul, ur, n, f);

@@ -29,15 +29,20 @@
 namespace fvx {
 
 using D4 = Dual<4>;
+using D1 = Dual<1>;
+
+/// Cells of a workgroup of `block` threads (k_jacobian).
+__host__ __device__ constexpr int jac_cells(int block) { return block == 64 ? 16 : block/8; }
 
 /// Thin-layer viscous flux of two cell states: face gradient (q_R - q_L)/|dr| along the unit
 /// centre-to-centre vector, q = (rho, vx, vy, T) (viscousphysics.cpp:124-246).
-template <class T>
+template <class TA, class TB, class T = FaceScalar<TA, TB>>
 __device__ __forceinline__ void thinlayer_flux(const GasParams& gp, const double* n,
                                                const double* xl, const double* xr,
-                                               const T* ul, const T* ur, T* vf)
+                                               const TA* ul, const TB* ur, T* vf)
 {
-	T wl[4], wr[4];
+	TA wl[4];
+	TB wr[4];
 	wl[0] = ul[0]; wl[1] = ul[1]/ul[0]; wl[2] = ul[2]/ul[0];
 	wl[3] = pressure(gp, ul)/ul[0]*gp.gM2;
 	wr[0] = ur[0]; wr[1] = ur[1]/ur[0]; wr[2] = ur[2]/ur[0];
@@ -73,40 +78,39 @@ __device__ __forceinline__ void thinlayer_flux(const GasParams& gp, const double
 	vf[3] = e;
 }
 
-/// Ghost state and du_g/du_in (row-major). Every kind except the isothermal wall is the exact
+/// Ghost state and column j of du_g/du_in. Every kind except the isothermal wall is the exact
 /// derivative of ghost_state (abc.cpp:86-140, 201-210, 228-262, 282-305, 425-437), obtained with
 /// duals; the isothermal wall uses the reference's own linearisation, including its ghost
 /// energy at the wall temperature (abc.cpp:371-409).
-__device__ __forceinline__ void ghost_jacobian(const GasParams& gp, const BCTable& bt, int bc,
-                                               const double* ui, const double* n, double* ug,
-                                               double* dug)
+__device__ __forceinline__ void ghost_column(const GasParams& gp, const BCTable& bt, int bc,
+                                             const double* ui, const double* n, int j,
+                                             double* ug, double* dug)
 {
 	if(bt.kind[bc] == 6) {
-		for(int k = 0; k < 16; k++) dug[k] = 0.0;
 		const double v0 = bt.v0[bc], v1 = bt.v1[bc];
 		const double tm = v0*ui[0];
-		ug[0] = ui[0]; dug[0] = 1.0;
-		ug[1] = 2.0*tm*n[1] - ui[1]; dug[4] = 2.0*v0*n[1]; dug[5] = -1.0;
-		ug[2] = -2.0*tm*n[0] - ui[2]; dug[8] = -2.0*v0*n[0]; dug[10] = -1.0;
+		ug[0] = ui[0];
+		ug[1] = 2.0*tm*n[1] - ui[1];
+		ug[2] = -2.0*tm*n[0] - ui[2];
 		const double m2 = ug[1]*ug[1] + ug[2]*ug[2];
 		const double ir2 = 1.0/(ui[0]*ui[0]);
 		const double vmag2 = m2*ir2;
 		const double coeff = 1.0/(gp.g*gp.gm1*gp.Minf*gp.Minf);
 		ug[3] = ui[0]*(v1*coeff + 0.5*vmag2);
 		const double dv0 = -2.0*m2*ir2/ui[0];
-		dug[12] = coeff*v1 + 0.5*(vmag2 + ui[0]*dv0);
-		dug[13] = ui[0]*0.5*(-ug[1]*ir2);
-		dug[14] = ui[0]*0.5*(-ug[2]*ir2);
-		dug[15] = 0.0;
+		dug[0] = j == 0 ? 1.0 : 0.0;
+		dug[1] = j == 0 ? 2.0*v0*n[1] : j == 1 ? -1.0 : 0.0;
+		dug[2] = j == 0 ? -2.0*v0*n[0] : j == 2 ? -1.0 : 0.0;
+		dug[3] = j == 0 ? coeff*v1 + 0.5*(vmag2 + ui[0]*dv0) : j == 1 ? ui[0]*0.5*(-ug[1]*ir2)
+		         : j == 2 ? ui[0]*0.5*(-ug[2]*ir2) : 0.0;
 		return;
 	}
-	D4 a[4], g[4];
-	for(int k = 0; k < 4; k++) { a[k] = D4(ui[k]); a[k].d[k] = 1.0; }
+	D1 a[4], g[4];
+#pragma unroll
+	for(int k = 0; k < 4; k++) { a[k] = D1(ui[k]); a[k].d[0] = k == j ? 1.0 : 0.0; }
 	ghost_state(gp, bt, bc, a, n, g);
-	for(int i = 0; i < 4; i++) {
-		ug[i] = g[i].v;
-		for(int j = 0; j < 4; j++) dug[i*4+j] = g[i].d[j];
-	}
+#pragma unroll
+	for(int i = 0; i < 4; i++) { ug[i] = g[i].v; dug[i] = g[i].d[0]; }
 }
 
 /// dF/du of the analytic directional flux (aphysics_defs.hpp:13-23), by duals.
@@ -121,24 +125,29 @@ __device__ __forceinline__ void phys_flux_jacobian(const GasParams& gp, const do
 		for(int j = 0; j < 4; j++) A[i*4+j] = f[i].d[j];
 }
 
-/// Face flux derivatives JL = dF/du_L, JR = dF/du_R of the Jacobian flux (plus the thin-layer
-/// viscous flux when VISC) at cell-centred states.
-template <int FLUX, bool VISC>
-__device__ __forceinline__ void face_jacobians(const GasParams& gp, const double* n,
-                                               const double* xl, const double* xr,
-                                               const double* ul, const double* ur,
-                                               double* JL, double* JR)
+/// Derivative dF/du of one side (SIDE 0: left, 1: right) of the Jacobian flux (plus the
+/// thin-layer viscous flux when VISC) at cell-centred states, row-major. Only the side's own
+/// variables are duals.
+template <int FLUX, bool VISC, int SIDE>
+__device__ __forceinline__ void side_jacobian(const GasParams& gp, const double* n,
+                                              const double* xl, const double* xr,
+                                              const double* ul, const double* ur, double* J)
 {
+	D4 s4[4], f[4];
+	Val o[4];
+	const double* us = SIDE == 0 ? ul : ur;
+	const double* uo = SIDE == 0 ? ur : ul;
+#pragma unroll
+	for(int k = 0; k < 4; k++) { s4[k] = D4(us[k]); s4[k].d[k] = 1.0; o[k] = Val(uo[k]); }
 	if constexpr(FLUX == 2 || FLUX == 3) {
-		phys_flux_jacobian(gp, ul, n, JL);
-		phys_flux_jacobian(gp, ur, n, JR);
+		phys_flux_jacobian(gp, us, n, J);
 		const SideVars<double> a = side_vars(gp, ul, n), b = side_vars(gp, ur, n);
 		const double ca = sqrt(gp.g*a.p/ul[0]), cb = sqrt(gp.g*b.p/ur[0]);
-		double wl, wr, dl, dr;     // JL <- wl JL + dl I, JR <- wr JR + dr I
+		double w, d;               // J <- w J + d I
 		if constexpr(FLUX == 3) {
 			const double ea = fabs(a.vn) + ca, eb = fabs(b.vn) + cb;
 			const double eig = ea >= eb ? ea : eb;
-			wl = 0.5; dl = 0.5*eig; wr = 0.5; dr = -0.5*eig;
+			w = 0.5; d = SIDE == 0 ? 0.5*eig : -0.5*eig;
 		} else {
 			const RoeAvg<double> m = roe_avg(gp, ul, ur, n, a, b);
 			double sl, sr;
@@ -146,75 +155,76 @@ __device__ __forceinline__ void face_jacobians(const GasParams& gp, const double
 			const double sr0 = sr > 0.0 ? 0.0 : sr, sl0 = sl > 0.0 ? 0.0 : sl;
 			const double t1 = (sr0 - sl0)/(sr - sl), t2 = 1.0 - t1;
 			const double t3 = 0.5*(sr*fabs(sl) - sl*fabs(sr))/(sr - sl);
-			wl = t2; dl = t3; wr = t1; dr = -t3;
+			w = SIDE == 0 ? t2 : t1; d = SIDE == 0 ? t3 : -t3;
 		}
-		for(int k = 0; k < 16; k++) { JL[k] *= wl; JR[k] *= wr; }
-		for(int i = 0; i < 4; i++) { JL[i*5] += dl; JR[i*5] += dr; }
+#pragma unroll
+		for(int k = 0; k < 16; k++) J[k] *= w;
+#pragma unroll
+		for(int i = 0; i < 4; i++) J[i*5] += d;
 		if constexpr(VISC) {
-			for(int side = 0; side < 2; side++) {
-				D4 a4[4], b4[4], vf[4];
-				for(int k = 0; k < 4; k++) {
-					a4[k] = D4(ul[k]); b4[k] = D4(ur[k]);
-					if(side == 0) a4[k].d[k] = 1.0; else b4[k].d[k] = 1.0;
-				}
-				thinlayer_flux(gp, n, xl, xr, a4, b4, vf);
-				double* J = side == 0 ? JL : JR;
-				for(int i = 0; i < 4; i++)
-					for(int j = 0; j < 4; j++) J[i*4+j] += vf[i].d[j];
-			}
+			if constexpr(SIDE == 0) thinlayer_flux(gp, n, xl, xr, s4, o, f);
+			else thinlayer_flux(gp, n, xl, xr, o, s4, f);
+#pragma unroll
+			for(int i = 0; i < 4; i++)
+#pragma unroll
+				for(int j = 0; j < 4; j++) J[i*4+j] += f[i].d[j];
 		}
 	} else {
-		for(int side = 0; side < 2; side++) {
-			D4 a4[4], b4[4], f[4];
-			for(int k = 0; k < 4; k++) {
-				a4[k] = D4(ul[k]); b4[k] = D4(ur[k]);
-				if(side == 0) a4[k].d[k] = 1.0; else b4[k].d[k] = 1.0;
-			}
-			num_flux<FLUX>(gp, a4, b4, n, f);
-			if constexpr(VISC) {
-				D4 vf[4];
-				thinlayer_flux(gp, n, xl, xr, a4, b4, vf);
-				for(int k = 0; k < 4; k++) f[k] += vf[k];
-			}
-			double* J = side == 0 ? JL : JR;
-			for(int i = 0; i < 4; i++)
-				for(int j = 0; j < 4; j++) J[i*4+j] = f[i].d[j];
+		if constexpr(SIDE == 0) num_flux<FLUX>(gp, s4, o, n, f);
+		else num_flux<FLUX>(gp, o, s4, n, f);
+		if constexpr(VISC) {
+			D4 vf[4];
+			if constexpr(SIDE == 0) thinlayer_flux(gp, n, xl, xr, s4, o, vf);
+			else thinlayer_flux(gp, n, xl, xr, o, s4, vf);
+#pragma unroll
+			for(int k = 0; k < 4; k++) f[k] += vf[k];
 		}
+#pragma unroll
+		for(int i = 0; i < 4; i++)
+#pragma unroll
+			for(int j = 0; j < 4; j++) J[i*4+j] = f[i].d[j];
 	}
 }
 
-/// Total derivative d/du_L of F(u_L, u_g(u_L)) at a boundary face.
+/// Column j of the total derivative d/du_L of F(u_L, u_g(u_L)) at a boundary face.
 template <int FLUX, bool VISC>
-__device__ __forceinline__ void boundary_jacobian(const GasParams& gp, const BCTable& bt, int bc,
-                                                  const double* n, const double* xl,
-                                                  const double* xg, const double* ul, double* J)
+__device__ __forceinline__ void boundary_column(const GasParams& gp, const BCTable& bt, int bc,
+                                                const double* n, const double* xl,
+                                                const double* xg, const double* ul, int j,
+                                                double* col)
 {
-	double ug[4], dug[16];
-	ghost_jacobian(gp, bt, bc, ul, n, ug, dug);
+	double ug[4], dug[4];
+	ghost_column(gp, bt, bc, ul, n, j, ug, dug);
 	if constexpr(FLUX == 2 || FLUX == 3) {
 		double JL[16], JR[16];
-		face_jacobians<FLUX, VISC>(gp, n, xl, xg, ul, ug, JL, JR);
-		for(int i = 0; i < 4; i++)
-			for(int j = 0; j < 4; j++) {
-				double s = 0.0;
-				for(int k = 0; k < 4; k++) s += JR[i*4+k]*dug[k*4+j];
-				J[i*4+j] = JL[i*4+j] + s;
-			}
-	} else {
-		D4 a4[4], g4[4], f[4];
+		side_jacobian<FLUX, VISC, 0>(gp, n, xl, xg, ul, ug, JL);
+		side_jacobian<FLUX, VISC, 1>(gp, n, xl, xg, ul, ug, JR);
+#pragma unroll
 		for(int i = 0; i < 4; i++) {
-			a4[i] = D4(ul[i]); a4[i].d[i] = 1.0;
-			g4[i] = D4(ug[i]);
-			for(int j = 0; j < 4; j++) g4[i].d[j] = dug[i*4+j];
+			double s = 0.0;
+#pragma unroll
+			for(int k = 0; k < 4; k++) s += JR[i*4+k]*dug[k];
+			double v = JL[i*4];
+#pragma unroll
+			for(int k = 1; k < 4; k++) v = j == k ? JL[i*4+k] : v;
+			col[i] = v + s;
 		}
-		num_flux<FLUX>(gp, a4, g4, n, f);
+	} else {
+		D1 a[4], g[4], f[4];
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			a[i] = D1(ul[i]); a[i].d[0] = i == j ? 1.0 : 0.0;
+			g[i] = D1(ug[i]); g[i].d[0] = dug[i];
+		}
+		num_flux<FLUX>(gp, a, g, n, f);
 		if constexpr(VISC) {
-			D4 vf[4];
-			thinlayer_flux(gp, n, xl, xg, a4, g4, vf);
+			D1 vf[4];
+			thinlayer_flux(gp, n, xl, xg, a, g, vf);
+#pragma unroll
 			for(int k = 0; k < 4; k++) f[k] += vf[k];
 		}
-		for(int i = 0; i < 4; i++)
-			for(int j = 0; j < 4; j++) J[i*4+j] = f[i].d[j];
+#pragma unroll
+		for(int i = 0; i < 4; i++) col[i] = f[i].d[0];
 	}
 }
 
@@ -230,11 +240,22 @@ template <> __device__ __forceinline__ void store_row<float>(float* p, const dou
 	                                            (float)v[3]);
 }
 
-/// One quad of lanes per cell; lane q owns local face q. When dt is given the pseudo-time term
-/// area/(cfl dt) is added to the diagonal and stored in dtm (SteadyBackwardEulerSolver::
-/// addPseudoTimeTerm, src/ode/aodesolver.cpp:300-329).
+/// A pair of waves per 16 cells: the quad of lanes of a cell owns its four faces in both, one
+/// wave differentiates the faces by their left states, the other by their right ones (a
+/// workgroup of one wave does both in turn), and the derivatives meet in LDS, from where the
+/// rows are written. When dt is given the pseudo-time term area/(cfl dt) is added to
+/// the diagonal and stored in dtm (SteadyBackwardEulerSolver::addPseudoTimeTerm,
+/// src/ode/aodesolver.cpp:300-329).
+///
+/// Bound by FP64 VALU work and its latency: ~1,000 instructions a face and side at two waves per
+/// SIMD (204-228 registers). One lane differentiating both sides in turn, all variables duals,
+/// needed 290-380 registers and spilled. Assembly on 98,304 cells, FP64, workgroups of 64: Roe
+/// 120 -> 43 us, HLLC 74 -> 44 us; 4,608 cells, workgroups of 256: Roe 25 -> 12 us, HLLC 19 -> 12
+/// us. Held to three waves per SIMD, HLLC spills 140 bytes (48 us). Boundary faces go column by
+/// column, their four columns on the cell's four lanes: with all columns on one lane the boundary
+/// code, both sides duals, would set the kernel's registers.
 template <int FLUX, bool VISC, class VT>
-__global__ __launch_bounds__(BLOCK)
+__global__ __launch_bounds__(BLOCK, 2)
 void k_jacobian(int ncell, const double* __restrict__ u, const int* __restrict__ nbr,
                 const int* __restrict__ face, const FaceGeom* __restrict__ fgeom,
                 const double* __restrict__ centre, const int* __restrict__ bcid,
@@ -253,59 +274,98 @@ void k_jacobian(int ncell, const double* __restrict__ u, const int* __restrict__
 	u += I*4L*ncell;
 	vals += I*80L*ncell;
 	if(dt) { dt += I*(long)ncell; dtm += I*(long)ncell; }
-	const int q = threadIdx.x & 3;
-	const int cell = xcd_block(xcd)*(int)(blockDim.x >> 2) + (threadIdx.x >> 2);
-	const bool valid = cell < ncell;
-	const int cc = valid ? cell : 0;
-	const int nb = nbr[cc*4 + q];
-	const bool act = valid && nb != SLOT_UNUSED;
-
-	double Jd[16], Jo[16];
-	for(int k = 0; k < 16; k++) { Jd[k] = 0.0; Jo[k] = 0.0; }
-	if(act) {
-		const FaceGeom G = fgeom[face[cc*4 + q]];
+	// LDS: per side, block entry and (cell, face) the derivatives -- two doubles of padding per
+	// entry spread the rows of a block, four entries apart, over the banks --, and the side of
+	// the cell's own state (2 boundary: its derivatives are under side 0; 3 none)
+	extern __shared__ double lds[];
+	const int cpb = jac_cells(blockDim.x), F = 4*cpb, S = F + 2;
+	unsigned char* skind = reinterpret_cast<unsigned char*>(lds + 32*S);
+	auto sj = [&](int side, int k, int f) -> double& { return lds[(16*side + k)*S + f]; };
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	const bool both = blockDim.x == 64;
+	const bool left = both || (wave & 1) == 0, right = both || (wave & 1) == 1;
+	const int slot = (both ? 0 : (wave >> 1)*64) + lane;      // 4 cell + face
+	const int c0 = xcd_block(xcd)*cpb;
+	const int cell = c0 + (slot >> 2), q = slot & 3;
+	const int nb = cell < ncell ? nbr[cell*4 + q] : SLOT_UNUSED;
+	const bool selfL = nb < 0 || cell < nb;
+	if(left) skind[slot] = nb == SLOT_UNUSED ? 3 : nb < 0 ? 2 : selfL ? 0 : 1;
+	if(nb >= 0) {
+		const FaceGeom G = fgeom[face[cell*4 + q]];
 		const double n[2] = { G.nx, G.ny };
-		double uo[4], xo[2];
-		load4(u + 4*cc, uo);
-		xo[0] = centre[2*cc]; xo[1] = centre[2*cc+1];
-		if(nb < 0) {
-			const int bc = bcid[-1 - nb];
-			const double xg[2] = { 2.0*G.mx - xo[0], 2.0*G.my - xo[1] };
-			boundary_jacobian<FLUX, VISC>(gp, bt, bc, n, xo, xg, uo, Jd);
-			for(int k = 0; k < 16; k++) Jd[k] *= G.len;
-		} else {
-			double un[4], xn[2];
-			load4(u + 4*nb, un);
-			xn[0] = centre[2*nb]; xn[1] = centre[2*nb+1];
-			const bool selfL = cc < nb;
-			double JL[16], JR[16];
-			if(selfL) face_jacobians<FLUX, VISC>(gp, n, xo, xn, uo, un, JL, JR);
-			else      face_jacobians<FLUX, VISC>(gp, n, xn, xo, un, uo, JL, JR);
-			const double s = selfL ? G.len : -G.len;
-			for(int k = 0; k < 16; k++) {
-				Jd[k] = s*(selfL ? JL[k] : JR[k]);
-				Jo[k] = s*(selfL ? JR[k] : JL[k]);
-			}
+		const int cl = selfL ? cell : nb, cr = selfL ? nb : cell;
+		double ul[4], ur[4], xl[2] = {0, 0}, xr[2] = {0, 0}, J[16];
+		load4(u + 4*cl, ul);
+		load4(u + 4*cr, ur);
+		if constexpr(VISC) {
+			xl[0] = centre[2*cl]; xl[1] = centre[2*cl+1];
+			xr[0] = centre[2*cr]; xr[1] = centre[2*cr+1];
+		}
+		const double sgn = selfL ? G.len : -G.len;
+		if(left) {
+			side_jacobian<FLUX, VISC, 0>(gp, n, xl, xr, ul, ur, J);
+#pragma unroll
+			for(int k = 0; k < 16; k++) sj(0, k, slot) = sgn*J[k];
+		}
+		if(right) {
+			side_jacobian<FLUX, VISC, 1>(gp, n, xl, xr, ul, ur, J);
+#pragma unroll
+			for(int k = 0; k < 16; k++) sj(1, k, slot) = sgn*J[k];
 		}
 	}
-	for(int k = 0; k < 16; k++) Jd[k] = quad_sum(Jd[k]);
-	if(!valid) return;
-	double add = 0.0;
-	if(dt) {
-		add = area[cc]/(cfl*dt[cc]);
-		if(q == 0) dtm[cc] = add;
+	// boundary faces: the cell's four lanes take a column each; even faces in the left wave, odd
+	// ones in the right
+	for(int k = 0; k < 4; k++) {
+		const int nk = __shfl(nb, (lane & ~3) + k);
+		if(nk >= 0 || nk == SLOT_UNUSED || !((k & 1) ? right : left)) continue;
+		const FaceGeom G = fgeom[-1 - nk];       // boundary faces are numbered first
+		const double n[2] = { G.nx, G.ny };
+		double ul[4], xl[2] = {0, 0}, xg[2] = {0, 0}, col[4];
+		load4(u + 4*cell, ul);
+		if constexpr(VISC) {
+			xl[0] = centre[2*cell]; xl[1] = centre[2*cell+1];
+			xg[0] = 2.0*G.mx - xl[0]; xg[1] = 2.0*G.my - xl[1];
+		}
+		boundary_column<FLUX, VISC>(gp, bt, bcid[-1 - nk], n, xl, xg, ul, q, col);
+#pragma unroll
+		for(int i = 0; i < 4; i++) sj(0, 4*i + q, (slot & ~3) + k) = col[i]*G.len;
 	}
-	double row[4];
-	for(int j = 0; j < 4; j++) {
-		// row q of the diagonal block, selected without dynamic register indexing
-		double v = Jd[j];
-		for(int r = 1; r < 4; r++) v = q == r ? Jd[r*4+j] : v;
-		row[j] = v + (j == q ? add : 0.0);
+	__syncthreads();
+	const int nc = min(cpb, ncell - c0);
+	// the neighbours' blocks: row r of slot 1 + k
+	for(int t = threadIdx.x; t < 16*nc; t += blockDim.x) {
+		const int f = t >> 2, r = t & 3, kind = skind[f];
+		double row[4];
+#pragma unroll
+		for(int j = 0; j < 4; j++) {
+			const double v = sj(kind == 0 ? 1 : 0, 4*r + j, f);
+			row[j] = kind < 2 ? v : 0.0;
+		}
+		store_row<VT>(vals + (size_t)(c0 + (f >> 2))*80 + 16*(1 + (f & 3)) + 4*r, row);
 	}
-	VT* blk = vals + (size_t)cc*80;
-	store_row<VT>(blk + 4*q, row);
-	VT* off = blk + 16*(1 + q);
-	for(int r = 0; r < 4; r++) store_row<VT>(off + 4*r, Jo + 4*r);
+	// the diagonal block: the own sides of the four faces, in the order (0 + 1) + (2 + 3)
+	for(int t = threadIdx.x; t < 4*nc; t += blockDim.x) {
+		const int lc = t >> 2, r = t & 3, c = c0 + lc;
+		double v[4][4];
+#pragma unroll
+		for(int k = 0; k < 4; k++) {
+			const int kind = skind[4*lc + k];
+#pragma unroll
+			for(int j = 0; j < 4; j++) {
+				const double a = sj(kind == 1 ? 1 : 0, 4*r + j, 4*lc + k);
+				v[k][j] = kind == 3 ? 0.0 : a;
+			}
+		}
+		double add = 0.0, row[4];
+		if(dt) {
+			add = area[c]/(cfl*dt[c]);
+			if(r == 0) dtm[c] = add;
+		}
+#pragma unroll
+		for(int j = 0; j < 4; j++)
+			row[j] = ((v[0][j] + v[1][j]) + (v[2][j] + v[3][j])) + (j == r ? add : 0.0);
+		store_row<VT>(vals + (size_t)c*80 + 4*r, row);
+	}
 }
 
 template <int FLUX, bool VISC>
@@ -315,15 +375,16 @@ static void launch_jac_t(const fvx_disc_s& d, const double* u, void* vals, int p
 {
 	const fvx_mesh_s* m = d.m;
 	const int n = m->nelem;
-	const int block = d.tune.jac_block, cpb = block/4;
+	const int block = d.tune.jac_block, cpb = jac_cells(block);
 	const dim3 g((n + cpb - 1)/cpb, nact);
+	const size_t lds = 32*(4*(size_t)cpb + 2)*sizeof(double) + 4*(size_t)cpb;
 	if(prec == FVX_PREC_F32)
-		hipLaunchKernelGGL((k_jacobian<FLUX, VISC, float>), g, dim3(block), 0, s, n, u,
+		hipLaunchKernelGGL((k_jacobian<FLUX, VISC, float>), g, dim3(block), lds, s, n, u,
 		                   m->d_nbr.p, m->d_face.p, m->d_fgeom.p, m->d_centre.p, d.d_bcid.p,
 		                   ba.gp ? ba.gp : d.d_gas.p, d.d_bct.p, ba, static_cast<float*>(vals), dt,
 		                   m->d_area.p, cfl, dtm, d.tune.jac_xcd);
 	else
-		hipLaunchKernelGGL((k_jacobian<FLUX, VISC, double>), g, dim3(block), 0, s, n, u,
+		hipLaunchKernelGGL((k_jacobian<FLUX, VISC, double>), g, dim3(block), lds, s, n, u,
 		                   m->d_nbr.p, m->d_face.p, m->d_fgeom.p, m->d_centre.p, d.d_bcid.p,
 		                   ba.gp ? ba.gp : d.d_gas.p, d.d_bct.p, ba, static_cast<double*>(vals),
 		                   dt, m->d_area.p, cfl, dtm, d.tune.jac_xcd);

@@ -725,6 +725,10 @@ void build_disc(fvx_disc_s& d)
 	// wave64 group on average (compact orders: Hilbert, structured natural orders); it spends
 	// fewer than 2.7 face evaluations per cell there against the quad form's 4 lanes per cell
 	d.tune.flux_wave = flux_wave_apply(d) && (long)m.nelem >= 24L*m.nwgroup;
+	// Jacobian assembly: workgroups of one wave (both sides of a face in turn) where they fill the
+	// chip several times over, else a pair of waves per 16 cells (98,304 cells 43 against 50 us,
+	// 4,608 cells 15 against 12 us; Roe)
+	d.tune.jac_block = m.nelem >= 32768 ? 64 : 256;
 }
 
 }
