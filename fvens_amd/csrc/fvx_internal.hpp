@@ -314,24 +314,24 @@ int max_dots();
 long partial_stride();
 void launch_mdot(long N, const double* V, long ldv, long sv, int nv, const double* w, long sw,
                  double* partial, double* out, long so, const Inst& L, hipStream_t s);
-void launch_gs_update(long N, const double* V, long ldv, long sv, int nv, const double* h,
-                      long sh, double* w, long sw, double* partial, double* nrm2, long sn,
-                      const Inst& L, hipStream_t s);
-void launch_scale(long N, const double* b, long sb, const double* nrm2, long sn, double* out,
-                  long so, const Inst& L, hipStream_t s);
-void launch_lincomb(long N, const double* Z, long ldz, long sz, int nv, const double* y,
-                    long sy, double* x, long sx, const Inst& L, hipStream_t s,
-                    const int* nvi = nullptr);
-/// Device least squares of FGMRES (linalg.hip): state doubles per instance and the launchers
-/// of the cycle start, the per-step rotation and the cycle end.
+/// Partial sums of |b|^2 (npart: reduction_blocks() per instance).
+void launch_sqnorm(long N, const double* b, long sb, double* npart, const Inst& L, hipStream_t s);
+/// One Arnoldi step from z: w = A z (A null: w already holds the operator's result), h_i = V_i . w,
+/// w -= sum h_i V_i, partial sums of |w|^2.
+void launch_arnoldi(long N, const fvx_matrix_s* A, const double* z, long sz, const double* V,
+                    long ldv, long sv, int nv, double* w, long sw, double* partial, double* npart,
+                    double* h, long sh, const Inst& L, hipStream_t s);
+/// FGMRES on the device (linalg.hip): state doubles per instance; the normalisation of a basis
+/// vector together with the least squares of step j (j < 0: the cycle start), h_r of the step in
+/// scal[I][r], the partial sums of the squared norm in npart (its sum goes to scal[I][slot]); the
+/// cycle end.
 long fgmres_state_size();
-void launch_fgmres_begin(int nids, const int* ids, const double* scal, long ns, int beta_slot,
-                         double* kst, int* list, int* hcount, hipStream_t s);
-void launch_fgmres_rotate(int j, double rtol, int nids, const int* ids, const double* scal,
-                          long ns, int h_slot, int nrm_slot, double* kst, int* list,
-                          int* hcount, hipStream_t s);
-void launch_fgmres_end(int nids, const int* ids, const double* kst, double* scal, long ns,
-                       int y_slot, int* its, hipStream_t s);
+void launch_scale_rotate(long N, const double* b, long sb, const double* npart, double* scal,
+                         long ns, int slot, double* out, long so, int j, double rtol, int nids,
+                         const int* ids, double* kst, int* next, int* hcount, const Inst& L,
+                         hipStream_t s);
+void launch_solution(long N, const double* Z, long ldz, long sz, const double* kst, double* x,
+                     long sx, int* its, const Inst& L, hipStream_t s);
 void launch_resnorm(int n, const double* r, const double* area, double* partial, double* out,
                     long so, const Inst& L, hipStream_t s);
 void launch_zero(long N, double* x, long sx, const Inst& L, hipStream_t s);

@@ -19,6 +19,7 @@
 #include "fvx_internal.hpp"
 #include "wave.hpp"
 #include "blocks.hpp"
+#include <algorithm>
 
 namespace fvx {
 
@@ -139,7 +140,11 @@ void k_pseudotime(int n, VT* __restrict__ vals, const double* __restrict__ dt,
 /* ---------------------------------------------------------- preconditioners ------------ */
 
 /// Inverts the diagonal block of every cell into fac slot 0; with copy_off, also copies the
-/// off-diagonal blocks (symmetric Gauss-Seidel sweeps read them from the factor array).
+/// off-diagonal blocks (symmetric Gauss-Seidel sweeps read them from the factor array). A
+/// workgroup serves 64 cells: its first wave inverts, one cell per lane, while the others copy
+/// rows in memory order. Bound by the inversion's chain of dependent FP64 operations on small
+/// meshes and by HBM on large ones; with the copy done by the inverting lane, block after block,
+/// 17 us on 4,608 cells and 28 us on 98,304 (FP64 from FP64).
 template <class VTA, class VTF>
 __global__ __launch_bounds__(BLOCK)
 void k_invert_diag(int n, const int* __restrict__ ilist, const VTA* __restrict__ vals,
@@ -148,17 +153,22 @@ void k_invert_diag(int n, const int* __restrict__ ilist, const VTA* __restrict__
 	const long I = inst_of(ilist);
 	if(I < 0) return;                     // a retired slot of a compacted list
 	vals += I*sa; fac += I*sa;
-	const int c = blockIdx.x*blockDim.x + threadIdx.x;
-	if(c >= n) return;
-	double a[16], inv[16];
-	load_block<VTA>(vals + (size_t)c*80, a);
-	invert4(a, inv);
-	put_block<VTF>(fac + (size_t)c*80, inv);
-	if(copy_off)
-		for(int s = 1; s < 5; s++) {
-			load_block<VTA>(vals + (size_t)c*80 + 16*s, a);
-			put_block<VTF>(fac + (size_t)c*80 + 16*s, a);
+	const int c0 = xcd_block()*CELLS_PER_BLOCK, nc = min(CELLS_PER_BLOCK, n - c0);
+	const int t = threadIdx.x;
+	if(t < 64) {
+		if(t >= nc) return;
+		double a[16], inv[16];
+		load_block<VTA>(vals + (size_t)(c0 + t)*80, a);
+		invert4(a, inv);
+		put_block<VTF>(fac + (size_t)(c0 + t)*80, inv);
+	} else if(copy_off) {
+		for(int r = t - 64; r < 16*nc; r += BLOCK - 64) {
+			const size_t at = (size_t)(c0 + (r >> 4))*80 + 16 + 4*(r & 15);
+			double a[4];
+			load_row<VTA>(vals + at, a);
+			put_row<VTF>(fac + at, a);
 		}
+	}
 }
 
 /// z = D^-1 r, one quad per cell.
@@ -588,6 +598,7 @@ void k_bj_ilu_apply(const int* __restrict__ bptr, const int* __restrict__ blvptr
 constexpr int RED_BLOCKS = 512;
 constexpr int MAX_DOTS = 32;
 constexpr long PART = (long)RED_BLOCKS*MAX_DOTS;   // per-instance partial-sum stride
+constexpr int FOLD_BLOCKS = 512;                   // see fold()
 
 /// Sum over the 256 threads of a block; the result is valid in every thread.
 __device__ __forceinline__ double block_sum(double v, double* sh)
@@ -600,30 +611,34 @@ __device__ __forceinline__ double block_sum(double v, double* sh)
 	return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-/// partial[b][i] = block b's part of dot(V_i, w), i < nv <= NVM (V_i = V + i*ldv). The NVM
-/// accumulators are indexed by compile-time constants only, so they stay in registers; each
-/// wave reduces all of them, then one barrier, then thread i adds the four waves' parts of dot
-/// i in the fixed order (w0 + w1) + (w2 + w3).
-template <int NVM>
-__global__ __launch_bounds__(BLOCK)
-void k_mdot(long N, const int* __restrict__ ilist, const double* __restrict__ V, long ldv,
-            long sv, int nv, const double* __restrict__ w, long sw, double* __restrict__ partial)
+/// Sum of nblk <= 512 partials `stride` apart by one wave: what a workgroup of 256 threads, each
+/// adding every 256th, would give (its four waves' sums one after the other, then added in pairs).
+__device__ __forceinline__ double wave_reduce(const double* __restrict__ partial, int stride,
+                                              int nblk)
 {
-	const long I = inst_of(ilist);
-	if(I < 0) return;                     // a retired slot of a compacted list
-	V += I*sv; w += I*sw; partial += I*PART;
+	const int lane = threadIdx.x & 63;
+	double s[4];
+#pragma unroll
+	for(int w = 0; w < 4; w++) {
+		double v = 0.0;
+		if(64*w < nblk) {
+			for(int b = 64*w + lane; b < nblk; b += 256) v += partial[(size_t)b*stride];
+			for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+		}
+		s[w] = v;
+	}
+	return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+/// Partial sums of nv dots from the threads' accumulators: each wave reduces all of them, then
+/// one barrier, then thread i adds the four waves' parts of dot i in the fixed order
+/// (w0 + w1) + (w2 + w3).
+template <int NVM>
+__device__ __forceinline__ void finish_dots(const double (&acc)[NVM], int nv, int blk,
+                                            double* __restrict__ partial)
+{
 	static_assert(BLOCK == 256, "the final sum adds four waves' parts");
 	__shared__ double sh[BLOCK/64][NVM];
-	double acc[NVM];
-#pragma unroll
-	for(int i = 0; i < NVM; i++) acc[i] = 0.0;
-	const long stride = (long)gridDim.x*blockDim.x;
-	for(long e = (long)blockIdx.x*blockDim.x + threadIdx.x; e < N; e += stride) {
-		const double we = w[e];
-#pragma unroll
-		for(int i = 0; i < NVM; i++)
-			if(i < nv) acc[i] += V[i*ldv + e]*we;
-	}
 	const int wv = threadIdx.x >> 6;
 #pragma unroll
 	for(int i = 0; i < NVM; i++) {
@@ -636,7 +651,70 @@ void k_mdot(long N, const int* __restrict__ ilist, const double* __restrict__ V,
 	__syncthreads();
 	const int t = threadIdx.x;
 	if(t < nv)
-		partial[(size_t)blockIdx.x*MAX_DOTS + t] = (sh[0][t] + sh[1][t]) + (sh[2][t] + sh[3][t]);
+		partial[(size_t)blk*MAX_DOTS + t] = (sh[0][t] + sh[1][t]) + (sh[2][t] + sh[3][t]);
+}
+
+/// partial[b][i] = block b's part of dot(V_i, w), i < nv <= NVM (V_i = V + i*ldv). The NVM
+/// accumulators are indexed by compile-time constants only, so they stay in registers.
+template <int NVM>
+__global__ __launch_bounds__(BLOCK)
+void k_mdot(long N, const int* __restrict__ ilist, const double* __restrict__ V, long ldv,
+            long sv, int nv, const double* __restrict__ w, long sw, double* __restrict__ partial)
+{
+	const long I = inst_of(ilist);
+	if(I < 0) return;                     // a retired slot of a compacted list
+	V += I*sv; w += I*sw; partial += I*PART;
+	double acc[NVM];
+#pragma unroll
+	for(int i = 0; i < NVM; i++) acc[i] = 0.0;
+	const long stride = (long)gridDim.x*blockDim.x;
+	for(long e = (long)blockIdx.x*blockDim.x + threadIdx.x; e < N; e += stride) {
+		const double we = w[e];
+#pragma unroll
+		for(int i = 0; i < NVM; i++)
+			if(i < nv) acc[i] += V[i*ldv + e]*we;
+	}
+	finish_dots<NVM>(acc, nv, blockIdx.x, partial);
+}
+
+/// y = A x and the dots of y with V_0 .. V_{nv-1} in one pass, for meshes of at most 64 cells per
+/// partial sum (each workgroup's 64 cells are the 256 values k_mdot gives the same block).
+template <class VT, int NVM>
+__global__ __launch_bounds__(BLOCK)
+void k_spmv_mdot(int n, const int* __restrict__ ilist, const VT* __restrict__ vals, long sa,
+                 const int* __restrict__ nbr, const double* __restrict__ x, long sx,
+                 double* __restrict__ y, long sy, const double* __restrict__ V, long ldv, long sv,
+                 int nv, double* __restrict__ partial)
+{
+	const long I = inst_of(ilist);
+	if(I < 0) return;                     // a retired slot of a compacted list
+	vals += I*sa; x += I*sx; y += I*sy; V += I*sv; partial += I*PART;
+	const int blk = xcd_block();
+	const int q = threadIdx.x & 3, c = blk*CELLS_PER_BLOCK + (threadIdx.x >> 2);
+	double acc[NVM];
+#pragma unroll
+	for(int i = 0; i < NVM; i++) acc[i] = 0.0;
+	if(c < n) {
+		const int4 nb = load_nbr(nbr, c);
+		const int nbs[4] = { nb.x, nb.y, nb.z, nb.w };
+		const VT* blkp = vals + (size_t)c*80 + 4*q;
+		double a[4], xv[4];
+		load_row<VT>(blkp, a);
+		load4(x + 4*c, xv);
+		double s = dot4(a, xv);
+		for(int k = 0; k < 4; k++) {
+			if(nbs[k] < 0) continue;
+			load_row<VT>(blkp + 16*(1 + k), a);
+			load4(x + 4*nbs[k], xv);
+			s += dot4(a, xv);
+		}
+		const long e = 4L*c + q;
+		y[e] = s;
+#pragma unroll
+		for(int i = 0; i < NVM; i++)
+			if(i < nv) acc[i] += V[i*ldv + e]*s;
+	}
+	finish_dots<NVM>(acc, nv, blk, partial);
 }
 
 /// out[i] = sum over blocks of partial[b][i], i < nv (one block per instance, fixed order).
@@ -647,28 +725,45 @@ void k_reduce(int nblk, const int* __restrict__ ilist, const double* __restrict_
 	const long I = inst_of(ilist);
 	if(I < 0) return;                     // a retired slot of a compacted list
 	partial += I*PART; out += I*so;
-	__shared__ double sh[4];
-	for(int i = 0; i < nv; i++) {
-		double v = 0.0;
-		for(int b = threadIdx.x; b < nblk; b += blockDim.x) v += partial[(size_t)b*MAX_DOTS + i];
-		const double s = block_sum(v, sh);
-		if(threadIdx.x == 0) out[i] = s;
-		__syncthreads();
+	for(int i = threadIdx.x >> 6; i < nv; i += BLOCK/64) {
+		const double s = wave_reduce(partial + i, MAX_DOTS, nblk);
+		if((threadIdx.x & 63) == 0) out[i] = s;
 	}
 }
 
-/// w -= sum_i h_i V_i (classical Gram-Schmidt update) and partial[b][0] = block part of |w|^2.
-__global__ __launch_bounds__(BLOCK)
-void k_gs_update(long N, const int* __restrict__ ilist, const double* __restrict__ V, long ldv,
-                 long sv, int nv, const double* __restrict__ h, long sh_, double* __restrict__ w,
-                 long sw, double* __restrict__ partial)
+/// *nrm2 = sum of the nblk partials npart (one wave per instance).
+__global__ __launch_bounds__(64)
+void k_reduce_norm(int nblk, const int* __restrict__ ilist, const double* __restrict__ npart,
+                   double* __restrict__ nrm2, long sn)
 {
 	const long I = inst_of(ilist);
 	if(I < 0) return;                     // a retired slot of a compacted list
-	V += I*sv; h += I*sh_; w += I*sw; partial += I*PART;
+	const double s = wave_reduce(npart + I*RED_BLOCKS, 1, nblk);
+	if(threadIdx.x == 0) nrm2[I*sn] = s;
+}
+
+/// w -= sum_i h_i V_i (classical Gram-Schmidt update); npart[b] = block b's part of |w|^2. With hblk
+/// > 0 the h_i are still hblk partial sums (k_mdot): every workgroup adds them for itself, the
+/// first also stores them in h.
+__global__ __launch_bounds__(BLOCK)
+void k_gs_update(long N, const int* __restrict__ ilist, const double* __restrict__ V, long ldv,
+                 long sv, int nv, const double* __restrict__ hpart, int hblk, double* h, long sh_,
+                 double* __restrict__ w, long sw, double* __restrict__ npart)
+{
+	const long I = inst_of(ilist);
+	if(I < 0) return;                     // a retired slot of a compacted list
+	V += I*sv; h += I*sh_; w += I*sw; hpart += I*PART; npart += I*RED_BLOCKS;
 	__shared__ double sh[4];
 	__shared__ double hs[MAX_DOTS];
-	if(threadIdx.x < MAX_DOTS) hs[threadIdx.x] = threadIdx.x < nv ? h[threadIdx.x] : 0.0;
+	if(hblk > 0) {
+		for(int i = threadIdx.x >> 6; i < nv; i += BLOCK/64) {
+			const double s = wave_reduce(hpart + i, MAX_DOTS, hblk);
+			if((threadIdx.x & 63) == 0) {
+				hs[i] = s;
+				if(blockIdx.x == 0) h[i] = s;
+			}
+		}
+	} else if((int)threadIdx.x < nv) hs[threadIdx.x] = h[threadIdx.x];
 	__syncthreads();
 	double acc = 0.0;
 	const long stride = (long)gridDim.x*blockDim.x;
@@ -680,7 +775,7 @@ void k_gs_update(long N, const int* __restrict__ ilist, const double* __restrict
 		acc += x*x;
 	}
 	const double s = block_sum(acc, sh);
-	if(threadIdx.x == 0) partial[(size_t)blockIdx.x*MAX_DOTS] = s;
+	if(threadIdx.x == 0) npart[blockIdx.x] = s;
 }
 
 /// out = b / sqrt(*nrm2) (out may alias b)
@@ -696,26 +791,23 @@ void k_scale(long N, const int* __restrict__ ilist, const double* b, long sb,
 	for(long e = (long)blockIdx.x*blockDim.x + threadIdx.x; e < N; e += stride) out[e] = b[e]/h;
 }
 
-/// x = sum_k y_k Z_k, k < nv (with nvi: nvi[I] terms for instance I; none when negative)
+/// npart[b] = block b's part of |b|^2, summed as k_mdot does.
 __global__ __launch_bounds__(BLOCK)
-void k_lincomb(long N, const int* __restrict__ ilist, const double* __restrict__ Z, long ldz,
-               long sz, int nv, const int* __restrict__ nvi, const double* __restrict__ y,
-               long sy, double* __restrict__ x, long sx)
+void k_sqnorm(long N, const int* __restrict__ ilist, const double* __restrict__ b, long sb,
+              double* __restrict__ npart)
 {
 	const long I = inst_of(ilist);
 	if(I < 0) return;                     // a retired slot of a compacted list
-	if(nvi) nv = nvi[I];
-	Z += I*sz; y += I*sy; x += I*sx;
-	__shared__ double ys[MAX_DOTS];
-	if(threadIdx.x < MAX_DOTS) ys[threadIdx.x] = threadIdx.x < nv ? y[threadIdx.x] : 0.0;
-	__syncthreads();
+	b += I*sb; npart += I*RED_BLOCKS;
+	__shared__ double sh[4];
+	double acc = 0.0;
 	const long stride = (long)gridDim.x*blockDim.x;
 	for(long e = (long)blockIdx.x*blockDim.x + threadIdx.x; e < N; e += stride) {
-		double s = 0.0;
-		for(int k = 0; k < MAX_DOTS; k++)
-			if(k < nv) s += ys[k]*Z[k*ldz + e];
-		x[e] = s;
+		const double x = b[e];
+		acc += x*x;
 	}
+	const double s = block_sum(acc, sh);
+	if(threadIdx.x == 0) npart[blockIdx.x] = s;
 }
 
 /// x = 0 over N values per instance (a kernel rather than hipMemsetAsync, so that callers may
@@ -873,7 +965,7 @@ static void pc_setup_t(fvx_pc_s& p, const VTA* vals, VTF* fac, const Inst& L, hi
 	const int n = p.m->nelem;
 	const long sa = mstride(p.m);
 	if(p.type == FVX_PC_JACOBI || pc_sgs(p.type)) {
-		hipLaunchKernelGGL((k_invert_diag<VTA, VTF>), dim3(thread_blocks(n), L.nact), dim3(BLOCK),
+		hipLaunchKernelGGL((k_invert_diag<VTA, VTF>), dim3(quad_blocks(n), L.nact), dim3(BLOCK),
 		                   0, s, n, L.list, vals, fac, sa, pc_sgs(p.type) ? 1 : 0);
 		FVX_HIP(hipGetLastError());
 		p.patch.claimed = false;
@@ -1089,45 +1181,95 @@ int reduction_blocks() { return RED_BLOCKS; }
 int max_dots() { return MAX_DOTS; }
 long partial_stride() { return PART; }
 
-void launch_mdot(long N, const double* V, long ldv, long sv, int nv, const double* w, long sw,
-                 double* partial, double* out, long so, const Inst& L, hipStream_t s)
+/// Workgroups of a reduction over N values: those beyond N/256 would add zeros.
+static inline int red_blocks(long N)
+{
+	return (int)std::max(1L, std::min((long)RED_BLOCKS, (N + BLOCK - 1)/BLOCK));
+}
+/// Whether the workgroups that read a reduction's result add its nblk partials themselves (all of
+/// them the same sum) instead of a launch of its own: a launch is ~2.7 us, the partials are
+/// 8 nv nblk bytes for each of `readers` workgroups. With the least squares and the normalisation
+/// in one launch, a pseudo-step's linear algebra takes 320 us instead of 388 on 4,608 cells (6
+/// iterations), 430 instead of 458 on 98,304 (3); up to 64 partials only, 333 and 437. Adding
+/// them in the last workgroup to finish (a fence in each) costs more than it saves from 384
+/// workgroups on.
+static inline bool fold(int nblk, int readers, int nact)
+{
+	return nblk <= FOLD_BLOCKS && (long)readers*nact <= 8L*FOLD_BLOCKS;
+}
+
+static void mdot(long N, const double* V, long ldv, long sv, int nv, const double* w, long sw,
+                 double* partial, const Inst& L, hipStream_t s)
 {
 	if(nv < 1 || nv > MAX_DOTS) throw Error(FVX_ERR_INVALID, "multi-dot of 1 to 32 vectors");
-#define FVX_MD(M) hipLaunchKernelGGL(k_mdot<M>, dim3(RED_BLOCKS, L.nact), dim3(BLOCK), 0, s, N, \
+#define FVX_MD(M) hipLaunchKernelGGL(k_mdot<M>, dim3(red_blocks(N), L.nact), dim3(BLOCK), 0, s, N, \
 	L.list, V, ldv, sv, nv, w, sw, partial)
 	if(nv <= 8) FVX_MD(8);
 	else if(nv <= 16) FVX_MD(16);
 	else FVX_MD(MAX_DOTS);
 #undef FVX_MD
-	hipLaunchKernelGGL(k_reduce, dim3(1, L.nact), dim3(BLOCK), 0, s, RED_BLOCKS, L.list, partial,
+	FVX_HIP(hipGetLastError());
+}
+
+static void reduce(int nblk, const double* partial, int nv, double* out, long so, const Inst& L,
+                   hipStream_t s)
+{
+	hipLaunchKernelGGL(k_reduce, dim3(1, L.nact), dim3(BLOCK), 0, s, nblk, L.list, partial,
 	                   nv, out, so);
 	FVX_HIP(hipGetLastError());
 }
 
-void launch_gs_update(long N, const double* V, long ldv, long sv, int nv, const double* h,
-                      long sh, double* w, long sw, double* partial, double* nrm2, long sn,
-                      const Inst& L, hipStream_t s)
+void launch_mdot(long N, const double* V, long ldv, long sv, int nv, const double* w, long sw,
+                 double* partial, double* out, long so, const Inst& L, hipStream_t s)
 {
-	hipLaunchKernelGGL(k_gs_update, dim3(RED_BLOCKS, L.nact), dim3(BLOCK), 0, s, N, L.list, V,
-	                   ldv, sv, nv, h, sh, w, sw, partial);
-	hipLaunchKernelGGL(k_reduce, dim3(1, L.nact), dim3(BLOCK), 0, s, RED_BLOCKS, L.list, partial,
-	                   1, nrm2, sn);
+	mdot(N, V, ldv, sv, nv, w, sw, partial, L, s);
+	reduce(red_blocks(N), partial, nv, out, so, L, s);
+}
+
+void launch_sqnorm(long N, const double* b, long sb, double* npart, const Inst& L, hipStream_t s)
+{
+	hipLaunchKernelGGL(k_sqnorm, dim3(red_blocks(N), L.nact), dim3(BLOCK), 0, s, N, L.list, b, sb,
+	                   npart);
 	FVX_HIP(hipGetLastError());
 }
 
-void launch_scale(long N, const double* b, long sb, const double* nrm2, long sn, double* out,
-                  long so, const Inst& L, hipStream_t s)
+/// y = A x and its dots with V_0 .. in one launch, where each workgroup's 64 cells are one partial
+/// sum's values; false otherwise.
+static bool spmv_mdot(const fvx_matrix_s& A, const double* x, long sx, double* y, long sy,
+                      const double* V, long ldv, long sv, int nv, double* partial, const Inst& L,
+                      hipStream_t s)
 {
-	hipLaunchKernelGGL(k_scale, dim3(stream_blocks(N), L.nact), dim3(BLOCK), 0, s, N, L.list, b,
-	                   sb, nrm2, sn, out, so);
+	const int n = A.m->nelem, nblk = quad_blocks(n);
+	if(nblk > RED_BLOCKS) return false;
+#define FVX_SM(T, P, M) hipLaunchKernelGGL((k_spmv_mdot<T, M>), dim3(nblk, L.nact), dim3(BLOCK), \
+	0, s, n, L.list, P, mstride(A.m), A.m->d_nbr.p, x, sx, y, sy, V, ldv, sv, nv, partial)
+	if(A.prec == FVX_PREC_F32) {
+		if(nv <= 8) FVX_SM(float, A.f32(), 8);
+		else if(nv <= 16) FVX_SM(float, A.f32(), 16);
+		else FVX_SM(float, A.f32(), MAX_DOTS);
+	} else {
+		if(nv <= 8) FVX_SM(double, A.f64(), 8);
+		else if(nv <= 16) FVX_SM(double, A.f64(), 16);
+		else FVX_SM(double, A.f64(), MAX_DOTS);
+	}
+#undef FVX_SM
 	FVX_HIP(hipGetLastError());
+	return true;
 }
 
-void launch_lincomb(long N, const double* Z, long ldz, long sz, int nv, const double* y,
-                    long sy, double* x, long sx, const Inst& L, hipStream_t s, const int* nvi)
+void launch_arnoldi(long N, const fvx_matrix_s* A, const double* z, long sz, const double* V,
+                    long ldv, long sv, int nv, double* w, long sw, double* partial, double* npart,
+                    double* h, long sh, const Inst& L, hipStream_t s)
 {
-	hipLaunchKernelGGL(k_lincomb, dim3(stream_blocks(N), L.nact), dim3(BLOCK), 0, s, N, L.list, Z,
-	                   ldz, sz, nv, nvi, y, sy, x, sx);
+	const int nblk = red_blocks(N);
+	if(!A || !spmv_mdot(*A, z, sz, w, sw, V, ldv, sv, nv, partial, L, s)) {
+		if(A) launch_spmv(*A, z, sz, w, sw, L, s);
+		mdot(N, V, ldv, sv, nv, w, sw, partial, L, s);
+	}
+	const bool f = fold(nblk, nblk, L.nact);
+	if(!f) reduce(nblk, partial, nv, h, sh, L, s);
+	hipLaunchKernelGGL(k_gs_update, dim3(nblk, L.nact), dim3(BLOCK), 0, s, N, L.list, V,
+	                   ldv, sv, nv, partial, f ? nblk : 0, h, sh, w, sw, npart);
 	FVX_HIP(hipGetLastError());
 }
 
@@ -1136,60 +1278,59 @@ void launch_lincomb(long N, const double* Z, long ldz, long sz, int nv, const do
 /* State of one FGMRES cycle per instance (KST doubles, instance-major): the Givens-rotated
  * Hessenberg columns R[r][j] (r <= j), the rotations cs, sn, the rotated right-hand side g,
  * beta = |b|, the iteration count and the status (1 running, 0 stopped, 2 zero right-hand
- * side, -1 non-finite). The kernels below run in one workgroup: thread t serves instance
- * ids[t], t < nids; thread 0 then writes the running instances, in the order of ids, to the
- * front of `list` and -1 behind them (the compacted list the next iteration's launches
- * read), and their number to *hcount (host memory, read by the host after the kernel). */
+ * side, -1 non-finite). The least squares run in one extra workgroup of the launch that
+ * normalises the next basis vector, which needs the same norm: thread t serves instance ids[t],
+ * t < nids; thread 0 then writes the running instances, in the order of ids, to the front of
+ * `next` and -1 behind them (the compacted list the next iteration's launches read; the launch
+ * itself reads another list), and their number to *hcount (host memory, read by the host after
+ * the kernel). */
 constexpr int KR = 0, KCS = MAX_DOTS*MAX_DOTS, KSN = KCS + MAX_DOTS, KG = KSN + MAX_DOTS;
 constexpr int KBETA = KG + MAX_DOTS + 1, KIT = KBETA + 1, KSTAT = KIT + 1;
 constexpr long KST = KSTAT + 1;
 
 __device__ __forceinline__ void fgmres_compact(int nids, const int* __restrict__ ids,
                                                const double* __restrict__ kst,
-                                               int* __restrict__ list, int* hcount)
+                                               int* __restrict__ next, int* hcount)
 {
 	__syncthreads();
 	if(threadIdx.x != 0) return;
 	int k = 0;
 	for(int t = 0; t < nids; t++)
-		if(kst[ids[t]*KST + KSTAT] == 1.0) list[k++] = ids[t];
-	for(int t = k; t < nids; t++) list[t] = -1;
+		if(kst[ids[t]*KST + KSTAT] == 1.0) next[k++] = ids[t];
+	for(int t = k; t < nids; t++) next[t] = -1;
 	if(hcount) __hip_atomic_store(hcount, k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-/// Cycle start: beta = sqrt(scal[I][beta_slot]), g = (beta, 0, ...), status.
-__global__ __launch_bounds__(BLOCK)
-void k_fgmres_begin(int nids, const int* __restrict__ ids, const double* __restrict__ scal,
-                    long ns, int beta_slot, double* __restrict__ kst, int* __restrict__ list,
-                    int* hcount)
+/// Cycle start: beta = sqrt(scal[I][slot]), g = (beta, 0, ...), status.
+__device__ __forceinline__ void fgmres_begin(int nids, const int* __restrict__ ids,
+                                             const double* __restrict__ scal, long ns, int slot,
+                                             double* __restrict__ kst)
 {
 	for(int t = threadIdx.x; t < nids; t += blockDim.x) {
 		const long I = ids[t];
 		double* st = kst + I*KST;
-		const double beta = sqrt(scal[I*ns + beta_slot]);
+		const double beta = sqrt(scal[I*ns + slot]);
 		st[KBETA] = beta;
 		st[KG] = beta;
 		st[KIT] = 0.0;
 		st[KSTAT] = !isfinite(beta) ? -1.0 : beta == 0.0 ? 2.0 : 1.0;
 	}
-	fgmres_compact(nids, ids, kst, list, hcount);
 }
 
-/// Iteration j: the new Hessenberg column h_0..h_j (scal[I][h_slot + r]) and |w|^2
-/// (scal[I][nrm_slot]) go through the previous rotations and a new one; an instance stops when
-/// |g_{j+1}| <= rtol beta or at an exact breakdown, and is marked non-finite on a non-finite
-/// norm.
-__global__ __launch_bounds__(BLOCK)
-void k_fgmres_rotate(int j, double rtol, int nids, const int* __restrict__ ids,
-                     const double* __restrict__ scal, long ns, int h_slot, int nrm_slot,
-                     double* __restrict__ kst, int* __restrict__ list, int* hcount)
+/// Iteration j: the new Hessenberg column h_0..h_j (scal[I][r]) and |w|^2 (scal[I][slot]) go
+/// through the previous rotations and a new one; an instance stops when |g_{j+1}| <= rtol beta
+/// or at an exact breakdown, and is marked non-finite on a non-finite norm.
+__device__ __forceinline__ void fgmres_rotate(int j, double rtol, int nids,
+                                              const int* __restrict__ ids,
+                                              const double* __restrict__ scal, long ns, int slot,
+                                              double* __restrict__ kst)
 {
 	for(int t = threadIdx.x; t < nids; t += blockDim.x) {
 		const long I = ids[t];
 		double* st = kst + I*KST;
 		if(st[KSTAT] != 1.0) continue;
-		const double* h = scal + I*ns + h_slot;
-		const double hn = sqrt(scal[I*ns + nrm_slot]);
+		const double* h = scal + I*ns;
+		const double hn = sqrt(scal[I*ns + slot]);
 		if(!isfinite(hn)) { st[KSTAT] = -1.0; continue; }
 		double* cs = st + KCS;
 		double* sn = st + KSN;
@@ -1209,54 +1350,111 @@ void k_fgmres_rotate(int j, double rtol, int nids, const int* __restrict__ ids,
 		st[KIT] = j + 1;
 		if(fabs(g[j + 1]) <= rtol*st[KBETA] || hn == 0.0) st[KSTAT] = 0.0;
 	}
-	fgmres_compact(nids, ids, kst, list, hcount);
 }
 
-/// Cycle end: the weights y of the instances' bases (back substitution of R y = g) into
-/// scal[I][y_slot ..], and the iteration count into its[I] (-1: non-finite).
+/// out = b / sqrt(nrm2) (out may alias b) for the instances of `ilist`, nrm2 the sum of the nblk
+/// partials npart, which every workgroup adds for itself (nblk 0: nrm2 = scal[I][slot]); in the
+/// last workgroup of grid row 0 the least squares of step j (j < 0: the cycle start).
 __global__ __launch_bounds__(BLOCK)
-void k_fgmres_end(int nids, const int* __restrict__ ids, const double* __restrict__ kst,
-                  double* __restrict__ scal, long ns, int y_slot, int* __restrict__ its)
+void k_scale_rotate(long N, const int* __restrict__ ilist, const double* b, long sb,
+                    const double* __restrict__ npart, int nblk, double* scal, long ns, int slot,
+                    double* out, long so, int j, double rtol, int nids,
+                    const int* __restrict__ ids, double* __restrict__ kst, int* __restrict__ next,
+                    int* hcount)
 {
-	for(int t = threadIdx.x; t < nids; t += blockDim.x) {
-		const long I = ids[t];
-		const double* st = kst + I*KST;
-		if(st[KSTAT] == -1.0) { its[I] = -1; continue; }
-		const int it = (int)st[KIT];
-		double* y = scal + I*ns + y_slot;
-		for(int r = it - 1; r >= 0; r--) {
-			double a = st[KG + r];
-			for(int k = r + 1; k < it; k++) a -= st[KR + r*MAX_DOTS + k]*y[k];
-			y[r] = a/st[KR + r*MAX_DOTS + r];
+	if(blockIdx.x == gridDim.x - 1) {
+		if(blockIdx.y != 0) return;
+		if(nblk > 0) {
+			for(int t = threadIdx.x >> 6; t < nids; t += BLOCK/64) {
+				const long I = ids[t];
+				const double s = wave_reduce(npart + I*RED_BLOCKS, 1, nblk);
+				if((threadIdx.x & 63) == 0) scal[I*ns + slot] = s;
+			}
+			__syncthreads();
 		}
-		its[I] = it;
+		if(j < 0) fgmres_begin(nids, ids, scal, ns, slot, kst);
+		else fgmres_rotate(j, rtol, nids, ids, scal, ns, slot, kst);
+		fgmres_compact(nids, ids, kst, next, hcount);
+		return;
+	}
+	const long I = inst_of(ilist);
+	if(I < 0) return;                     // a retired slot of a compacted list
+	b += I*sb; out += I*so;
+	__shared__ double nrm2;
+	if(nblk > 0) {
+		if(threadIdx.x < 64) {
+			const double s = wave_reduce(npart + I*RED_BLOCKS, 1, nblk);
+			if(threadIdx.x == 0) nrm2 = s;
+		}
+		__syncthreads();
+	}
+	const double h = sqrt(nblk > 0 ? nrm2 : scal[I*ns + slot]);
+	const long stride = (long)(gridDim.x - 1)*blockDim.x;
+	for(long e = (long)blockIdx.x*blockDim.x + threadIdx.x; e < N; e += stride) out[e] = b[e]/h;
+}
+
+/// Cycle end: the weights y of an instance's basis (back substitution of R y = g, in every
+/// workgroup for itself) and x = sum_k y_k Z_k; the iteration count goes to its[I] (-1:
+/// non-finite, x = 0), host memory read after the kernel.
+__global__ __launch_bounds__(BLOCK)
+void k_solution(long N, const int* __restrict__ ids, const double* __restrict__ Z, long ldz,
+                long sz, const double* __restrict__ kst, double* __restrict__ x, long sx, int* its)
+{
+	const long I = ids[blockIdx.y];
+	const double* st = kst + I*KST;
+	const int it = st[KSTAT] == -1.0 ? -1 : (int)st[KIT];
+	if(blockIdx.x == 0 && threadIdx.x == 0)
+		__hip_atomic_store(its + I, it, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+	Z += I*sz; x += I*sx;
+	__shared__ double R[MAX_DOTS][MAX_DOTS + 1], ys[MAX_DOTS];
+	for(int t = threadIdx.x; t < MAX_DOTS*MAX_DOTS; t += BLOCK) {
+		const int r = t/MAX_DOTS, k = t % MAX_DOTS;
+		if(r <= k && k < it) R[r][k] = st[KR + t];
+	}
+	if((int)threadIdx.x < it) ys[threadIdx.x] = st[KG + threadIdx.x];
+	__syncthreads();
+	if(threadIdx.x == 0)
+		for(int r = it - 1; r >= 0; r--) {
+			double a = ys[r];
+			for(int k = r + 1; k < it; k++) a -= R[r][k]*ys[k];
+			ys[r] = a/R[r][r];
+		}
+	__syncthreads();
+	const long stride = (long)gridDim.x*blockDim.x;
+	for(long e = (long)blockIdx.x*blockDim.x + threadIdx.x; e < N; e += stride) {
+		double s = 0.0;
+		for(int k = 0; k < MAX_DOTS; k++)
+			if(k < it) s += ys[k]*Z[k*ldz + e];
+		x[e] = s;
 	}
 }
 
 long fgmres_state_size() { return KST; }
 
-void launch_fgmres_begin(int nids, const int* ids, const double* scal, long ns, int beta_slot,
-                         double* kst, int* list, int* hcount, hipStream_t s)
+void launch_scale_rotate(long N, const double* b, long sb, const double* npart, double* scal,
+                         long ns, int slot, double* out, long so, int j, double rtol, int nids,
+                         const int* ids, double* kst, int* next, int* hcount, const Inst& L,
+                         hipStream_t s)
 {
-	hipLaunchKernelGGL(k_fgmres_begin, dim3(1), dim3(BLOCK), 0, s, nids, ids, scal, ns,
-	                   beta_slot, kst, list, hcount);
+	const int nblk = red_blocks(N), readers = stream_blocks(N);
+	// unlike the dots, a norm's partials are few enough for more workgroups to read
+	const bool f = (long)readers*L.nact <= 8L*FOLD_BLOCKS;
+	if(!f) {
+		hipLaunchKernelGGL(k_reduce_norm, dim3(1, L.nact), dim3(64), 0, s, nblk, L.list, npart,
+		                   scal + slot, ns);
+		FVX_HIP(hipGetLastError());
+	}
+	hipLaunchKernelGGL(k_scale_rotate, dim3(readers + 1, L.nact), dim3(BLOCK), 0, s, N,
+	                   L.list, b, sb, npart, f ? nblk : 0, scal, ns, slot, out, so, j, rtol, nids,
+	                   ids, kst, next, hcount);
 	FVX_HIP(hipGetLastError());
 }
 
-void launch_fgmres_rotate(int j, double rtol, int nids, const int* ids, const double* scal,
-                          long ns, int h_slot, int nrm_slot, double* kst, int* list,
-                          int* hcount, hipStream_t s)
+void launch_solution(long N, const double* Z, long ldz, long sz, const double* kst, double* x,
+                     long sx, int* its, const Inst& L, hipStream_t s)
 {
-	hipLaunchKernelGGL(k_fgmres_rotate, dim3(1), dim3(BLOCK), 0, s, j, rtol, nids, ids, scal, ns,
-	                   h_slot, nrm_slot, kst, list, hcount);
-	FVX_HIP(hipGetLastError());
-}
-
-void launch_fgmres_end(int nids, const int* ids, const double* kst, double* scal, long ns,
-                       int y_slot, int* its, hipStream_t s)
-{
-	hipLaunchKernelGGL(k_fgmres_end, dim3(1), dim3(BLOCK), 0, s, nids, ids, kst, scal, ns,
-	                   y_slot, its);
+	hipLaunchKernelGGL(k_solution, dim3(stream_blocks(N), L.nact), dim3(BLOCK), 0, s, N, L.list, Z,
+	                   ldz, sz, kst, x, sx, its);
 	FVX_HIP(hipGetLastError());
 }
 

@@ -420,21 +420,21 @@ void pc_set_sweeps(fvx_pc_s& p, int sweeps)
 using Op = std::function<void(const double* x, long sx, double* y, long sy, const Inst& L)>;
 
 /// Device storage of one FGMRES cycle for up to `cap` instances: bases, per-instance scalar
-/// slots (h column, norms, solution weights), the least-squares state of the cycle
+/// slots (h column, norms), the least-squares state of the cycle
 /// (k_fgmres_* in linalg.hip), the cycle's instance list and its compacted running list, and
 /// pinned host words through which the device reports how many instances still run.
 struct Krylov {
 	long N = 0;
 	int m = 0, cap = 0;
-	DBuf<double> V, Z, partial, scal, kst;
-	DBuf<int> dlist, dlist_in, dids, dits;  // caller's lists / running list / cycle / counts
-	std::vector<int> dlist_ids;             // the list dlist holds on the device
+	DBuf<double> V, Z, partial, npart, scal, kst;
+	DBuf<int> dlist, dlist_in, dids;        // caller's list / running lists (2) / cycle's list
+	std::vector<int> dlist_ids, dids_ids;   // the lists dlist and dids hold on the device
 	double* hpin = nullptr;
 	int* ipin = nullptr;
 	int* hcnt = nullptr;                    // [m + 2] running instances after each step
 	int* itspin = nullptr;                  // [cap] iteration counts of the last cycle
 	std::vector<hipEvent_t> ev;
-	static constexpr int H0 = 0, NRM = 34, BETA = 35, XX = 36, RES = 37, Y0 = 40, NSCAL = 80;
+	static constexpr int H0 = 0, NRM = 34, BETA = 35, XX = 36, RES = 37, NSCAL = 40;
 
 	void ensure(long n_, int m_, int cap_)
 	{
@@ -450,12 +450,13 @@ struct Krylov {
 		kst.alloc((size_t)cap*fgmres_state_size());
 		dlist.alloc(cap);
 		dlist_ids.clear();
-		dlist_in.alloc(cap);
+		dids_ids.clear();
+		dlist_in.alloc(2*(size_t)cap);
 		dids.alloc(cap);
-		dits.alloc(cap);
+		npart.alloc((size_t)cap*reduction_blocks());
 		FVX_HIP(hipHostMalloc((void**)&hpin, (size_t)cap*NSCAL*sizeof(double)));
 		FVX_HIP(hipHostMalloc((void**)&ipin, (size_t)cap*sizeof(int)));
-		FVX_HIP(hipHostMalloc((void**)&itspin, (size_t)cap*sizeof(int)));
+		FVX_HIP(hipHostMalloc((void**)&itspin, (size_t)cap*sizeof(int), hipHostMallocCoherent));
 		FVX_HIP(hipHostMalloc((void**)&hcnt, (size_t)(m + 2)*sizeof(int), hipHostMallocCoherent));
 		std::memset(hpin, 0, (size_t)cap*NSCAL*sizeof(double));
 		ev.assign(m + 2, nullptr);
@@ -514,46 +515,49 @@ struct Krylov {
 	/// after the previous step?) to decide whether to enqueue another step, so it never waits
 	/// for the step it has just enqueued. The launches take the device list also for a single
 	/// instance (the list {0}).
-	void solve(const Op& op, const Op& pc, const double* b, double* x, int mm, double rtol,
-	           const std::vector<int>& ids, bool single, std::vector<int>& its, hipStream_t s)
+	/// The operator is the matrix `mat`, or op where mat is null.
+	void solve(const fvx_matrix_s* mat, const Op& op, const Op& pc, const double* b, double* x, int mm, double rtol,
+	           const std::vector<int>& ids, std::vector<int>& its, hipStream_t s)
 	{
-		(void)single;
 		its.assign(cap, 0);
 		const int nids = (int)ids.size();
 		if(nids == 0) return;
-		std::memcpy(ipin, ids.data(), nids*sizeof(int));
-		FVX_HIP(hipMemcpyAsync(dids.p, ipin, nids*sizeof(int), hipMemcpyHostToDevice, s));
+		if(ids != dids_ids) {
+			std::memcpy(ipin, ids.data(), nids*sizeof(int));
+			FVX_HIP(hipMemcpyAsync(dids.p, ipin, nids*sizeof(int), hipMemcpyHostToDevice, s));
+			FVX_HIP(hipStreamSynchronize(s));
+			dids_ids = ids;
+		}
 		const Inst A{dids.p, nids};            // every instance of the cycle
-		const Inst L{dlist_in.p, nids};        // the running ones, compacted on the device
-		launch_mdot(N, b, 0, N, 1, b, N, partial.p, scal.p + BETA, NSCAL, A, s);
-		launch_fgmres_begin(nids, dids.p, scal.p, NSCAL, BETA, kst.p, dlist_in.p, hcnt, s);
+		// the running ones, compacted on the device: step j reads one list and writes the other
+		auto running = [&](int j) { return Inst{dlist_in.p + (size_t)(j & 1)*cap, nids}; };
+		auto next = [&](int j) { return dlist_in.p + (size_t)((j + 1) & 1)*cap; };
+		launch_sqnorm(N, b, N, npart.p, A, s);
+		launch_scale_rotate(N, b, N, npart.p, scal.p, NSCAL, BETA, V.p, sV(), -1, rtol, nids, dids.p,
+		                    kst.p, next(-1), hcnt, A, s);
 		FVX_HIP(hipEventRecord(ev[0], s));
-		launch_scale(N, b, N, scal.p + BETA, NSCAL, V.p, sV(), L, s);
 		for(int j = 0; j < mm; j++) {
+			const Inst L = running(j);
 			double* vj = V.p + (size_t)j*N;
 			double* zj = Z.p + (size_t)j*N;
 			double* w = V.p + (size_t)(j + 1)*N;
 			pc(vj, sV(), zj, sZ(), L);
-			op(zj, sZ(), w, sV(), L);
-			launch_mdot(N, V.p, N, sV(), j + 1, w, sV(), partial.p, scal.p + H0, NSCAL, L, s);
-			launch_gs_update(N, V.p, N, sV(), j + 1, scal.p + H0, NSCAL, w, sV(), partial.p,
-			                 scal.p + NRM, NSCAL, L, s);
-			// normalise v_{j+1}; after an exact breakdown (norm 0) the vector is never used
-			launch_scale(N, w, sV(), scal.p + NRM, NSCAL, w, sV(), L, s);
-			launch_fgmres_rotate(j, rtol, nids, dids.p, scal.p, NSCAL, H0, NRM, kst.p,
-			                     dlist_in.p, hcnt + j + 1, s);
+			if(!mat) op(zj, sZ(), w, sV(), L);
+			launch_arnoldi(N, mat, zj, sZ(), V.p, N, sV(), j + 1, w, sV(), partial.p, npart.p,
+			               scal.p + H0, NSCAL, L, s);
+			// normalise v_{j+1} (after an exact breakdown, norm 0, the vector is never used) and
+			// do the least squares of the step
+			launch_scale_rotate(N, w, sV(), npart.p, scal.p, NSCAL, NRM, w, sV(), j, rtol, nids,
+			                    dids.p, kst.p, next(j), hcnt + j + 1, L, s);
 			FVX_HIP(hipEventRecord(ev[j + 1], s));
 			// step j is queued; stop if nothing ran after step j - 1 (step j then found an
 			// empty list and did nothing)
 			FVX_HIP(hipEventSynchronize(ev[j]));
 			if(__atomic_load_n(hcnt + j, __ATOMIC_ACQUIRE) == 0) break;
 		}
-		int* dits_p = dits.p;
-		launch_fgmres_end(nids, dids.p, kst.p, scal.p, NSCAL, Y0, dits_p, s);
-		launch_lincomb(N, Z.p, N, sZ(), mm, scal.p + Y0, NSCAL, x, N, A, s, dits_p);
-		FVX_HIP(hipMemcpyAsync(itspin, dits_p, cap*sizeof(int), hipMemcpyDeviceToHost, s));
+		launch_solution(N, Z.p, N, sZ(), kst.p, x, N, itspin, A, s);
 		FVX_HIP(hipStreamSynchronize(s));
-		for(int i : ids) its[i] = itspin[i];
+		for(int i : ids) its[i] = __atomic_load_n(itspin + i, __ATOMIC_ACQUIRE);
 	}
 };
 
@@ -573,11 +577,9 @@ int linear_solve(const fvx_matrix_s& A, fvx_pc_s& p, const double* b, double* x,
 	Krylov& k = *p.kry;
 	k.ensure(4L*A.m->nelem, restart, 1);
 	std::vector<int> its;
-	k.solve([&](const double* xi, long sx, double* yo, long sy, const Inst& L) {
-	            launch_spmv(A, xi, sx, yo, sy, L, s); },
-	        [&](const double* r, long sr, double* z, long sz, const Inst& L) {
+	k.solve(&A, Op(), [&](const double* r, long sr, double* z, long sz, const Inst& L) {
 	            launch_pc_apply(p, r, sr, z, sz, L, s); },
-	        b, x, restart, rtol, {0}, true, its, s);
+	        b, x, restart, rtol, {0}, its, s);
 	if(its[0] < 0) throw Error(FVX_ERR_NONFINITE, "non-finite value in the Krylov solve");
 	return its[0];
 }
@@ -775,16 +777,13 @@ void steady_core(fvx_disc_s& d, const fvx_solver_cfg& c, double* u, int ninst,
 					              K.partial.p, K.scal.p + Krylov::XX,
 					              Krylov::NSCAL, LL, bb, grad, rgrad, ughost, s);
 				};
-			else
-				op = [&](const double* x, long sx, double* y, long sy, const Inst& LL) {
-					launch_spmv(w.A, x, sx, y, sy, LL, s);
-				};
 			std::vector<double> rn2(ninst);
 			for(int i : act) rn2[i] = K.h(i, Krylov::RES);
 			const double tl0 = now();
-			K.solve(op, [&](const double* r, long sr, double* z, long sz, const Inst& LL) {
+			K.solve(c.matrix_free ? nullptr : &w.A, op,
+			        [&](const double* r, long sr, double* z, long sz, const Inst& LL) {
 			            launch_pc_apply(w.P, r, sr, z, sz, LL, s); },
-			        w.r.p, w.du.p, c.krylov_restart, c.krylov_rtol, act, single, its, s);
+			        w.r.p, w.du.p, c.krylov_restart, c.krylov_rtol, act, its, s);
 			linw += now() - tl0;
 			std::vector<int> upd;
 			for(int i : act) {
