@@ -408,11 +408,12 @@ struct Mpnn {
 	DBuf<float> d_invdeg, d_stat, d_edge;
 	DBuf<float> w, wq, am, av, grad, loss;
 	DBuf<unsigned short> frag;
-	DBuf<float> h[mpnn::NL + 1], pq[mpnn::NL];
+	DBuf<float> h[mpnn::NL], q[2];          // a layer's input; Q of a layer and of the next
 	DBuf<unsigned short> ab[mpnn::NL];
-	DBuf<unsigned long long> umask[mpnn::NL];
-	DBuf<float> g0, g1, gpart, da, y, part, gfeat;
-	DBuf<unsigned short> dpre, dpq;
+	DBuf<unsigned char> umask[mpnn::NL - 1]; // relu masks of the updates, 8 bytes a row
+	DBuf<unsigned> mmask[mpnn::NL];        // relu masks of the messages, 8 words a row
+	DBuf<float> gpart, da[2], y, part, gfeat;
+	DBuf<unsigned short> dpre[2], dpq;
 	DBuf<double> pp;
 	std::vector<float> hgf;
 	std::vector<double> hpp;
@@ -422,7 +423,9 @@ struct Mpnn {
 	int npoints = 0;                       // graphs described by the last set_points
 	void set_points(int G, const double* mach, const double* aoa, double gamma, hipStream_t s);
 	void pack(hipStream_t s);
-	void forward(int G, bool train, hipStream_t s);
+	/// With targets (training) keeps what the backward pass needs and enters it; without, the outputs
+	/// go to yout.
+	void forward(int G, const float* targets, float* yout, hipStream_t s);
 	void predict(int G, float* yout, hipStream_t s);
 	void gradient(int G, const float* targets, const int* sample_ids, hipStream_t s);
 	void adam_step(double lr, hipStream_t s);

@@ -12,16 +12,19 @@
  *   h' = h + relu(hb Wu + ab Wv + bu)                   ab: a rounded to bf16
  *   y = h4 Wdec + bdec                                  4 outputs per cell
  *
- * Data layout: rows are cells of G graphs (row = g*N + cell); activations are row-major
- * [rows][64] fp32, the P|Q pair [rows][128] fp32, GEMM-only operands (a, dL/dpre, dL/dP|dQ)
- * bf16. Per row and layer the relu pattern of the update is kept as one 64-bit mask.
+ * Data layout: rows are cells of G graphs (row = g*N + cell). Activations, Q, their gradients and
+ * da are [rows][64] fp32 in the channel order of load_row; GEMM-only operands (a, dL/dpre,
+ * dL/dP|dQ) bf16 in plain order. Per row and layer the relu patterns of the update (8 bytes) and
+ * of the four messages (32 bytes) are kept for the backward pass.
  *
- * Matrix products run on the MFMA units (v_mfma_f32_16x16x32_bf16): a wavefront keeps all 16
- * B fragments of a 64x128 or 128x64 weight matrix in registers and streams 16-row tiles of A.
- * Weight gradients (A^T B over all rows) stage 32-row chunks transposed in LDS and write one
+ * Matrix products run on the MFMA units (v_mfma_f32_16x16x32_bf16), one 16-row tile per wavefront
+ * at a time with the weights' B fragments in LDS; a launch is a whole layer, forward or backward.
+ * Weight gradients (A^T B over all rows) stage 64-row chunks transposed in LDS and write one
  * partial per workgroup; partials are summed in a fixed order, so every result is deterministic.
  */
 #include "fvx_internal.hpp"
+#include "wave.hpp"
+#include <algorithm>
 #include <cmath>
 
 namespace fvx {
@@ -33,7 +36,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short bf16_t;
 
 constexpr int RB = 256;                 // threads per workgroup of every kernel here
-constexpr int GEMM_BLOCKS = 2048;       // workgroup cap of the row-GEMM kernels
+constexpr int TILE_BLOCKS = 768;        // workgroup cap of the row-tile kernels
 constexpr int RED_BLOCKS = 512;         // workgroups that write reduction partials
 
 __device__ __forceinline__ bf16_t f2bf(float f)
@@ -121,211 +124,94 @@ __global__ void __launch_bounds__(RB) k_pack(const float* __restrict__ w, float*
 }
 
 // ------------------------------------------------------------------------------------------
-// row GEMM driver: each wavefront holds the 16 B fragments and walks 16-row tiles
+// row tiles: a wavefront takes 16 rows at a time. A operands (and everything loaded from or
+// stored to row-major arrays) are in the A layout -- lane holds row lane & 15, channels
+// 32 s + 8 (lane >> 4) .. + 7 of slice s --, products come in the C layout -- rows
+// 4 (lane >> 4) + q, channel 16 j + (lane & 15). A 16 x 64 tile in LDS, private to the wave, turns
+// one into the other. The weight fragments lie in LDS for all waves of the workgroup: in
+// registers (64-128 of them) they left two waves per SIMD.
 // ------------------------------------------------------------------------------------------
 
-template <int S, int NT, class ALoad, class Epi>
-__device__ __forceinline__ void row_gemm(int ntiles, const bf16_t* __restrict__ frag, ALoad&& aload,
-                                         Epi&& epi)
+constexpr int TLD = 68;                 // floats per tile row: both layouts free of bank conflicts
+constexpr int TILE = 16*TLD;
+constexpr int WAVES = RB/64;
+
+/// Scalar: a branch on it must not leave an MFMA to the exec mask, which it ignores.
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+__device__ __forceinline__ void wave_sync()
 {
-	static_assert(S*NT == 16, "every packed matrix has 16 fragments");
-	const int lane = threadIdx.x & 63;
-	const int wave = blockIdx.x*(RB/64) + (threadIdx.x >> 6);
-	const int nwave = gridDim.x*(RB/64);
-	bf16x8 b[S][NT];
-	const bf16x8* F = reinterpret_cast<const bf16x8*>(frag);
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ void tile_put_c(float* t, int lane, const f32x4* acc)
+{
+	wave_sync();
+#pragma unroll
+	for(int j = 0; j < 4; j++)
+#pragma unroll
+		for(int q = 0; q < 4; q++) t[(4*(lane >> 4) + q)*TLD + 16*j + (lane & 15)] = acc[j][q];
+	wave_sync();
+}
+__device__ __forceinline__ void tile_get_a(const float* t, int lane, int s, float* v)
+{
+	load8(t + (lane & 15)*TLD + 32*s + 8*(lane >> 4), v);
+}
+/// fp32 rows (h, Q, da, the gradients) are kept in an order of their own: position 32 s + 16 b +
+/// 4 g + i holds channel 32 s + 8 g + 4 b + i, so that each of the two 16-byte accesses of a lane's
+/// 8 channels makes, with the other lane groups, a full 64-byte segment of every row. In channel
+/// order every access touched twice the segments: k_layer_bwd took 643 us instead of 565.
+__device__ __forceinline__ void load_row(const float* __restrict__ rows, size_t r, int s, int lane,
+                                         float* v)
+{
+	const float* p = rows + r*W + 32*s + 4*(lane >> 4);
+	const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 16);
+#pragma unroll
+	for(int e = 0; e < 4; e++) { v[e] = a[e]; v[4 + e] = b[e]; }
+}
+__device__ __forceinline__ void store_row(float* __restrict__ rows, size_t r, int s, int lane,
+                                          const float* v)
+{
+	float* p = rows + r*W + 32*s + 4*(lane >> 4);
+	*reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+	*reinterpret_cast<f32x4*>(p + 16) = f32x4{v[4], v[5], v[6], v[7]};
+}
+/// Channel at position p of a row.
+__device__ __forceinline__ int chan(int p) { return (p & 35) | ((p & 12) << 1) | ((p & 16) >> 2); }
+
+/// acc[j] = sum over S slices of a[s] x the fragments f[(s*NT + J0 + j)*64 ..] in LDS, j < 4.
+template <int S, int NT, int J0 = 0>
+__device__ __forceinline__ void tile_mm(const bf16x8* f, int lane, const bf16x8* a, f32x4* acc)
+{
+#pragma unroll
+	for(int j = 0; j < 4; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
 	for(int s = 0; s < S; s++)
 #pragma unroll
-		for(int j = 0; j < NT; j++) b[s][j] = F[(s*NT + j)*64 + lane];
-	for(int t = wave; t < ntiles; t += nwave) {
-		f32x4 acc[NT];
-#pragma unroll
-		for(int j = 0; j < NT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-		for(int s = 0; s < S; s++) {
-			const bf16x8 a = aload(t, s, lane);
-#pragma unroll
-			for(int j = 0; j < NT; j++) acc[j] = mfma(a, b[s][j], acc[j]);
-		}
-		epi(t, lane, acc);
+		for(int j = 0; j < 4; j++) acc[j] = mfma(a[s], f[(s*NT + J0 + j)*64 + lane], acc[j]);
+}
+
+/// Fragments [s][j0 .. j0 + nj) of a packed matrix of NT columns of fragments to LDS.
+__device__ __forceinline__ void stage_frags(bf16x8* dst, const bf16_t* __restrict__ frag, int S,
+                                            int NT, int j0, int nj)
+{
+	const bf16x8* src = reinterpret_cast<const bf16x8*>(frag);
+	for(int i = threadIdx.x; i < S*nj*64; i += RB) {
+		const int l = i & 63, f = i >> 6, s = f/nj, j = f - s*nj;
+		dst[i] = src[(s*NT + j0 + j)*64 + l];
 	}
 }
 
-/// P|Q = hb [Wa | Wb]   (K = 64, 128 outputs)
-__global__ void __launch_bounds__(RB) k_pq(int R, const float* __restrict__ h,
-                                           const bf16_t* __restrict__ frag, float* __restrict__ pq)
+/// The tiles of a wavefront: every XCD owns a contiguous range and its wavefronts walk it side by
+/// side, so that the rows gathered from neighbouring cells are mostly in its L2 (a contiguous range
+/// per workgroup: k_layer 299 us instead of 274 on 786,432 rows).
+struct Tiles { int t, end, step; };
+__device__ __forceinline__ Tiles my_tiles(int ntile)
 {
-	row_gemm<2, 8>((R + 15)/16, frag,
-		[&](int t, int s, int lane) {
-			const int r = 16*t + (lane & 15);
-			if(r >= R) return zero_frag();
-			float v[8];
-			load8(h + (size_t)r*W + 32*s + 8*(lane >> 4), v);
-			return to_frag(v);
-		},
-		[&](int t, int lane, const f32x4* acc) {
-#pragma unroll
-			for(int j = 0; j < 8; j++)
-#pragma unroll
-				for(int q = 0; q < 4; q++) {
-					const int row = 16*t + 4*(lane >> 4) + q;
-					if(row < R) pq[(size_t)row*2*W + 16*j + (lane & 15)] = acc[j][q];
-				}
-		});
+	const int nb = gridDim.x, nx = min(nb, 8), x = blockIdx.x % nx, local = blockIdx.x/nx;
+	const int wgs = nb/nx + (x < nb % nx), per = (ntile + nx - 1)/nx;
+	const int wave = wave_id();
+	return { x*per + local*WAVES + wave, min((x + 1)*per, ntile), wgs*WAVES };
 }
-
-/// Aggregation of the messages of cell row r over channels c0..c0+7: a = (1/deg) sum relu(s).
-__device__ __forceinline__ void aggregate8(const Graph& g, int r, int c0, const float* __restrict__ pq,
-                                           const float* __restrict__ wl, float* a)
-{
-	const int node = r % g.N;
-	const size_t base = (size_t)(r - node);
-	float p[8], we[4][8], bm[8];
-	load8(pq + (size_t)r*2*W + c0, p);
-#pragma unroll
-	for(int f = 0; f < 4; f++) load8(wl + L_WE + f*W + c0, we[f]);
-	load8(wl + L_BM + c0, bm);
-#pragma unroll
-	for(int e = 0; e < 8; e++) a[e] = 0.f;
-#pragma unroll
-	for(int k = 0; k < 4; k++) {
-		const int j = g.nbr[node*4 + k];
-		if(j < 0) continue;
-		float q[8];
-		load8(pq + (base + j)*2*W + W + c0, q);
-		const f32x4 ef = *reinterpret_cast<const f32x4*>(g.edge + ((size_t)node*4 + k)*4);
-#pragma unroll
-		for(int e = 0; e < 8; e++) {
-			const float s = p[e] + q[e] + (ef[0]*we[0][e] + ef[1]*we[1][e] + ef[2]*we[2][e]
-			                               + ef[3]*we[3][e]) + bm[e];
-			a[e] += fmaxf(s, 0.f);
-		}
-	}
-	const float id = g.invdeg[node];
-#pragma unroll
-	for(int e = 0; e < 8; e++) a[e] *= id;
-}
-
-/// Message aggregation and residual update of one layer:
-///   h_out = h + relu([hb | ab] [Wu; Wv] + bu)   (K = 128, 64 outputs)
-/// Training passes also keep ab (bf16) and the relu mask of every row.
-__global__ void __launch_bounds__(RB) k_update(Graph g, const float* __restrict__ h,
-                                               const float* __restrict__ pq,
-                                               const float* __restrict__ wl,
-                                               const bf16_t* __restrict__ frag,
-                                               float* __restrict__ hout, bf16_t* __restrict__ ab,
-                                               unsigned long long* __restrict__ umask)
-{
-	const int R = g.R;
-	row_gemm<4, 4>((R + 15)/16, frag,
-		[&](int t, int s, int lane) {
-			const int r = 16*t + (lane & 15);
-			if(r >= R) return zero_frag();
-			float v[8];
-			if(s < 2) {
-				load8(h + (size_t)r*W + 32*s + 8*(lane >> 4), v);
-			} else {
-				const int c0 = 32*(s - 2) + 8*(lane >> 4);
-				aggregate8(g, r, c0, pq, wl, v);
-				const bf16x8 fr = to_frag(v);
-				if(ab) *reinterpret_cast<bf16x8*>(ab + (size_t)r*W + c0) = fr;
-				return fr;
-			}
-			return to_frag(v);
-		},
-		[&](int t, int lane, const f32x4* acc) {
-			unsigned long long bits[4][4];
-#pragma unroll
-			for(int j = 0; j < 4; j++) {
-				const int col = 16*j + (lane & 15);
-				const float bu = wl[L_BU + col];
-#pragma unroll
-				for(int q = 0; q < 4; q++) {
-					const int row = 16*t + 4*(lane >> 4) + q;
-					const float pre = acc[j][q] + bu;
-					bits[j][q] = __ballot(pre > 0.f);
-					if(row < R) hout[(size_t)row*W + col] = h[(size_t)row*W + col] + fmaxf(pre, 0.f);
-				}
-			}
-			if(umask && lane < 16) {
-				const int gq = lane >> 2, qq = lane & 3;
-				unsigned long long m = 0;
-#pragma unroll
-				for(int j = 0; j < 4; j++) {
-					const unsigned long long b = qq == 0 ? bits[j][0] : qq == 1 ? bits[j][1]
-					                             : qq == 2 ? bits[j][2] : bits[j][3];
-					m |= ((b >> (16*gq)) & 0xFFFFull) << (16*j);
-				}
-				const int row = 16*t + lane;
-				if(row < R) umask[row] = m;
-			}
-		});
-}
-
-/// Backward of the update: dpre = g * mask (kept as bf16), then
-///   [dh_part | da] = dpre [Wu^T | Wv^T],  dh_part += g   (K = 64, 128 outputs)
-__global__ void __launch_bounds__(RB) k_update_bwd(int R, const float* __restrict__ gin,
-                                                   const unsigned long long* __restrict__ umask,
-                                                   const bf16_t* __restrict__ frag,
-                                                   bf16_t* __restrict__ dpre,
-                                                   float* __restrict__ gpart, float* __restrict__ da)
-{
-	row_gemm<2, 8>((R + 15)/16, frag,
-		[&](int t, int s, int lane) {
-			const int r = 16*t + (lane & 15);
-			if(r >= R) return zero_frag();
-			const int c0 = 32*s + 8*(lane >> 4);
-			float v[8];
-			load8(gin + (size_t)r*W + c0, v);
-			const unsigned m = (unsigned)(umask[r] >> c0) & 0xFFu;
-#pragma unroll
-			for(int e = 0; e < 8; e++) v[e] = (m >> e) & 1u ? v[e] : 0.f;
-			const bf16x8 fr = to_frag(v);
-			*reinterpret_cast<bf16x8*>(dpre + (size_t)r*W + c0) = fr;
-			return fr;
-		},
-		[&](int t, int lane, const f32x4* acc) {
-#pragma unroll
-			for(int j = 0; j < 8; j++)
-#pragma unroll
-				for(int q = 0; q < 4; q++) {
-					const int row = 16*t + 4*(lane >> 4) + q;
-					const int col = 16*j + (lane & 15);
-					if(row >= R) continue;
-					if(j < 4) gpart[(size_t)row*W + col] = gin[(size_t)row*W + col] + acc[j][q];
-					else da[(size_t)row*W + col - W] = acc[j][q];
-				}
-		});
-}
-
-/// dh = dh_part + [dP | dQ] [Wa^T; Wb^T]   (K = 128, 64 outputs)
-__global__ void __launch_bounds__(RB) k_pq_bwd(int R, const bf16_t* __restrict__ dpq,
-                                               const bf16_t* __restrict__ frag,
-                                               const float* __restrict__ gpart,
-                                               float* __restrict__ gout)
-{
-	row_gemm<4, 4>((R + 15)/16, frag,
-		[&](int t, int s, int lane) {
-			const int r = 16*t + (lane & 15);
-			if(r >= R) return zero_frag();
-			return *reinterpret_cast<const bf16x8*>(dpq + (size_t)r*2*W + 32*s + 8*(lane >> 4));
-		},
-		[&](int t, int lane, const f32x4* acc) {
-#pragma unroll
-			for(int j = 0; j < 4; j++)
-#pragma unroll
-				for(int q = 0; q < 4; q++) {
-					const int row = 16*t + 4*(lane >> 4) + q;
-					const int col = 16*j + (lane & 15);
-					if(row < R) gout[(size_t)row*W + col] = gpart[(size_t)row*W + col] + acc[j][q];
-				}
-		});
-}
-
-// ------------------------------------------------------------------------------------------
-// VALU kernels: encoder, decoder + loss, message backward (with partial weight sums)
-// ------------------------------------------------------------------------------------------
 
 __device__ __forceinline__ void node_x(const Graph& g, int r, float* x)
 {
@@ -336,303 +222,598 @@ __device__ __forceinline__ void node_x(const Graph& g, int r, float* x)
 	x[7] = g.gfeat[2*gi + 1];
 }
 
-/// h0 = x Wenc + benc; one thread per (row, channel).
-__global__ void __launch_bounds__(RB) k_encode(Graph g, const float* __restrict__ wq,
-                                               float* __restrict__ h0)
+/// h0 = x Wenc + benc and Q0 = h0b Wb of the first layer.
+__global__ void __launch_bounds__(RB) k_embed(Graph g, int ntile, const float* __restrict__ wq,
+                                              const bf16_t* __restrict__ fpq,
+                                              float* __restrict__ h0, float* __restrict__ q0)
 {
-	const size_t t = (size_t)blockIdx.x*RB + threadIdx.x;
-	if(t >= (size_t)g.R*W) return;
-	const int r = (int)(t / W), c = (int)(t % W);
-	float x[FIN];
-	node_x(g, r, x);
-	float s = wq[OFF_BENC + c];
+	__shared__ bf16x8 wf[8*64];
+	__shared__ __attribute__((aligned(16))) float we[(FIN + 1)*W], tile[WAVES*TILE];
+	stage_frags(wf, fpq, 2, 8, 4, 4);
+	for(int i = threadIdx.x; i < (FIN + 1)*W; i += RB)
+		we[i] = i < FIN*W ? wq[OFF_WENC + i] : wq[OFF_BENC + i - FIN*W];
+	__syncthreads();
+	const int lane = threadIdx.x & 63, wave = wave_id();
+	float* t = tile + wave*TILE;
+	const Tiles ts = my_tiles(ntile);
+	for(int tt = ts.t; tt < ts.end; tt += ts.step) {
+		const int r = 16*tt + (lane & 15), rc = min(r, g.R - 1);
+		float x[FIN];
+		node_x(g, rc, x);
+		bf16x8 a[2];
 #pragma unroll
-	for(int f = 0; f < FIN; f++) s += x[f]*wq[OFF_WENC + f*W + c];
-	h0[t] = s;
+		for(int s = 0; s < 2; s++) {
+			const int c0 = 32*s + 8*(lane >> 4);
+			float v[8], w[8];
+			load8(we + FIN*W + c0, v);
+#pragma unroll
+			for(int f = 0; f < FIN; f++) {
+				load8(we + f*W + c0, w);
+#pragma unroll
+				for(int e = 0; e < 8; e++) v[e] += x[f]*w[e];
+			}
+			if(r < g.R) store_row(h0, r, s, lane, v);
+			a[s] = to_frag(v);
+		}
+		f32x4 acc[4];
+		tile_mm<2, 4>(wf, lane, a, acc);
+		tile_put_c(t, lane, acc);
+#pragma unroll
+		for(int s = 0; s < 2; s++) {
+			float v[8];
+			tile_get_a(t, lane, s, v);
+			if(r < g.R) store_row(q0, r, s, lane, v);
+		}
+	}
 }
 
-/// Decoder y = h4 Wdec + bdec (16 lanes per row, 4 channels each). With targets: the loss
-/// gradient dy = 2 (y - t) / count, dh4 = dy Wdec^T and workgroup partials of dWdec, dbdec and
-/// the squared error. Targets of graph gi are rows ids[gi] of the target set.
-__global__ void __launch_bounds__(RB) k_decode(Graph g, const float* __restrict__ h4,
-                                               const float* __restrict__ wq,
-                                               float* __restrict__ y,
-                                               const float* __restrict__ tgt, const int* __restrict__ ids,
-                                               double inv_count, float* __restrict__ gout,
-                                               float* __restrict__ part)
+/// Backward of the update, from the gradient gn of its output rows and its relu mask (A layout,
+/// both slices; mk[s] bit e): dpre = gn * mask (kept as bf16), [dh_part | da] = dpre [Wu^T | Wv^T],
+/// gpart = gn + dh_part, and da is multiplied by the 1/deg (id) of the mean.
+__device__ __forceinline__ void update_bwd_tile(const bf16x8* wf, float* t, int lane, int r, bool ok,
+                                                const float (&gn)[2][8], const unsigned (&mk)[2],
+                                                float id, bf16_t* __restrict__ dpre,
+                                                float* __restrict__ gpart, float* __restrict__ da)
 {
-	__shared__ float red[RB*21];
-	const int cg = threadIdx.x & 15, c0 = 4*cg;
-	float acc[21];
+	bf16x8 a[2];
 #pragma unroll
-	for(int v = 0; v < 21; v++) acc[v] = 0.f;
-	float wd[4][4];
+	for(int s = 0; s < 2; s++) {
+		float v[8];
 #pragma unroll
-	for(int cc = 0; cc < 4; cc++)
-#pragma unroll
-		for(int o = 0; o < 4; o++) wd[cc][o] = wq[OFF_WDEC + (c0 + cc)*FO + o];
-	const int stride = gridDim.x*(RB/16);
-	// every lane runs the same number of iterations (the shuffles below need all 16 lanes)
-	const int niter = (g.R + stride - 1)/stride;
-	for(int it = 0; it < niter; it++) {
-		const int r = it*stride + blockIdx.x*(RB/16) + (threadIdx.x >> 4);
-		const bool ok = r < g.R;
-		f32x4 hv = f32x4{0.f, 0.f, 0.f, 0.f};
-		if(ok) hv = *reinterpret_cast<const f32x4*>(h4 + (size_t)r*W + c0);
-		float yo[4];
-#pragma unroll
-		for(int o = 0; o < 4; o++) {
-			float s = hv[0]*wd[0][o] + hv[1]*wd[1][o] + hv[2]*wd[2][o] + hv[3]*wd[3][o];
-			s += __shfl_xor(s, 8, 16);
-			s += __shfl_xor(s, 4, 16);
-			s += __shfl_xor(s, 2, 16);
-			s += __shfl_xor(s, 1, 16);
-			yo[o] = s + wq[OFF_BDEC + o];
-		}
-		if(!ok) continue;
-		if(!tgt) {
-			if(cg == 0) *reinterpret_cast<f32x4*>(y + (size_t)r*FO) = f32x4{yo[0], yo[1], yo[2], yo[3]};
-			continue;
-		}
-		const int node = r % g.N, gi = r / g.N;
-		const f32x4 tv = *reinterpret_cast<const f32x4*>(tgt + ((size_t)ids[gi]*g.N + node)*FO);
-		float dy[4];
-#pragma unroll
-		for(int o = 0; o < 4; o++) {
-			const float d = yo[o] - tv[o];
-			dy[o] = (float)(2.0*(double)d*inv_count);
-			if(cg == 0) { acc[16 + o] += dy[o]; acc[20] += d*d; }
-		}
-		f32x4 gv;
-#pragma unroll
-		for(int cc = 0; cc < 4; cc++) {
-			gv[cc] = dy[0]*wd[cc][0] + dy[1]*wd[cc][1] + dy[2]*wd[cc][2] + dy[3]*wd[cc][3];
-#pragma unroll
-			for(int o = 0; o < 4; o++) acc[cc*4 + o] += hv[cc]*dy[o];
-		}
-		*reinterpret_cast<f32x4*>(gout + (size_t)r*W + c0) = gv;
+		for(int e = 0; e < 8; e++) v[e] = (mk[s] >> e) & 1u ? gn[s][e] : 0.f;
+		a[s] = to_frag(v);
+		if(ok) *reinterpret_cast<bf16x8*>(dpre + (size_t)r*W + 32*s + 8*(lane >> 4)) = a[s];
 	}
-	if(!tgt) return;
-	// reduce over the 16 row slots; partial layout: Wdec[c][o] (256), bdec (4), loss (1)
-	float* out = part + (size_t)blockIdx.x*261;
-	const int tid = threadIdx.x, slot = tid >> 4;
+	f32x4 acc[4];
+	tile_mm<2, 8>(wf, lane, a, acc);
+	tile_put_c(t, lane, acc);
 #pragma unroll
-	for(int v = 0; v < 21; v++) red[(slot*16 + cg)*21 + v] = acc[v];
+	for(int s = 0; s < 2; s++) {
+		float v[8];
+		tile_get_a(t, lane, s, v);
+#pragma unroll
+		for(int e = 0; e < 8; e++) v[e] = gn[s][e] + v[e];
+		if(ok) store_row(gpart, r, s, lane, v);
+	}
+	tile_mm<2, 8, 4>(wf, lane, a, acc);
+	tile_put_c(t, lane, acc);
+#pragma unroll
+	for(int s = 0; s < 2; s++) {
+		float v[8];
+		tile_get_a(t, lane, s, v);
+#pragma unroll
+		for(int e = 0; e < 8; e++) v[e] *= id;
+		if(ok) store_row(da, r, s, lane, v);
+	}
+}
+
+/// One layer: P = hb Wa (kept in the wave), messages and their mean a over the cell's slots from
+/// the neighbours' Q, h_out = h + relu([hb | ab] [Wu; Wv] + bu), and the next layer's
+/// Q = h_outb Wb. TRAIN keeps ab, the relu mask of the update (byte [row][s][lane >> 4]) and those
+/// of the messages (word [row][s][lane >> 4], byte k = slot k).
+/// LAST goes on with the decoder y = h_out Wdec + bdec instead of storing h_out and Q. In inference
+/// y is the result. In training the targets of graph gi are rows ids[gi] of the target set and
+/// dy = 2 (y - t) inv_count, gn = dy Wdec^T goes through the backward of the update (update_bwd_tile)
+/// right here, and workgroup partials of dWdec, dbdec and the squared error are left in part.
+///
+/// Bound by HBM and the gathers: per row h 256 + Q about 256 + edges 80 read, h 256 + Q 256
+/// (+ 168 in training) written. P|Q written by a launch of its own and read back took 565 us per
+/// layer on 786,432 rows (117 + 449), this takes 277 (1.1 GB, 77% of the copy rate). Three workgroups a
+/// compute unit; LAST in training holds 69 sums per lane, so two.
+template <bool TRAIN, bool LAST>
+__global__ void __launch_bounds__(RB, TRAIN && LAST ? 2 : 3)
+k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict__ q,
+        const float* __restrict__ wl, const bf16_t* __restrict__ fpq, const bf16_t* __restrict__ fupd,
+        const bf16_t* __restrict__ fnext, const float* __restrict__ wq,
+        float* __restrict__ hout, float* __restrict__ qout,                       // !LAST
+        bf16_t* __restrict__ ab, unsigned char* __restrict__ umask, unsigned* __restrict__ mmask, // TRAIN
+        float* __restrict__ y,                                                    // LAST, inference
+        const float* __restrict__ tgt, const int* __restrict__ ids, double inv_count, // LAST, training
+        bf16_t* __restrict__ dpre, float* __restrict__ gpart, float* __restrict__ da,
+        float* __restrict__ part)
+{
+	constexpr int NF = !LAST ? 32 : TRAIN ? 40 : 24;
+	__shared__ bf16x8 wf[NF*64];
+	__shared__ __attribute__((aligned(16))) float we[6*W], tile[WAVES*TILE];
+	__shared__ __attribute__((aligned(16))) float wd[LAST ? FO*W + FO : 1];
+	stage_frags(wf, fpq, 2, 8, 0, 4);
+	stage_frags(wf + 8*64, fupd, 4, 4, 0, 4);
+	if constexpr(!LAST) stage_frags(wf + 24*64, fnext, 2, 8, 4, 4);      // the next layer's Wb
+	else if constexpr(TRAIN) stage_frags(wf + 24*64, fnext, 2, 8, 0, 8); // this layer's [Wu^T|Wv^T]
+	for(int i = threadIdx.x; i < 6*W; i += RB)      // We, bm, bu
+		we[i] = wl[i < 4*W ? L_WE + i : i < 5*W ? L_BM + i - 4*W : L_BU + i - 5*W];
+	if constexpr(LAST)
+		for(int i = threadIdx.x; i < FO*W + FO; i += RB) wd[i] = wq[OFF_WDEC + i];
 	__syncthreads();
-	for(int i = tid; i < 261; i += RB) {
-		float s = 0.f;
-		if(i < 256) {
-			const int c = i / 4, o = i % 4, grp = c / 4, cc = c % 4;
-			for(int sl = 0; sl < RB/16; sl++) s += red[(sl*16 + grp)*21 + cc*4 + o];
+	const int lane = threadIdx.x & 63, wave = wave_id(), R = g.R;
+	float* t = tile + wave*TILE;
+	float dacc[TRAIN && LAST ? 69 : 1];
+	for(float& v : dacc) v = 0.f;
+	const Tiles ts = my_tiles(ntile);
+	for(int tt = ts.t; tt < ts.end; tt += ts.step) {
+		const int r = 16*tt + (lane & 15), rc = min(r, R - 1);
+		const int node = rc % g.N;
+		const size_t base = (size_t)(rc - node);
+		float hv[2][8];
+		bf16x8 a[4];
+#pragma unroll
+		for(int s = 0; s < 2; s++) {
+			load_row(h, rc, s, lane, hv[s]);
+			a[s] = to_frag(hv[s]);
+		}
+		const int4 nb = *reinterpret_cast<const int4*>(g.nbr + 4*node);
+		const int nbs[4] = { nb.x, nb.y, nb.z, nb.w };
+		f32x4 ef[4];
+#pragma unroll
+		for(int k = 0; k < 4; k++)
+			ef[k] = *reinterpret_cast<const f32x4*>(g.edge + ((size_t)node*4 + k)*4);
+		const float id = g.invdeg[node];
+		f32x4 acc[4];
+		tile_mm<2, 4>(wf, lane, a, acc);
+		tile_put_c(t, lane, acc);
+		unsigned mm[2] = {0u, 0u};
+#pragma unroll
+		for(int s = 0; s < 2; s++) {
+			const int c0 = 32*s + 8*(lane >> 4);
+			float p[8], qv[4][8], w[4][8], bm[8], av[8];
+#pragma unroll
+			for(int k = 0; k < 4; k++)
+				load_row(q, base + (nbs[k] >= 0 ? nbs[k] : node), s, lane, qv[k]);
+			tile_get_a(t, lane, s, p);
+#pragma unroll
+			for(int f = 0; f < 4; f++) load8(we + f*W + c0, w[f]);
+			load8(we + 4*W + c0, bm);
+#pragma unroll
+			for(int e = 0; e < 8; e++) av[e] = 0.f;
+#pragma unroll
+			for(int k = 0; k < 4; k++) {
+				const bool on = nbs[k] >= 0;
+				unsigned bits = 0u;
+#pragma unroll
+				for(int e = 0; e < 8; e++) {
+					const float m = p[e] + qv[k][e] + (ef[k][0]*w[0][e] + ef[k][1]*w[1][e]
+					                                   + ef[k][2]*w[2][e] + ef[k][3]*w[3][e]) + bm[e];
+					av[e] += on ? fmaxf(m, 0.f) : 0.f;
+					if constexpr(TRAIN) bits |= m > 0.f ? 1u << e : 0u;
+				}
+				if constexpr(TRAIN) mm[s] |= on ? bits << 8*k : 0u;
+			}
+#pragma unroll
+			for(int e = 0; e < 8; e++) av[e] *= id;
+			a[2 + s] = to_frag(av);
+			if constexpr(TRAIN) {
+				if(r < R) {
+					*reinterpret_cast<bf16x8*>(ab + (size_t)r*W + c0) = a[2 + s];
+					mmask[(size_t)r*8 + 4*s + (lane >> 4)] = mm[s];
+				}
+			}
+		}
+		tile_mm<4, 4>(wf + 8*64, lane, a, acc);
+#pragma unroll
+		for(int j = 0; j < 4; j++) {
+			const float bu = we[5*W + 16*j + (lane & 15)];
+#pragma unroll
+			for(int i = 0; i < 4; i++) acc[j][i] = fmaxf(acc[j][i] + bu, 0.f);
+		}
+		tile_put_c(t, lane, acc);
+		float yo[FO] = {0.f, 0.f, 0.f, 0.f};
+		unsigned um[2];
+#pragma unroll
+		for(int s = 0; s < 2; s++) {
+			const int c0 = 32*s + 8*(lane >> 4);
+			float u[8];
+			tile_get_a(t, lane, s, u);
+			um[s] = 0u;
+#pragma unroll
+			for(int e = 0; e < 8; e++) {
+				if constexpr(TRAIN) um[s] |= u[e] > 0.f ? 1u << e : 0u;
+				hv[s][e] = hv[s][e] + u[e];
+			}
+			if constexpr(!LAST) {
+				if(r < R) store_row(hout, r, s, lane, hv[s]);
+				if(TRAIN && r < R) umask[(size_t)r*8 + 4*s + (lane >> 4)] = (unsigned char)um[s];
+				a[s] = to_frag(hv[s]);
+			} else {
+#pragma unroll
+				for(int e = 0; e < 8; e++) {
+					const f32x4 d = *reinterpret_cast<const f32x4*>(wd + (c0 + e)*FO);
+#pragma unroll
+					for(int o = 0; o < FO; o++) yo[o] += hv[s][e]*d[o];
+				}
+			}
+		}
+		if constexpr(!LAST) {
+			tile_mm<2, 4>(wf + 24*64, lane, a, acc);
+			tile_put_c(t, lane, acc);
+#pragma unroll
+			for(int s = 0; s < 2; s++) {
+				float v[8];
+				tile_get_a(t, lane, s, v);
+				if(r < R) store_row(qout, r, s, lane, v);
+			}
 		} else {
-			const int v = i - 256 + 16;          // bdec 0..3 -> 16..19, loss -> 20
-			for(int sl = 0; sl < RB/16; sl++) s += red[(sl*16 + 0)*21 + v];
+#pragma unroll
+			for(int o = 0; o < FO; o++) {
+				yo[o] += __shfl_xor(yo[o], 16);
+				yo[o] += __shfl_xor(yo[o], 32);
+				yo[o] += wd[FO*W + o];
+			}
+			if constexpr(!TRAIN) {
+				if(lane < 16 && r < R)
+					*reinterpret_cast<f32x4*>(y + (size_t)r*FO) = f32x4{yo[0], yo[1], yo[2], yo[3]};
+			} else {
+				const f32x4 tv = *reinterpret_cast<const f32x4*>(tgt + ((size_t)ids[rc/g.N]*g.N + node)*FO);
+				float dy[FO], gn[2][8];
+#pragma unroll
+				for(int o = 0; o < FO; o++) {
+					const float d = r < R ? yo[o] - tv[o] : 0.f;
+					dy[o] = (float)(2.0*(double)d*inv_count);
+					dacc[64 + o] += dy[o];
+					dacc[68] += d*d;
+				}
+#pragma unroll
+				for(int s = 0; s < 2; s++)
+#pragma unroll
+					for(int e = 0; e < 8; e++) {
+						const f32x4 d = *reinterpret_cast<const f32x4*>(wd + (32*s + 8*(lane >> 4) + e)*FO);
+						gn[s][e] = dy[0]*d[0] + dy[1]*d[1] + dy[2]*d[2] + dy[3]*d[3];
+#pragma unroll
+						for(int o = 0; o < FO; o++) dacc[(8*s + e)*FO + o] += hv[s][e]*dy[o];
+					}
+				update_bwd_tile(wf + 24*64, t, lane, r, r < R, gn, um, id, dpre, gpart, da);
+			}
 		}
-		out[i] = s;
+	}
+	if constexpr(TRAIN && LAST) {
+		// partial layout: Wdec[c][o] (256), bdec (4), squared error (1)
+		float* red = t;
+		wave_sync();
+#pragma unroll
+		for(int i = 0; i < 69; i++) {
+			float v = dacc[i];
+			v += __shfl_xor(v, 8);
+			v += __shfl_xor(v, 4);
+			v += __shfl_xor(v, 2);
+			v += __shfl_xor(v, 1);
+			if((lane & 15) == 0) {
+				if(i < 64) red[(32*(i >> 5) + 8*(lane >> 4))*FO + (i & 31)] = v;
+				else if(lane == 0) red[256 + i - 64] = v;
+			}
+		}
+		__syncthreads();
+		for(int i = threadIdx.x; i < 261; i += RB) {
+			float v = 0.f;
+			for(int w = 0; w < WAVES; w++) v += tile[w*TILE + i];
+			part[(size_t)blockIdx.x*261 + i] = v;
+		}
 	}
 }
 
-/// Backward of the aggregation (16 lanes per cell, 4 channels each):
-///   ds_ik = (1/deg_i) da_i [s_ik > 0];  dP_i = sum_k ds_ik;  dQ_j = sum over the slots of j
-/// of ds at the neighbour's reverse slot; workgroup partials of dWe = sum e_ik ds_ik and
-/// dbm = sum ds_ik. Writes dP|dQ as bf16 (the operand of the following GEMMs).
-__global__ void __launch_bounds__(RB) k_message_bwd(Graph g, const float* __restrict__ pq,
-                                                    const float* __restrict__ da,
-                                                    const float* __restrict__ wl,
-                                                    bf16_t* __restrict__ dpq,
-                                                    float* __restrict__ part)
+/// Backward through one layer's messages and P|Q, and through the previous layer's update.
+///   ds_ik = da_i [s_ik > 0] (the forward pass's masks; da holds the factor 1/deg already);
+///   dP_i = sum_k ds_ik;
+///   dQ_i = sum over the slots of i of ds at the neighbour's reverse slot;
+///   gn = gpart + [dP | dQ] [Wa^T; Wb^T], the gradient of the layer's input;
+/// then update_bwd_tile with the previous layer's mask and weights (FIRST: gn itself is written,
+/// for the encoder). dP|dQ are kept as bf16 (an operand of the weight gradients); workgroup
+/// partials of dWe = sum e_ik ds_ik and dbm = sum dP.
+///
+/// Bound by HBM and the gathers of da: per row da 256 + about 256 + masks 64 + edges 80 + gpart 256
+/// read, dP|dQ 256 + dpre 128 + gpart 256 + da 256 written. Three launches that recomputed the
+/// messages from P|Q took 1,148 us per layer on 786,432 rows (790 + 166 + 192), this takes 565
+/// (1.5 GB): the 80 partial sums per lane leave two waves per SIMD, whose waits for the gathers
+/// are the rest.
+template <bool FIRST>
+__global__ void __launch_bounds__(RB, 2) k_layer_bwd(Graph g, int ntile,
+                                                     const float* __restrict__ da,
+                                                     const unsigned* __restrict__ mmask,
+                                                     const bf16_t* __restrict__ fbpq,
+                                                     const bf16_t* __restrict__ fbupd,
+                                                     const unsigned char* __restrict__ umask,
+                                                     bf16_t* __restrict__ dpq,
+                                                     float* __restrict__ gpart,
+                                                     bf16_t* __restrict__ dpre,
+                                                     float* __restrict__ daout,
+                                                     float* __restrict__ part)
 {
-	__shared__ float red[RB*20];
-	const int cg = threadIdx.x & 15, c0 = 4*cg;
-	float we[4][4], bm[4];
+	__shared__ bf16x8 wf[(FIRST ? 16 : 32)*64];
+	__shared__ __attribute__((aligned(16))) float tile[WAVES*TILE];
+	stage_frags(wf, fbpq, 4, 4, 0, 4);
+	if constexpr(!FIRST) stage_frags(wf + 16*64, fbupd, 2, 8, 0, 8);
+	__syncthreads();
+	const int lane = threadIdx.x & 63, wave = wave_id(), R = g.R, gl = lane >> 4;
+	float* t = tile + wave*TILE;
+	float wacc[5][2][8];
 #pragma unroll
-	for(int f = 0; f < 4; f++)
+	for(int f = 0; f < 5; f++)
 #pragma unroll
-		for(int cc = 0; cc < 4; cc++) we[f][cc] = wl[L_WE + f*W + c0 + cc];
+		for(int s = 0; s < 2; s++)
 #pragma unroll
-	for(int cc = 0; cc < 4; cc++) bm[cc] = wl[L_BM + c0 + cc];
-	float acc[20];
+			for(int e = 0; e < 8; e++) wacc[f][s][e] = 0.f;
+	const Tiles ts = my_tiles(ntile);
+	for(int tt = ts.t; tt < ts.end; tt += ts.step) {
+		const int r = 16*tt + (lane & 15), rc = min(r, R - 1);
+		const bool ok = r < R;
+		const int node = rc % g.N;
+		const size_t base = (size_t)(rc - node);
+		const int4 nb = *reinterpret_cast<const int4*>(g.nbr + 4*node);
+		const int4 rv = *reinterpret_cast<const int4*>(g.rev + 4*node);
+		const int nbs[4] = { nb.x, nb.y, nb.z, nb.w }, rvs[4] = { rv.x, rv.y, rv.z, rv.w };
+		size_t rj[4];
 #pragma unroll
-	for(int v = 0; v < 20; v++) acc[v] = 0.f;
-	const int stride = gridDim.x*(RB/16);
-	for(int r = blockIdx.x*(RB/16) + (threadIdx.x >> 4); r < g.R; r += stride) {
-		const int node = r % g.N;
-		const size_t base = (size_t)(r - node);
-		const f32x4 dj = *reinterpret_cast<const f32x4*>(da + (size_t)r*W + c0);
-		const f32x4 pj = *reinterpret_cast<const f32x4*>(pq + (size_t)r*2*W + c0);
-		const f32x4 qj = *reinterpret_cast<const f32x4*>(pq + (size_t)r*2*W + W + c0);
-		const float idj = g.invdeg[node];
-		float dP[4] = {0.f, 0.f, 0.f, 0.f}, dQ[4] = {0.f, 0.f, 0.f, 0.f};
 		for(int k = 0; k < 4; k++) {
-			const int j = g.nbr[node*4 + k];
-			if(j < 0) continue;
-			const size_t rj = base + j;
-			const f32x4 e = *reinterpret_cast<const f32x4*>(g.edge + ((size_t)node*4 + k)*4);
-			const f32x4 qn = *reinterpret_cast<const f32x4*>(pq + rj*2*W + W + c0);
-			// own edge i -> j
+			rj[k] = base + (nbs[k] >= 0 ? nbs[k] : node);
+		}
+		bf16x8 a[4];
 #pragma unroll
-			for(int cc = 0; cc < 4; cc++) {
-				const float s = pj[cc] + qn[cc] + (e[0]*we[0][cc] + e[1]*we[1][cc] + e[2]*we[2][cc]
-				                                   + e[3]*we[3][cc]) + bm[cc];
-				const float ds = s > 0.f ? idj*dj[cc] : 0.f;
-				dP[cc] += ds;
+		for(int s = 0; s < 2; s++) {
+			const int c0 = 32*s + 8*gl;
+			float d[8], dn[4][8], dP[8], dQ[8];
+			load_row(da, rc, s, lane, d);
+			// a row past the end contributes nothing
+			const unsigned mo = ok ? mmask[(size_t)rc*8 + 4*s + gl] : 0u;
+			unsigned mn[4];
 #pragma unroll
-				for(int f = 0; f < 4; f++) acc[f*4 + cc] += e[f]*ds;
-				acc[16 + cc] += ds;
+			for(int k = 0; k < 4; k++) {
+				load_row(da, rj[k], s, lane, dn[k]);
+				mn[k] = mmask[rj[k]*8 + 4*s + gl] >> 8*(rvs[k] & 3);
+				if(nbs[k] < 0) mn[k] = 0u;
 			}
-			// reverse edge j -> this cell, seen from the neighbour's slot
-			const int kk = g.rev[node*4 + k];
-			const f32x4 e2 = *reinterpret_cast<const f32x4*>(g.edge + ((size_t)j*4 + kk)*4);
-			const f32x4 pn = *reinterpret_cast<const f32x4*>(pq + rj*2*W + c0);
-			const f32x4 dn = *reinterpret_cast<const f32x4*>(da + rj*W + c0);
-			const float idn = g.invdeg[j];
 #pragma unroll
-			for(int cc = 0; cc < 4; cc++) {
-				const float s = pn[cc] + qj[cc] + (e2[0]*we[0][cc] + e2[1]*we[1][cc] + e2[2]*we[2][cc]
-				                                   + e2[3]*we[3][cc]) + bm[cc];
-				dQ[cc] += s > 0.f ? idn*dn[cc] : 0.f;
+			for(int e = 0; e < 8; e++) { dP[e] = 0.f; dQ[e] = 0.f; }
+#pragma unroll
+			for(int k = 0; k < 4; k++) {
+				const f32x4 ef = *reinterpret_cast<const f32x4*>(g.edge + ((size_t)node*4 + k)*4);
+#pragma unroll
+				for(int e = 0; e < 8; e++) {
+					const float ds = (mo >> (8*k + e)) & 1u ? d[e] : 0.f;
+					dP[e] += ds;
+#pragma unroll
+					for(int f = 0; f < 4; f++) wacc[f][s][e] += ef[f]*ds;
+					dQ[e] += (mn[k] >> e) & 1u ? dn[k][e] : 0.f;
+				}
+			}
+#pragma unroll
+			for(int e = 0; e < 8; e++) wacc[4][s][e] += dP[e];
+			a[s] = to_frag(dP);
+			a[2 + s] = to_frag(dQ);
+			if(ok) {
+				*reinterpret_cast<bf16x8*>(dpq + (size_t)r*2*W + c0) = a[s];
+				*reinterpret_cast<bf16x8*>(dpq + (size_t)r*2*W + W + c0) = a[2 + s];
 			}
 		}
-		const unsigned p0 = pack2(dP[0], dP[1]), p1 = pack2(dP[2], dP[3]);
-		const unsigned q0 = pack2(dQ[0], dQ[1]), q1 = pack2(dQ[2], dQ[3]);
-		*reinterpret_cast<uint2*>(dpq + (size_t)r*2*W + c0) = make_uint2(p0, p1);
-		*reinterpret_cast<uint2*>(dpq + (size_t)r*2*W + W + c0) = make_uint2(q0, q1);
-	}
-	// partial layout: We[f][c] (256), bm[c] (64)
-	float* out = part + (size_t)blockIdx.x*320;
-	const int tid = threadIdx.x, slot = tid >> 4;
+		f32x4 acc[4];
+		tile_mm<4, 4>(wf, lane, a, acc);
+		tile_put_c(t, lane, acc);
+		float gn[2][8];
 #pragma unroll
-	for(int v = 0; v < 20; v++) red[(slot*16 + cg)*20 + v] = acc[v];
+		for(int s = 0; s < 2; s++) {
+			float v[8];
+			tile_get_a(t, lane, s, v);
+			load_row(gpart, rc, s, lane, gn[s]);
+#pragma unroll
+			for(int e = 0; e < 8; e++) gn[s][e] = gn[s][e] + v[e];
+			if constexpr(FIRST) { if(ok) store_row(gpart, r, s, lane, gn[s]); }
+		}
+		if constexpr(!FIRST) {
+			const unsigned mk[2] = { umask[(size_t)rc*8 + gl], umask[(size_t)rc*8 + 4 + gl] };
+			update_bwd_tile(wf + 16*64, t, lane, r, ok, gn, mk, g.invdeg[node], dpre, gpart, daout);
+		}
+	}
+	// partial layout: We[f][c] (256), bm[c] (64): sum over the 16 rows of a tile by lane
+	// exchanges, then over the waves in order
+	wave_sync();
+#pragma unroll
+	for(int f = 0; f < 5; f++)
+#pragma unroll
+		for(int s = 0; s < 2; s++)
+#pragma unroll
+			for(int e = 0; e < 8; e++) {
+				float v = wacc[f][s][e];
+				v += __shfl_xor(v, 8);
+				v += __shfl_xor(v, 4);
+				v += __shfl_xor(v, 2);
+				v += __shfl_xor(v, 1);
+				if((lane & 15) == 0) t[f*W + 32*s + 8*gl + e] = v;
+			}
 	__syncthreads();
-	for(int i = tid; i < 320; i += RB) {
-		int grp, v;
-		if(i < 256) { const int f = i / W, c = i % W; grp = c / 4; v = f*4 + c % 4; }
-		else { const int c = i - 256; grp = c / 4; v = 16 + c % 4; }
+	for(int i = threadIdx.x; i < 320; i += RB) {
 		float s = 0.f;
-		for(int sl = 0; sl < RB/16; sl++) s += red[(sl*16 + grp)*20 + v];
-		out[i] = s;
+		for(int w = 0; w < WAVES; w++) s += tile[w*TILE + i];
+		part[(size_t)blockIdx.x*320 + i] = s;
 	}
 }
 
 /// Encoder backward partials: dWenc[f][c] = sum_r x_f g0[r][c], dbenc[c] = sum_r g0[r][c];
-/// four row slots of 64 channels per workgroup.
+/// 16 lanes per row, 4 channels each. Bound by the read of g0: one row per wave at a time took
+/// 284 us on 786,432 rows, this takes 78.
 __global__ void __launch_bounds__(RB) k_encode_bwd(Graph g, const float* __restrict__ g0,
                                                    float* __restrict__ part)
 {
-	__shared__ float red[RB*9];
-	const int c = threadIdx.x & 63, slot = threadIdx.x >> 6;
-	float acc[9];
+	__shared__ float red[WAVES][576];
+	const int cg = threadIdx.x & 15, lane = threadIdx.x & 63, wave = wave_id();
+	float acc[9][4];
 #pragma unroll
-	for(int v = 0; v < 9; v++) acc[v] = 0.f;
-	for(int r = blockIdx.x*4 + slot; r < g.R; r += gridDim.x*4) {
+	for(int v = 0; v < 9; v++)
+#pragma unroll
+		for(int i = 0; i < 4; i++) acc[v][i] = 0.f;
+	const int stride = gridDim.x*(RB/16);
+#pragma unroll 4
+	for(int r = blockIdx.x*(RB/16) + (threadIdx.x >> 4); r < g.R; r += stride) {
+		const f32x4 gv = *reinterpret_cast<const f32x4*>(g0 + (size_t)r*W + 4*cg);
 		float x[FIN];
 		node_x(g, r, x);
-		const float gv = g0[(size_t)r*W + c];
 #pragma unroll
-		for(int f = 0; f < FIN; f++) acc[f] += x[f]*gv;
-		acc[8] += gv;
+		for(int i = 0; i < 4; i++) {
+#pragma unroll
+			for(int f = 0; f < FIN; f++) acc[f][i] += x[f]*gv[i];
+			acc[8][i] += gv[i];
+		}
 	}
 #pragma unroll
-	for(int v = 0; v < 9; v++) red[(slot*64 + c)*9 + v] = acc[v];
+	for(int f = 0; f < 9; f++)
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			float v = acc[f][i];
+			v += __shfl_xor(v, 16);
+			v += __shfl_xor(v, 32);
+			if(lane < 16) red[wave][f*W + chan(4*cg) + i] = v;
+		}
 	__syncthreads();
-	float* out = part + (size_t)blockIdx.x*576;
 	for(int i = threadIdx.x; i < 576; i += RB) {
-		const int f = i < 512 ? i / W : 8, cc = i < 512 ? i % W : i - 512;
-		float s = 0.f;
-		for(int sl = 0; sl < 4; sl++) s += red[(sl*64 + cc)*9 + f];
-		out[i] = s;
+		float v = 0.f;
+		for(int w = 0; w < WAVES; w++) v += red[w][i];
+		part[(size_t)blockIdx.x*576 + i] = v;
 	}
 }
 
 // ------------------------------------------------------------------------------------------
-// weight gradients on the MFMA units: C[K][NO] = sum_r A[r][k] B[r][n] (+ bias row sum_r B)
+// weight gradients on the MFMA units
 // ------------------------------------------------------------------------------------------
 
-constexpr int CH = 32;          // rows per LDS chunk (the MFMA reduction depth)
-constexpr int LDS_LD = 40;      // bf16 per transposed LDS row (32 + 8 padding, 80 bytes)
+constexpr int CH = 64;          // rows per LDS chunk
+constexpr int WG_PART = 2*W*W + W + 2*W*W;
 
-/// A = [h (fp32, rounded to bf16) | a2 (bf16, when K = 128)], B = bf16 [R][NO].
-template <int K, int NO, bool BIAS>
-__global__ void __launch_bounds__(RB) k_wgrad(int R, int chunks_per_block,
-                                              const float* __restrict__ h,
-                                              const bf16_t* __restrict__ a2,
-                                              const bf16_t* __restrict__ bsrc,
-                                              float* __restrict__ part)
+/// One layer's [dWu; dWv] = [hb | ab]^T dpre, dbu = sum dpre, [dWa | dWb] = hb^T dpq: the products'
+/// depth is the rows, so chunks of 64 rows are transposed through LDS: a thread loads two channels
+/// of 8 rows (a wave: whole rows) and writes 16 bytes per channel, the 16-byte units of a channel
+/// exchanged by (channel/2) mod 8 and the two channels in the order of bit 3 of their pair, which
+/// keeps writes and reads free of bank conflicts. The next chunk is loaded while this one is
+/// multiplied. Wave w takes rows 16 w of dWu, dWv and [dWa | dWb].
+///
+/// Bound by HBM: 768 bytes per row. Two kernels that read h once each and transposed with
+/// two-byte writes took 296 us on 786,432 rows, this takes 142 (604 MB, 83% of the copy rate).
+__global__ void __launch_bounds__(RB, 2) k_wgrad(int R, int chunks_per_block,
+                                                 const float* __restrict__ h,
+                                                 const bf16_t* __restrict__ ab,
+                                                 const bf16_t* __restrict__ dpre,
+                                                 const bf16_t* __restrict__ dpq,
+                                                 float* __restrict__ part)
 {
-	__shared__ __attribute__((aligned(16))) bf16_t AT[K*LDS_LD];
-	__shared__ __attribute__((aligned(16))) bf16_t BT[NO*LDS_LD];
-	constexpr int TN = NO/16, NTILE = (K/16)*TN, PER = NTILE/4;
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	f32x4 acc[PER];
+	__shared__ __attribute__((aligned(16))) bf16_t T[5*W*CH];
+	const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+	const int p = tid & 31, rg = tid >> 5, odd = (p >> 3) & 1;
+	const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+	f32x4 accu[2][4], accp[8], accb = zero;
 #pragma unroll
-	for(int m = 0; m < PER; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-	float bsum = 0.f;
-	const int c_begin = blockIdx.x*chunks_per_block;
+	for(int j = 0; j < 4; j++) { accu[0][j] = zero; accu[1][j] = zero; }
+#pragma unroll
+	for(int j = 0; j < 8; j++) accp[j] = zero;
+	const float one[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+	const bf16x8 ones = to_frag(one);
 	const int nchunk = (R + CH - 1)/CH;
+	const int c_begin = blockIdx.x*chunks_per_block;
 	const int c_end = min(c_begin + chunks_per_block, nchunk);
+	float2 vh[8];
+	unsigned vb[4][8];
+	auto load = [&](int ch) {
+#pragma unroll
+		for(int i = 0; i < 8; i++) {
+			const int r = ch*CH + 8*rg + i;
+			const size_t rc = min(r, R - 1);
+			vh[i] = *reinterpret_cast<const float2*>(h + rc*W + 2*p);
+			vb[0][i] = *reinterpret_cast<const unsigned*>(ab + rc*W + 2*p);
+			vb[1][i] = *reinterpret_cast<const unsigned*>(dpre + rc*W + 2*p);
+			vb[2][i] = *reinterpret_cast<const unsigned*>(dpq + rc*2*W + 2*p);
+			vb[3][i] = *reinterpret_cast<const unsigned*>(dpq + rc*2*W + W + 2*p);
+		}
+		if((ch + 1)*CH > R) {       // rows past the end count nothing
+#pragma unroll
+			for(int i = 0; i < 8; i++)
+				if(ch*CH + 8*rg + i >= R) {
+					vh[i] = make_float2(0.f, 0.f);
+#pragma unroll
+					for(int a = 0; a < 4; a++) vb[a][i] = 0u;
+				}
+		}
+	};
+	auto put = [&](int a, const unsigned* v) {      // v[i]: channels 2p (low), 2p + 1 of row 8 rg + i
+		u32x4 lo, hi;
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			lo[i] = (v[2*i] & 0xFFFFu) | (v[2*i + 1] << 16);
+			hi[i] = (v[2*i] >> 16) | (v[2*i + 1] & 0xFFFF0000u);
+		}
+		bf16_t* d = T + (W*a + 2*p)*CH + 8*(rg ^ (p & 7));
+		*reinterpret_cast<u32x4*>(d + odd*CH) = odd ? hi : lo;
+		*reinterpret_cast<u32x4*>(d + (1 - odd)*CH) = odd ? lo : hi;
+	};
+	auto frag = [&](int c16, int rgl) {
+		const int c = c16 + (lane & 15);
+		return *reinterpret_cast<const bf16x8*>(T + c*CH + 8*(rgl ^ ((c >> 1) & 7)));
+	};
+	if(c_begin < c_end) load(c_begin);
 	for(int ch = c_begin; ch < c_end; ch++) {
-		const int r0 = ch*CH;
 		__syncthreads();
-		{   // h chunk: 32 rows x 64 fp32, 8 values per thread
-			const int row = tid >> 3, c8 = (tid & 7)*8;
-			float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-			if(r0 + row < R) load8(h + (size_t)(r0 + row)*W + c8, v);
+		{
+			unsigned v[8];
 #pragma unroll
-			for(int e = 0; e < 8; e++) AT[(c8 + e)*LDS_LD + row] = f2bf(v[e]);
-		}
-		if(K == 128) {
-			const int row = tid >> 3, c8 = (tid & 7)*8;
-			u32x4 v = {0u, 0u, 0u, 0u};
-			if(r0 + row < R) v = *reinterpret_cast<const u32x4*>(a2 + (size_t)(r0 + row)*W + c8);
+			for(int i = 0; i < 8; i++) v[i] = pack2(vh[i].x, vh[i].y);
+			put(0, v);
 #pragma unroll
-			for(int e = 0; e < 8; e++)
-				AT[(W + c8 + e)*LDS_LD + row] = (bf16_t)(v[e/2] >> (16*(e & 1)));
-		}
-#pragma unroll
-		for(int it = 0; it < NO/64; it++) {
-			const int idx = tid + RB*it;
-			const int row = idx / (NO/8), c8 = (idx % (NO/8))*8;
-			u32x4 v = {0u, 0u, 0u, 0u};
-			if(r0 + row < R) v = *reinterpret_cast<const u32x4*>(bsrc + (size_t)(r0 + row)*NO + c8);
-#pragma unroll
-			for(int e = 0; e < 8; e++)
-				BT[(c8 + e)*LDS_LD + row] = (bf16_t)(v[e/2] >> (16*(e & 1)));
+			for(int a = 0; a < 4; a++) put(1 + a, vb[a]);
 		}
 		__syncthreads();
+		if(ch + 1 < c_end) load(ch + 1);
 #pragma unroll
-		for(int m = 0; m < PER; m++) {
-			const int tt = wave + 4*m, tk = tt / TN, tn = tt % TN;
-			const bf16x8 a = *reinterpret_cast<const bf16x8*>(AT + (16*tk + (lane & 15))*LDS_LD
-			                                                   + 8*(lane >> 4));
-			const bf16x8 b = *reinterpret_cast<const bf16x8*>(BT + (16*tn + (lane & 15))*LDS_LD
-			                                                   + 8*(lane >> 4));
-			acc[m] = mfma(a, b, acc[m]);
-		}
-		if(BIAS && tid < NO) {
-			float s = 0.f;
-			for(int rr = 0; rr < CH; rr++) s += bf2f(BT[tid*LDS_LD + rr]);
-			bsum += s;
+		for(int t = 0; t < CH/32; t++) {
+			const int rgl = 4*t + (lane >> 4);
+			const bf16x8 ah = frag(16*wave, rgl), aa = frag(W + 16*wave, rgl);
+#pragma unroll
+			for(int j = 0; j < 4; j++) {
+				const bf16x8 b = frag(2*W + 16*j, rgl);
+				accu[0][j] = mfma(ah, b, accu[0][j]);
+				accu[1][j] = mfma(aa, b, accu[1][j]);
+				if(j == wave) accb = mfma(ones, b, accb);
+			}
+#pragma unroll
+			for(int j = 0; j < 8; j++) accp[j] = mfma(ah, frag(3*W + 16*j, rgl), accp[j]);
 		}
 	}
-	float* out = part + (size_t)blockIdx.x*(K*NO + (BIAS ? NO : 0));
+	float* out = part + (size_t)blockIdx.x*WG_PART;
+	float* outp = out + 2*W*W + W;
 #pragma unroll
-	for(int m = 0; m < PER; m++) {
-		const int tt = wave + 4*m, tk = tt / TN, tn = tt % TN;
+	for(int i = 0; i < 4; i++) {
+		const int k = 16*wave + 4*(lane >> 4) + i, kh = chan(k), n = lane & 15;
 #pragma unroll
-		for(int q = 0; q < 4; q++)
-			out[(16*tk + 4*(lane >> 4) + q)*NO + 16*tn + (lane & 15)] = acc[m][q];
+		for(int j = 0; j < 4; j++) {
+			out[kh*W + 16*j + n] = accu[0][j][i];
+			out[(W + k)*W + 16*j + n] = accu[1][j][i];
+		}
+#pragma unroll
+		for(int j = 0; j < 8; j++) outp[kh*2*W + 16*j + n] = accp[j][i];
 	}
-	if(BIAS && tid < NO) out[K*NO + tid] = bsum;
+	if(lane < 16) out[2*W*W + 16*wave + lane] = accb[0];
 }
 
 /// Sums `nblk` partials of `width` values into the flat gradient. A workgroup owns 16
 /// consecutive values; its 16 lane groups each sum every 16th partial (in increasing order), and
-/// the 16 group sums are added in group order, so the result is deterministic. Modes:
-/// 0 contiguous at off1; 1 columns split (a [rows][width/rows] matrix whose left half goes to
-/// off1 and right half to off2); 2 rows split (rows < half -> off1, the rest -> off2).
+/// the 16 group sums are added in group order, so the result is deterministic. Plain partials
+/// go to off on, the last value to `extra` if given; k_wgrad's (weights) to their places among the
+/// layer's weights, which start at off.
 constexpr int RED_COLS = 16, RED_GROUPS = RB/RED_COLS;
-__global__ void __launch_bounds__(RB) k_reduce(int nblk, int width, int ncols, int mode,
-                                               int off1, int off2, const float* __restrict__ part,
+__global__ void __launch_bounds__(RB) k_reduce(int nblk, int width, bool weights, int off,
+                                               const float* __restrict__ part,
                                                float* __restrict__ grad, float* __restrict__ extra)
 {
 	__shared__ double sh[RB];
@@ -646,18 +827,17 @@ __global__ void __launch_bounds__(RB) k_reduce(int nblk, int width, int ncols, i
 	if(grp != 0 || i >= width) return;
 	double s = 0.0;
 	for(int g = 0; g < RED_GROUPS; g++) s += sh[g*RED_COLS + c];
-	const int k = i / ncols, n = i % ncols;
-	if(mode == 0) {
-		if(extra && i == width - 1) { *extra = (float)s; return; }
-		grad[off1 + i] = (float)s;
-	} else if(mode == 1) {
-		const int hc = ncols/2;
-		if(n < hc) grad[off1 + k*hc + n] = (float)s;
-		else grad[off2 + k*hc + n - hc] = (float)s;
-	} else {
-		if(k < W) grad[off1 + k*ncols + n] = (float)s;
-		else grad[off2 + (k - W)*ncols + n] = (float)s;
+	int to = i;
+	if(weights) {
+		const int ip = i - (2*W*W + W);         // >= 0: [dWa | dWb]
+		if(ip >= 0) to = (ip % (2*W) < W ? L_WA : L_WB - W) + ip/(2*W)*W + ip % (2*W);
+		else if(i >= 2*W*W) to = L_BU + i - 2*W*W;
+		else to = i < W*W ? L_WU + i : L_WV + i - W*W;
+	} else if(extra && i == width - 1) {
+		*extra = (float)s;
+		return;
 	}
+	grad[off + to] = (float)s;
 }
 
 /// Adam (Kingma and Ba, 2015) on the fp32 master weights.
@@ -730,7 +910,6 @@ double point_segment(double px, double py, double ax, double ay, double bx, doub
 }
 
 int blocks_for(size_t n) { return (int)((n + RB - 1)/RB); }
-int reduce_grid(int width) { return (width + RED_COLS - 1)/RED_COLS; }
 
 }
 
@@ -812,16 +991,20 @@ void Mpnn::init(const fvx_mesh_s& m, int wall_tag, int max_graphs)
 	FVX_HIP(hipMemset(am.p, 0, NPARAM*sizeof(float)));
 	FVX_HIP(hipMemset(av.p, 0, NPARAM*sizeof(float)));
 	frag.alloc((size_t)NL*4*FRAG_MAT);
-	for(int l = 0; l <= NL; l++) h[l].alloc(R16*W);
 	for(int l = 0; l < NL; l++) {
-		pq[l].alloc(R16*2*W);
+		h[l].alloc(R16*W);
 		ab[l].alloc(R16*W);
-		umask[l].alloc(R16);
+		mmask[l].alloc(R16*8);
+		if(l + 1 < NL) umask[l].alloc(R16*8);
 	}
-	g0.alloc(R16*W); g1.alloc(R16*W); gpart.alloc(R16*W); da.alloc(R16*W);
-	dpre.alloc(R16*W); dpq.alloc(R16*2*W);
+	for(int i = 0; i < 2; i++) {
+		q[i].alloc(R16*W);
+		da[i].alloc(R16*W);
+		dpre[i].alloc(R16*W);
+	}
+	gpart.alloc(R16*W); dpq.alloc(R16*2*W);
 	y.alloc(R16*FO);
-	part.alloc((size_t)RED_BLOCKS*(2*W*W + W));
+	part.alloc((size_t)RED_BLOCKS*WG_PART);
 	gfeat.alloc(2*(size_t)cap);
 	pp.alloc(3*(size_t)cap);
 	ids.alloc(cap);
@@ -867,32 +1050,35 @@ void Mpnn::pack(hipStream_t s)
 	dirty = false;
 }
 
-static int gemm_grid(int R) { return std::max(1, std::min(GEMM_BLOCKS, ((R + 15)/16 + 3)/4)); }
+/// Workgroups of the row-tile kernels: as many as are resident at once (LDS: 3 a compute unit).
+static int tile_grid(int R) { return std::max(1, std::min(TILE_BLOCKS, ((R + 15)/16 + WAVES - 1)/WAVES)); }
 
-void Mpnn::forward(int G, bool train, hipStream_t s)
+void Mpnn::forward(int G, const float* targets, float* yout, hipStream_t s)
 {
 	pack(s);
 	const Graph g = make_graph(*this, G);
-	const int R = g.R;
-	k_encode<<<blocks_for((size_t)R*W), RB, 0, s>>>(g, wq.p, h[0].p);
+	const int R = g.R, nt = (R + 15)/16, nb = tile_grid(R);
+	const double inv = 1.0/((double)R*FO);
+	k_embed<<<nb, RB, 0, s>>>(g, nt, wq.p, frag.p + M_PQ*FRAG_MAT, h[0].p, q[0].p);
 	for(int l = 0; l < NL; l++) {
 		const bf16_t* fl = frag.p + (size_t)l*4*FRAG_MAT;
-		k_pq<<<gemm_grid(R), RB, 0, s>>>(R, h[l].p, fl + M_PQ*FRAG_MAT, pq[l].p);
-		k_update<<<gemm_grid(R), RB, 0, s>>>(g, h[l].p, pq[l].p, wq.p + OFF_L0 + l*LSZ,
-		                                     fl + M_UPD*FRAG_MAT, h[l + 1].p,
-		                                     train ? ab[l].p : nullptr,
-		                                     train ? umask[l].p : nullptr);
+		const bool last = l + 1 == NL;
+		auto run = [&](auto kernel) {
+			kernel<<<nb, RB, 0, s>>>(g, nt, h[l].p, q[l & 1].p, wq.p + OFF_L0 + l*LSZ,
+				fl + M_PQ*FRAG_MAT, fl + M_UPD*FRAG_MAT, fl + (last ? M_BUPD : 4 + M_PQ)*FRAG_MAT, wq.p,
+				last ? nullptr : h[l + 1].p, q[(l + 1) & 1].p, ab[l].p, last ? nullptr : umask[l].p, mmask[l].p,
+				yout, targets, ids.p, inv, dpre[l & 1].p, gpart.p, da[l & 1].p, part.p);
+		};
+		if(!last) { if(targets) run(k_layer<true, false>); else run(k_layer<false, false>); }
+		else if(targets) run(k_layer<true, true>);
+		else run(k_layer<false, true>);
 	}
 	FVX_HIP(hipGetLastError());
 }
 
 void Mpnn::predict(int G, float* yout, hipStream_t s)
 {
-	forward(G, false, s);
-	const Graph g = make_graph(*this, G);
-	k_decode<<<RED_BLOCKS, RB, 0, s>>>(g, h[NL].p, wq.p, yout, nullptr, nullptr, 0.0, nullptr,
-	                                   nullptr);
-	FVX_HIP(hipGetLastError());
+	forward(G, nullptr, yout, s);
 }
 
 void Mpnn::gradient(int G, const float* targets, const int* sample_ids, hipStream_t s)
@@ -901,40 +1087,34 @@ void Mpnn::gradient(int G, const float* targets, const int* sample_ids, hipStrea
 		if(sample_ids[i] < 0) throw Error(FVX_ERR_INVALID, "negative sample index");
 	hids.assign(sample_ids, sample_ids + G);
 	FVX_HIP(hipMemcpyAsync(ids.p, hids.data(), G*sizeof(int), hipMemcpyHostToDevice, s));
-	forward(G, true, s);
+	forward(G, targets, nullptr, s);
 	const Graph g = make_graph(*this, G);
-	const int R = g.R;
-	float* gc = g0.p;
-	float* gn = g1.p;
-	k_decode<<<RED_BLOCKS, RB, 0, s>>>(g, h[NL].p, wq.p, nullptr, targets, ids.p,
-	                                   1.0/((double)R*FO), gc, part.p);
-	k_reduce<<<reduce_grid(261), RB, 0, s>>>(RED_BLOCKS, 261, 261, 0, OFF_WDEC, 0, part.p, grad.p,
-	                                        loss.p);
+	const int R = g.R, nt = (R + 15)/16, nb = tile_grid(R);
+	auto reduce = [&](int nblk, int width, bool weights, int off, float* extra) {
+		k_reduce<<<(width + RED_COLS - 1)/RED_COLS, RB, 0, s>>>(nblk, width, weights, off, part.p,
+		                                                       grad.p, extra);
+	};
+	reduce(nb, 261, false, OFF_WDEC, loss.p);
 	const int nchunk = (R + CH - 1)/CH;
-	const int nwb = std::min(RED_BLOCKS, nchunk);
-	const int cpb = (nchunk + nwb - 1)/nwb;
-	const int nwb_used = (nchunk + cpb - 1)/cpb;
+	const int cpb = (nchunk + RED_BLOCKS - 1)/RED_BLOCKS;
+	const int nwb = (nchunk + cpb - 1)/cpb;
+	// da[l & 1] and dpre[l & 1] hold layer l's; the backward pass of a layer leaves those of the one
+	// before it
 	for(int l = NL - 1; l >= 0; l--) {
 		const bf16_t* fl = frag.p + (size_t)l*4*FRAG_MAT;
-		const float* wl = wq.p + OFF_L0 + l*LSZ;
-		const int base = OFF_L0 + l*LSZ;
-		k_update_bwd<<<gemm_grid(R), RB, 0, s>>>(R, gc, umask[l].p, fl + M_BUPD*FRAG_MAT, dpre.p,
-		                                         gpart.p, da.p);
-		k_message_bwd<<<RED_BLOCKS, RB, 0, s>>>(g, pq[l].p, da.p, wl, dpq.p, part.p);
-		k_reduce<<<reduce_grid(320), RB, 0, s>>>(RED_BLOCKS, 320, 320, 0, base + L_WE, 0, part.p,
-		                                        grad.p, nullptr);
-		k_pq_bwd<<<gemm_grid(R), RB, 0, s>>>(R, dpq.p, fl + M_BPQ*FRAG_MAT, gpart.p, gn);
-		k_wgrad<W, 2*W, false><<<nwb_used, RB, 0, s>>>(R, cpb, h[l].p, nullptr, dpq.p, part.p);
-		k_reduce<<<reduce_grid(W*2*W), RB, 0, s>>>(nwb_used, W*2*W, 2*W, 1, base + L_WA, base + L_WB,
-		                                          part.p, grad.p, nullptr);
-		k_wgrad<2*W, W, true><<<nwb_used, RB, 0, s>>>(R, cpb, h[l].p, ab[l].p, dpre.p, part.p);
-		k_reduce<<<reduce_grid(2*W*W + W), RB, 0, s>>>(nwb_used, 2*W*W + W, W, 2, base + L_WU,
-		                                              base + L_WV, part.p, grad.p, nullptr);
-		std::swap(gc, gn);
+		const int base = OFF_L0 + l*LSZ, a = l & 1, b = 1 - a;
+		if(l > 0)
+			k_layer_bwd<false><<<nb, RB, 0, s>>>(g, nt, da[a].p, mmask[l].p, fl + M_BPQ*FRAG_MAT,
+				fl + (M_BUPD - 4)*FRAG_MAT, umask[l - 1].p, dpq.p, gpart.p, dpre[b].p, da[b].p, part.p);
+		else
+			k_layer_bwd<true><<<nb, RB, 0, s>>>(g, nt, da[a].p, mmask[l].p, fl + M_BPQ*FRAG_MAT, nullptr,
+				nullptr, dpq.p, gpart.p, nullptr, nullptr, part.p);
+		reduce(nb, 320, false, base + L_WE, nullptr);
+		k_wgrad<<<nwb, RB, 0, s>>>(R, cpb, h[l].p, ab[l].p, dpre[a].p, dpq.p, part.p);
+		reduce(nwb, WG_PART, true, base, nullptr);
 	}
-	k_encode_bwd<<<RED_BLOCKS, RB, 0, s>>>(g, gc, part.p);
-	k_reduce<<<reduce_grid(576), RB, 0, s>>>(RED_BLOCKS, 576, 576, 0, OFF_WENC, 0, part.p, grad.p,
-	                                        nullptr);
+	k_encode_bwd<<<RED_BLOCKS, RB, 0, s>>>(g, gpart.p, part.p);
+	reduce(RED_BLOCKS, 576, false, OFF_WENC, nullptr);
 	FVX_HIP(hipGetLastError());
 }
 
