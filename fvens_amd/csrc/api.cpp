@@ -593,13 +593,14 @@ fvx_status fvx_set_launch(fvx_disc d, int kernel, int block, int xcd)
 		require(xcd == 0 || xcd == 1, "xcd must be 0 or 1");
 		if(kernel == FVX_KERNEL_GRADIENTS) { d->tune.grad_block = block; d->tune.grad_xcd = xcd; }
 		else if(kernel == FVX_KERNEL_FLUX) {
-			d->tune.flux_block = block; d->tune.flux_xcd = xcd; d->tune.flux_wave = 0;
+			d->tune.flux_block = block; d->tune.flux_xcd = xcd;
+			d->tune.flux_wave = d->tune.flux_group = 0;
 		}
 		else if(kernel == FVX_KERNEL_FLUX_WAVE) {
 			require(block == 64, "the wave-task flux kernel runs one wave64 per workgroup");
 			require(fvx::flux_wave_apply(*d), "the wave-task flux form applies to inviscid "
 			        "first-order or linear reconstruction only");
-			d->tune.flux_xcd = xcd; d->tune.flux_wave = 1;
+			d->tune.flux_xcd = xcd; d->tune.flux_wave = 1; d->tune.flux_group = 0;
 		}
 		else if(kernel == FVX_KERNEL_JACOBIAN) {
 			require(block <= 256, "the Jacobian kernel takes at most 256 threads per workgroup");

@@ -40,9 +40,11 @@ void FVX_CAT(launch_flux_, FVX_FLUX_ID)(int mode, bool visc, int ncell, const do
 #undef FVX_LAUNCH
 }
 
-void FVX_CAT(launch_flux_wave_, FVX_FLUX_ID)(int mode, int ncell, int ngroup, const double* u,
-                                             const double* rgrad, const int* tasks,
-                                             const int2* groups, const unsigned* slots,
+void FVX_CAT(launch_flux_wave_, FVX_FLUX_ID)(int mode, bool visc, int ncell, int ngroup,
+                                             const double* u, const double* rgrad,
+                                             const double* grad, const int* tasks,
+                                             const int2* groups, const int* cells,
+                                             const unsigned* slots,
                                              const FaceGeom* fg, const double* centre,
                                              const double* area, const int* bcid,
                                              const GasParams* gpa, const BCTable* bta,
@@ -50,14 +52,19 @@ void FVX_CAT(launch_flux_wave_, FVX_FLUX_ID)(int mode, int ncell, int ngroup, co
                                              const BatchArg& ba, int nact, int xcd,
                                              hipStream_t s)
 {
-	if(mode == 0)
-		hipLaunchKernelGGL((k_flux_wave<FVX_FLUX_ID, 0>), dim3(ngroup, nact), dim3(64), 0, s, ncell,
-		                   u, rgrad, tasks, groups, slots, fg, centre, area, bcid, gpa, bta, ba,
-		                   res, dt, getdt, xcd);
-	else
-		hipLaunchKernelGGL((k_flux_wave<FVX_FLUX_ID, 1>), dim3(ngroup, nact), dim3(64), 0, s, ncell,
-		                   u, rgrad, tasks, groups, slots, fg, centre, area, bcid, gpa, bta, ba,
-		                   res, dt, getdt, xcd);
+#define FVX_LAUNCH(M, V) hipLaunchKernelGGL((k_flux_wave<FVX_FLUX_ID, M, V>), dim3(ngroup, nact), \
+		dim3(64), 0, s, ncell, u, rgrad, grad, tasks, groups, cells, slots, fg, centre, area, bcid, \
+		gpa, bta, ba, res, dt, getdt, xcd)
+	if(!visc) {
+		if(mode == 0) FVX_LAUNCH(0, false);
+		else if(mode == 1) FVX_LAUNCH(1, false);
+		else FVX_LAUNCH(2, false);
+	} else {
+		if(mode == 0) FVX_LAUNCH(0, true);
+		else if(mode == 1) FVX_LAUNCH(1, true);
+		else FVX_LAUNCH(2, true);
+	}
+#undef FVX_LAUNCH
 }
 
 }

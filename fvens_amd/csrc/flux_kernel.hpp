@@ -93,6 +93,42 @@ __device__ __forceinline__ void load_grad(const double* __restrict__ g, int c, d
 	load4(g + 8*c + 4, v + 4);
 }
 
+/// MUSCL-Van Albada face values, kappa = 1/3, eps = 1e-8, of the primitive states wl, wr with
+/// gradients gl, gr, (ex, ey) from centre to centre; a boundary face has no right value.
+__device__ __forceinline__ void muscl_states(const double* wl, const double* wr, const double* gl,
+                                             const double* gr, double ex, double ey, bool bnd,
+                                             double* rl, double* rr)
+{
+	const double kap = 1.0/3.0, eps = 1e-8;
+	for(int k = 0; k < 4; k++) {
+		const double dw = wr[k] - wl[k];
+		const double dm = 2.0*(gl[2*k]*ex + gl[2*k+1]*ey) - dw;
+		double pl = (2.0*dm*dw + eps)/(dm*dm + dw*dw + eps);
+		if(pl < 0.0) pl = 0.0;
+		rl[k] = wl[k] + pl*0.25*((1.0 - kap*pl)*dm + (1.0 + kap*pl)*dw);
+		if(!bnd) {
+			const double dp = 2.0*(gr[2*k]*ex + gr[2*k+1]*ey) - dw;
+			double pr = (2.0*dp*dw + eps)/(dp*dp + dw*dw + eps);
+			if(pr < 0.0) pr = 0.0;
+			rr[k] = wr[k] - pr*0.25*((1.0 - kap*pr)*dp + (1.0 + kap*pr)*dw);
+		}
+	}
+}
+
+/// Spectral radius times length of one side of a face, for the time step of its cell.
+template <bool VISC>
+__device__ __forceinline__ double face_radius(const GasParams& gp, const FaceState& S, double len,
+                                              const double* __restrict__ area, int cell)
+{
+	double srad = (fabs(S.vn) + S.c)*len;
+	if constexpr(VISC) {
+		const double mu = gp.constvisc ? 1.0/gp.Reinf : sutherland(gp, S.p*S.ir*gp.gM2);
+		const double co = fmax(4.0/(3*S.r), gp.g/S.r);
+		srad += co*mu/gp.Pr*len*len/area[cell];
+	}
+	return srad;
+}
+
 template <int FLUX, int MODE, bool VISC>
 __global__ __launch_bounds__(MAX_BLOCK)
 void k_flux(int ncell, const double* __restrict__ u, const double* __restrict__ rgrad,
@@ -170,26 +206,10 @@ void k_flux(int ncell, const double* __restrict__ u, const double* __restrict__ 
 			}
 		}
 		else {
-			// MUSCL-Van Albada, kappa = 1/3, eps = 1e-8
-			double gL[8], gR[8];
+			double gL[8], gR[8], rl[4], rr[4];
 			load_grad(grad, cL, gL);
 			if(!bnd) load_grad(grad, cR, gR);
-			const double ex = xR[0] - xL[0], ey = xR[1] - xL[1];
-			const double kap = 1.0/3.0, eps = 1e-8;
-			double rl[4], rr[4];
-			for(int k = 0; k < 4; k++) {
-				const double dw = wR[k] - wL[k];
-				const double dm = 2.0*(gL[2*k]*ex + gL[2*k+1]*ey) - dw;
-				double pl = (2.0*dm*dw + eps)/(dm*dm + dw*dw + eps);
-				if(pl < 0.0) pl = 0.0;
-				rl[k] = wL[k] + pl*0.25*((1.0 - kap*pl)*dm + (1.0 + kap*pl)*dw);
-				if(!bnd) {
-					const double dp = 2.0*(gR[2*k]*ex + gR[2*k+1]*ey) - dw;
-					double pr = (2.0*dp*dw + eps)/(dp*dp + dw*dw + eps);
-					if(pr < 0.0) pr = 0.0;
-					rr[k] = wR[k] - pr*0.25*((1.0 - kap*pr)*dp + (1.0 + kap*pr)*dw);
-				}
-			}
+			muscl_states(wL, wR, gL, gR, xR[0] - xL[0], xR[1] - xL[1], bnd, rl, rr);
 			A = fs_prim(gp, rl, n, igm1);
 			if(!bnd) B = fs_prim(gp, rr, n, igm1);
 		}
@@ -222,12 +242,7 @@ void k_flux(int ncell, const double* __restrict__ u, const double* __restrict__ 
 
 		if(getdt) {
 			const FaceState& S = selfL ? A : B;
-			srad = (fabs(S.vn) + S.c)*G.len;
-			if constexpr(VISC) {
-				const double mu = gp.constvisc ? 1.0/gp.Reinf : sutherland(gp, S.p*S.ir*gp.gM2);
-				const double co = fmax(4.0/(3*S.r), gp.g/S.r);
-				srad += co*mu/gp.Pr*G.len*G.len/area[cc];
-			}
+			srad = face_radius<VISC>(gp, S, G.len, area, cc);
 		}
 	}
 	for(int k = 0; k < 4; k++) F[k] = quad_sum(F[k]);

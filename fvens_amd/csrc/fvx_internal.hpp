@@ -97,11 +97,13 @@ struct fvx_mesh_s {
 	fvx::DBuf<double> d_centre;            // [nelem][2]
 	fvx::DBuf<double> d_area;              // [nelem]
 	fvx::DBuf<int> d_bhost, d_btag;        // [nbface] host cell and marker of boundary faces
-	// wave-task form of the flux pass (flux_wave.hpp): per group of consecutive cells whose
-	// faces make at most 64 tasks, the tasks, the group's cells and each cell's slot codes
+	// wave-task form of the flux pass (flux_wave.hpp): per group of neighbouring cells whose faces
+	// make at most 64 tasks, the tasks, the group's cells and each cell's slot codes
 	int nwgroup = 0;
+	bool wave_order = false;               // the cell order is compact, groups are consecutive cells
+	fvx::DBuf<int> d_wcell;                // [nelem] the groups' cells, group after group (!wave_order)
 	fvx::DBuf<int> d_wtask;                // [ngroup][64] face of each task, -1 none
-	fvx::DBuf<int2> d_wgroup;              // [ngroup] {first cell, cells}
+	fvx::DBuf<int2> d_wgroup;              // [ngroup] {first entry in d_wcell, cells}
 	fvx::DBuf<unsigned> d_wslot;           // [ngroup][64] per cell: byte k = 2 task + side of
 	                                       // slot k, 0xff unused
 };
@@ -136,7 +138,8 @@ namespace fvx {
 struct Tuning {
 	int flux_block = 256, grad_block = 256, jac_block = 256;
 	int flux_xcd = 1, grad_xcd = 1, jac_xcd = 1;
-	int flux_wave = 0;     ///< 1: wave-task form of the flux pass where it applies
+	int flux_wave = 0;     ///< 1: wave-task form of the flux pass, as selected by a caller
+	int flux_group = 1;    ///< 1: wave-task form whatever flux_wave says (nothing selected)
 };
 }
 

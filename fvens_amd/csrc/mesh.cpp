@@ -231,65 +231,120 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 	build_wave_tasks(m);
 }
 
-/* Tables of the wave-task flux kernel (flux_wave.hpp). Cells are taken in order into groups of
- * at most 64 while the faces touching the group make at most 64 tasks: a cell adds one task
- * per face to the boundary, to a later cell or to a cell outside the group, none for a face to
- * an earlier cell of the group (that face's task then serves both cells). A task is its face's
- * index (the face record holds the two cells); a cell's slot word holds, in byte k, 2 task +
- * side for its local face k (side 1: the cell is the face's right cell), 0xff when unused. */
+/* Tables of the wave-task flux kernel (flux_wave.hpp). Groups of at most 64 cells grow while the
+ * faces touching the group make at most 64 tasks: a cell adds one task per face, less the faces
+ * to cells already in the group (those faces' tasks serve both cells).
+ *
+ * Where the cell order itself is compact, at least 24 consecutive cells per group on average
+ * (Hilbert, structured natural orders), groups are consecutive cells: 28.3 on the half-triangle
+ * airfoil in Hilbert order, and on 1,572,864 cells the pass took 122 us against 142 us with groups
+ * grown as below, whose gathers touch more lines.
+ * Elsewhere (RCM order: 16 to 20 consecutive cells) a group starts at the lowest cell without one
+ * and takes, of the group's neighbours that still fit, the cell with the most faces to the group,
+ * then with the fewest neighbours left without a group (no holes stay behind), then the one met
+ * first: 25.6 quadrilaterals per group, 31 cells where half are triangles.
+ *
+ * A task is its face's index (the face record holds the two cells); a cell's slot word holds, in
+ * byte k, 2 task + side for its local face k (side 1: the cell is the face's right cell), 0xff when
+ * unused. */
 void build_wave_tasks(fvx_mesh_s& m)
 {
 	const int n = m.nelem;
-	std::vector<int> tasks;
-	std::vector<int2> groups;
-	std::vector<unsigned> slots;
-	int c = 0;
-	while(c < n) {
+	// first cells of the groups of consecutive cells
+	std::vector<int> consec;
+	for(int c = 0; c < n; ) {
 		const int c0 = c;
-		int ntask = 0;
-		while(c < n && c - c0 < 64) {
-			int add = 0;
+		consec.push_back(c0);
+		for(int nt = 0; c < n && c - c0 < 64; c++) {
 			for(int k = 0; k < m.nnode[c]; k++) {
 				const int o = m.esuel[(size_t)c*4 + k];
-				if(!(o < n && o >= c0 && o < c)) add++;
+				nt += !(o < n && o >= c0 && o < c);
 			}
-			if(ntask + add > 64) break;
-			ntask += add;
-			c++;
+			if(nt > 64) break;
 		}
-		const int c1 = c, g = (int)groups.size();
-		groups.push_back(make_int2(c0, c1 - c0));
+	}
+	m.wave_order = n >= 24L*(long)consec.size();
+	std::vector<int> tasks, cells, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand;
+	std::vector<int2> groups;
+	std::vector<unsigned> slots;
+	cells.reserve(n);
+	consec.push_back(n);
+	int seed = 0;
+	while((int)cells.size() < n) {
+		const int g = (int)groups.size(), first = (int)cells.size();
+		if(m.wave_order)
+			for(int c = consec[g]; c < consec[g + 1]; c++) { grp[c] = g; cells.push_back(c); }
+		else while(grp[seed] >= 0) seed++;
+		cand.assign(1, seed);
+		seen[seed] = g;
+		links[seed] = met[seed] = 0;
+		int ntask = 0, nmet = 1;
+		while(!m.wave_order && (int)cells.size() - first < 64) {
+			int best = -1, bl = 0, bo = 0;
+			for(int i = 0; i < (int)cand.size(); i++) {
+				const int c = cand[i], l = links[c];
+				if(ntask + m.nnode[c] - l > 64) continue;
+				int open = 0;
+				for(int k = 0; k < m.nnode[c]; k++) {
+					const int o = m.esuel[(size_t)c*4 + k];
+					open += o < n && grp[o] < 0;
+				}
+				if(best < 0 || l > bl || (l == bl && (open < bo || (open == bo && met[c] < met[cand[best]])))) {
+					best = i; bl = l; bo = open;
+				}
+			}
+			if(best < 0) break;
+			const int c = cand[best];
+			cand[best] = cand.back();
+			cand.pop_back();
+			grp[c] = g;
+			cells.push_back(c);
+			ntask += m.nnode[c] - links[c];
+			for(int k = 0; k < m.nnode[c]; k++) {
+				const int o = m.esuel[(size_t)c*4 + k];
+				if(o >= n || grp[o] >= 0) continue;
+				if(seen[o] != g) { seen[o] = g; links[o] = 0; met[o] = nmet++; cand.push_back(o); }
+				links[o]++;
+			}
+		}
+		const int ng = (int)cells.size() - first;
+		std::sort(cells.begin() + first, cells.end());
+		groups.push_back(make_int2(first, ng));
 		const size_t tb = tasks.size();
 		tasks.resize(tb + 64, -1);
 		slots.resize(slots.size() + 64, 0xffffffffu);
 		unsigned* sl = &slots[(size_t)g*64];
-		auto set_code = [&](int cell, int k, int task, int side) {
-			unsigned& w = sl[cell - c0];
-			w = (w & ~(0xffu << 8*k)) | ((unsigned)(2*task + side) << 8*k);
+		auto set_code = [&](int j, int k, int task, int side) {
+			sl[j] = (sl[j] & ~(0xffu << 8*k)) | ((unsigned)(2*task + side) << 8*k);
 		};
 		int nt = 0;
-		for(int cc = c0; cc < c1; cc++)
+		for(int j = 0; j < ng; j++) {
+			const int cc = cells[first + j];
 			for(int k = 0; k < m.nnode[cc]; k++) {
 				const int o = m.esuel[(size_t)cc*4 + k];
 				const int f = m.elemface[(size_t)cc*4 + k];
-				if(o >= c0 && o < c1) {
+				if(o < n && grp[o] == g) {
 					if(o < cc) continue;             // the earlier cell made the task
 					int ko = -1;
-					for(int j = 0; j < m.nnode[o]; j++)
-						if(m.elemface[(size_t)o*4 + j] == f) ko = j;
+					for(int i = 0; i < m.nnode[o]; i++)
+						if(m.elemface[(size_t)o*4 + i] == f) ko = i;
 					if(ko < 0) throw Error(FVX_ERR_INVALID, "face missing from its right cell");
-					set_code(o, ko, nt, 1);
+					const int jo = (int)(std::lower_bound(cells.begin() + first, cells.end(), o)
+					                     - cells.begin()) - first;
+					set_code(jo, ko, nt, 1);
 				}
 				// a boundary face's left cell is its interior cell; otherwise left = lower index
 				tasks[tb + nt] = f;
-				set_code(cc, k, nt, o < n && o < cc ? 1 : 0);
+				set_code(j, k, nt, o < n && o < cc ? 1 : 0);
 				nt++;
 			}
-		if(nt != ntask) throw Error(FVX_ERR_INVALID, "wave-task count mismatch");
+		}
+		if(nt > 64 || (!m.wave_order && nt != ntask)) throw Error(FVX_ERR_INVALID, "wave-task count mismatch");
 	}
 	m.nwgroup = (int)groups.size();
 	m.d_wtask.upload(tasks);
 	m.d_wgroup.upload(groups);
+	if(!m.wave_order) m.d_wcell.upload(cells);
 	m.d_wslot.upload(slots);
 }
 
@@ -721,10 +776,9 @@ void build_disc(fvx_disc_s& d)
 	d.d_rgrad.alloc((size_t)ne*8);
 	d.d_ughost.alloc((size_t)std::max(m.nbface, 1)*4);
 	d.d_scratch.alloc(4096);
-	// the wave-task flux form where it applies and the cell order packs at least 24 cells per
-	// wave64 group on average (compact orders: Hilbert, structured natural orders); it spends
-	// fewer than 2.7 face evaluations per cell there against the quad form's 4 lanes per cell
-	d.tune.flux_wave = flux_wave_apply(d) && (long)m.nelem >= 24L*m.nwgroup;
+	// the form reported as selected: wave tasks where a caller may select them and the cell order
+	// is compact
+	d.tune.flux_wave = flux_wave_apply(d) && m.wave_order;
 	// Jacobian assembly: workgroups of one wave (both sides of a face in turn) where they fill the
 	// chip several times over, else a pair of waves per 16 cells (98,304 cells 43 against 50 us,
 	// 4,608 cells 15 against 12 us; Roe)

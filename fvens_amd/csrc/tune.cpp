@@ -58,6 +58,7 @@ void autotune_launch(fvx_disc_s& d, const double* u, int reps, std::vector<fvx_t
 	const bool limited = rec == FVX_RECON_VENKATAKRISHNAN || rec == FVX_RECON_BARTHJESPERSEN;
 	const bool visc = d.pc.viscous != 0;
 	const bool wave = flux_wave_apply(d);
+	d.tune.flux_group = 0;
 	for(int kernel = FVX_KERNEL_GRADIENTS; kernel <= FVX_KERNEL_JACOBIAN; kernel++) {
 		if(kernel == FVX_KERNEL_GRADIENTS && !order2) continue;
 		if(kernel == FVX_KERNEL_JACOBIAN && !jac) continue;
@@ -96,6 +97,11 @@ void autotune_launch(fvx_disc_s& d, const double* u, int reps, std::vector<fvx_t
 			for(const fvx_tune_row& w : rows)
 				if(w.kernel == FVX_KERNEL_FLUX && w.ms < bq) { bq = w.ms; d.tune.flux_block = w.block; }
 			d.tune.flux_xcd = bx; d.tune.flux_wave = bw;
+			if(!wave) {       // the wave-task form is not a caller's choice here, but the library's
+				d.tune.flux_group = 1;
+				const double t = T.ms([&] { launch_residual(d, u, r.p, 1, dt.p, s); }, reps, s);
+				d.tune.flux_group = t < best;
+			}
 		}
 		else { d.tune.jac_block = bb; d.tune.jac_xcd = bx; }
 	}

@@ -416,11 +416,11 @@ fvx_status fvx_mpnn_train_step(fvx_mpnn n, int ngraph, const float* targets, con
 /* ---- timing: the TimingData role of the reference (src/ode/aodesolver.hpp:46-67) ---- */
 
 /* Kernel ids for fvx_profile_read and fvx_set_launch / fvx_get_launch. FVX_KERNEL_FLUX_WAVE
- * is the wave-task form of the face-flux pass (inviscid, first-order or linear reconstruction):
- * each wave64 owns a group of consecutive cells and evaluates each face touching them once;
- * setting a launch for it (block 64) selects that form (FVX_ERR_INVALID for a viscous or MUSCL
- * discretisation), setting one for FVX_KERNEL_FLUX selects the quad-per-cell form. The two
- * forms give bitwise equal residuals and time steps; the wave form's time is read as
+ * is the wave-task form of the face-flux pass: each wave64 owns a group of neighbouring cells
+ * and evaluates each face touching them once. Without a setting the library chooses between it
+ * and the quad-per-cell form by size; setting a launch for it (block 64) selects it always
+ * (FVX_ERR_INVALID for a viscous or MUSCL discretisation), setting one for FVX_KERNEL_FLUX
+ * selects the quad form. The two forms give bitwise equal residuals and time steps; the wave form's time is read as
  * FVX_KERNEL_FLUX. */
 enum { FVX_KERNEL_GRADIENTS = 0, FVX_KERNEL_FLUX = 1, FVX_KERNEL_JACOBIAN = 2,
        FVX_KERNEL_PC = 3, FVX_KERNEL_FLUX_WAVE = 4 };

@@ -1,0 +1,73 @@
+"""The wave-task flux pass where the library chooses it by itself: RCM orders, whose groups are
+grown over neighbouring cells, MUSCL and viscous discretisations, and batches. Both forms evaluate
+a face from the same states in the same way and add a cell's slots in the same order, so the
+results are bitwise equal to the quad-per-cell form's."""
+import numpy as np
+import pytest
+
+from fvens_amd import fvx, meshgen, states
+
+pytestmark = pytest.mark.gpu
+
+INVISCID = [(2, "slipwall"), (4, "farfield")]
+VISCOUS = [(4, "inflowoutflow"), (2, "adiabaticwall", (0.0, 0.0))]
+FORMS = [("ROE", "NONE", "first"), ("HLLC", "LEASTSQUARES", "VENKATAKRISHNAN"),
+         ("ROE", "LEASTSQUARES", "VANALBADA"), ("AUSM", "GREENGAUSS", "NONE"),
+         ("LLF", "LEASTSQUARES", "WENO")]
+
+
+def _num(flux, grad, recon):
+    return (fvx.numerics_cfg(flux=flux, gradient="NONE", order2=False) if recon == "first"
+            else fvx.numerics_cfg(flux=flux, gradient=grad, recon=recon))
+
+
+def _phys(viscous, M=0.5, a=1.0):
+    extra = dict(Tinf=288.15, Reinf=5000.0, Pr=0.72, viscous=True) if viscous else {}
+    return fvx.physics_cfg(Minf=M, aoa_deg=a, bcs=VISCOUS if viscous else INVISCID, **extra)
+
+
+# triangles outside quadrilaterals, and quadrilaterals only; 24,640 and 20,007 cells
+@pytest.mark.parametrize("shape", [(224, 80, 30), (247, 81, 0)])
+@pytest.mark.parametrize("viscous", [False, True])
+@pytest.mark.parametrize("form", FORMS, ids=lambda f: f[2])
+def test_single(torch_cuda, shape, viscous, form):
+    import torch
+    raw = meshgen.airfoil_omesh(shape[0], shape[1], shape[2])
+    raw = raw.permuted(fvx.rcm_permutation(raw))
+    assert raw.nelem >= 20000
+    d = fvx.FlowFV(fvx.Mesh(raw), _phys(viscous), _num(*form))
+    u = torch.tensor(states.perturbed_freestream(raw, Minf=0.5, aoa_deg=1.0), device="cuda")
+    out = []
+    for quad in (False, True):
+        if quad:
+            d.set_launch("flux", 256, True)
+        for steps in (True, False):
+            r = torch.full_like(u, 0.5)
+            dt = torch.zeros(raw.nelem, dtype=torch.float64, device="cuda")
+            d.compute_residual(u, r, steps, dt if steps else None)
+            out.append((r, dt))
+    for a, b in zip(out[:2], out[2:]):
+        assert torch.isfinite(a[0]).all()
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("viscous", [False, True])
+def test_batch(torch_cuda, viscous):
+    import torch
+    raw = meshgen.airfoil_omesh(61, 23, 9)
+    raw = raw.permuted(fvx.rcm_permutation(raw))
+    n = 20000 // raw.nelem + 1
+    mach, aoa = np.linspace(0.3, 0.6, n), np.linspace(-2.0, 3.0, n)
+    gm = fvx.Mesh(raw)
+    d = fvx.FlowFV(gm, _phys(viscous), _num(*FORMS[2 if viscous else 1]))
+    b = fvx.Batch(d, mach, aoa)
+    u = torch.tensor(np.stack([states.perturbed_freestream(raw, Minf=m, aoa_deg=a, seed=i)
+                               for i, (m, a) in enumerate(zip(mach, aoa))]), device="cuda")
+    r, dt = torch.zeros_like(u), torch.zeros(u.shape[:2], dtype=torch.float64, device="cuda")
+    b.compute_residual(u, r, True, dt)
+    for i in range(n):
+        di = fvx.FlowFV(gm, _phys(viscous, mach[i], aoa[i]), _num(*FORMS[2 if viscous else 1]))
+        di.set_launch("flux", 256, True)
+        ri, dti = torch.zeros_like(u[i]), torch.zeros_like(dt[i])
+        di.compute_residual(u[i].contiguous(), ri, True, dti)
+        assert torch.equal(r[i], ri) and torch.equal(dt[i], dti), i
