@@ -1,4 +1,5 @@
-/* flux_wave.hpp -- wave-task form of the face-flux / residual-gather pass.
+/* flux_wave.hpp -- wave-task form of the face-flux / residual-gather pass, for first-order and
+ * linear reconstruction.
  *
  * Reference semantics: FlowFV::compute_residual with compute_fluxes and compute_max_timestep
  * (src/spatial/flow_spatial.cpp:488-816); the reconstruction modes are those of flux_kernel.hpp.
@@ -16,9 +17,8 @@
  * Bound by FP64 arithmetic and the latency of the gathers (in Hilbert order on 1.57M cells by
  * HBM): a group holds 25 (quadrilaterals) to 31 cells (half triangles) in any cell order against the
  * quad form's 16 per wave, so the face arithmetic falls by 1.6 to 1.9x. 16 instances of 98,304 cells
- * in RCM order, Roe: 134 us in the quad form, 89 here; viscous MUSCL on 262,144 quadrilaterals: 64
- * and 49. Waves per SIMD: viscous with gradients spills at 4 (98,304 cells 28.3 us at 3, 29.4 at
- * 4), Roe at 7.
+ * in RCM order, Roe, limited: 134 us in the quad form, 86 here. Waves per SIMD: viscous with
+ * gradients spills at 4 (98,304 cells 27.7 us at 3, 30.0 at 4), Roe at 7.
  *
  * Host tables (mesh.cpp, build_wave_tasks): tasks[64 g + t] = the face of task t (-1: no task;
  * the face record holds its left cell and its right cell or -1-ib); groups[g] = {first entry in
@@ -36,7 +36,7 @@
 namespace fvx {
 
 template <int FLUX, int MODE, bool VISC>
-__global__ __launch_bounds__(64, VISC && MODE ? 3 : VISC || MODE == 2 ? 4 : FLUX == 0 ? 6 : 7)
+__global__ __launch_bounds__(64, VISC && MODE ? 3 : VISC ? 4 : FLUX == 0 ? 6 : 7)
 void k_flux_wave(int ncell, const double* __restrict__ u, const double* __restrict__ rgrad,
                  const double* __restrict__ grad, const int* __restrict__ tasks,
                  const int2* __restrict__ groups, const int* __restrict__ gcells,
@@ -86,28 +86,18 @@ void k_flux_wave(int ncell, const double* __restrict__ u, const double* __restri
 			A = fs_both(gp, uL, wL, irL, n);
 			B = fs_both(gp, uR, wR, irR, n);
 		} else {
-			if constexpr(MODE == 1) {
-				double gL[8], r[4];
-				load_grad(rgrad, cL, gL);
-				const double dx = G.mx - xL[0], dy = G.my - xL[1];
-				for(int k = 0; k < 4; k++) r[k] = wL[k] + gL[2*k]*dx + gL[2*k+1]*dy;
-				A = fs_prim(gp, r, n, igm1);
-				if(!bnd) {
-					double gR[8];
-					load_grad(rgrad, cR, gR);
-					const double ex = G.mx - xR[0], ey = G.my - xR[1];
-					for(int k = 0; k < 4; k++) r[k] = wR[k] + gR[2*k]*ex + gR[2*k+1]*ey;
-					B = fs_prim(gp, r, n, igm1);
-				}
+			double gL[8], r[4];
+			load_grad(rgrad, cL, gL);
+			const double dx = G.mx - xL[0], dy = G.my - xL[1];
+			for(int k = 0; k < 4; k++) r[k] = wL[k] + gL[2*k]*dx + gL[2*k+1]*dy;
+			A = fs_prim(gp, r, n, igm1);
+			if(!bnd) {
+				double gR[8];
+				load_grad(rgrad, cR, gR);
+				const double ex = G.mx - xR[0], ey = G.my - xR[1];
+				for(int k = 0; k < 4; k++) r[k] = wR[k] + gR[2*k]*ex + gR[2*k+1]*ey;
+				B = fs_prim(gp, r, n, igm1);
 			} else {
-				double gL[8], gR[8], rl[4], rr[4];
-				load_grad(grad, cL, gL);
-				if(!bnd) load_grad(grad, cR, gR);
-				muscl_states(wL, wR, gL, gR, xR[0] - xL[0], xR[1] - xL[1], bnd, rl, rr);
-				A = fs_prim(gp, rl, n, igm1);
-				if(!bnd) B = fs_prim(gp, rr, n, igm1);
-			}
-			if(bnd) {
 				const double UL[4] = { A.r, A.mx, A.my, A.E };
 				double UG[4];
 				ghost_state(gp, bt, bc, UL, n, UG);

@@ -44,6 +44,22 @@ struct BatchArg {
 	const double* cfl = nullptr;           ///< per-instance CFL numbers (Jacobian kernel)
 };
 
+/// Tables of the one-launch residual (residual_patch.hpp), on the device.
+constexpr int PATCH_TASKS = 256;      ///< face tasks, and threads, per patch
+constexpr int PATCH_MAX = 256;        ///< patch and halo cells
+struct PatchGroup {
+	int list, nown, nlist, nstate;     ///< first entry in cells; patch cells, those and halo, all entries
+	int local, slots;                  ///< first entries in local and slots
+};
+struct PatchTables {
+	const PatchGroup* groups;
+	const int* cells;                  ///< per patch its cells, its halo, then further cells and -1 - boundary faces
+	const unsigned short* local;       ///< [patch and halo cells][4] list entry behind each slot, 0xffff unused
+	const int* face;                   ///< [patch][256] face of each task, -1 none
+	const unsigned* sides;             ///< [patch][256] list entries of its left and right side (low, high 16 bits)
+	const ushort4* slots;              ///< per patch cell and slot 2 task + side, 0xffff unused
+};
+
 /// Host-side description of a launch's instances: the device list of active instance ids
 /// (null for a single instance) and how many there are (gridDim.y).
 struct Inst {
@@ -104,6 +120,13 @@ struct fvx_mesh_s {
 	fvx::DBuf<int> d_wcell;                // [nelem] the groups' cells, group after group (!wave_order)
 	fvx::DBuf<int> d_wtask;                // [ngroup][64] face of each task, -1 none
 	fvx::DBuf<int2> d_wgroup;              // [ngroup] {first entry in d_wcell, cells}
+	// patches of the one-launch residual (residual_patch.hpp)
+	int npatch = 0, patch_nw = 0, patch_ns = 0; // the most states, and patch and halo cells, in one
+	fvx::DBuf<fvx::PatchGroup> d_pgroup;
+	fvx::DBuf<int> d_pcell, d_pface;
+	fvx::DBuf<unsigned short> d_plocal;
+	fvx::DBuf<unsigned> d_psides;
+	fvx::DBuf<ushort4> d_pslot;
 	fvx::DBuf<unsigned> d_wslot;           // [ngroup][64] per cell: byte k = 2 task + side of
 	                                       // slot k, 0xff unused
 };
@@ -121,6 +144,7 @@ struct Profiler {
 	long count[NKERNEL] = {};
 	void start(int k, hipStream_t s);
 	void stop(hipStream_t s);
+	void skip(int k);                      ///< counts a pass done inside another kernel (no time)
 	void collect();
 	void reset();
 	~Profiler();
@@ -139,7 +163,7 @@ struct Tuning {
 	int flux_block = 256, grad_block = 256, jac_block = 256;
 	int flux_xcd = 1, grad_xcd = 1, jac_xcd = 1;
 	int flux_wave = 0;     ///< 1: wave-task form of the flux pass, as selected by a caller
-	int flux_group = 1;    ///< 1: wave-task form whatever flux_wave says (nothing selected)
+	int flux_group = 1;    ///< 1: no form selected, the library's choice by kind and size
 };
 }
 
@@ -272,6 +296,7 @@ void find_lines(const fvx_mesh_desc& d, double threshold, std::vector<std::vecto
 void line_order(const fvx_mesh_desc& d, double threshold, int graph_ordering, int* perm);
 void hilbert_order(const fvx_mesh_desc& d, int* perm);
 void build_wave_tasks(fvx_mesh_s& m);
+void build_patches(fvx_mesh_s& m);
 void build_disc(fvx_disc_s& d);
 GasParams make_gas(const fvx_physics_cfg& p);
 

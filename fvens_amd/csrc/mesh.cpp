@@ -229,6 +229,7 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 	m.d_bhost.upload(host);
 	m.d_btag.upload(m.btag);
 	build_wave_tasks(m);
+	build_patches(m);
 }
 
 /* Tables of the wave-task flux kernel (flux_wave.hpp). Groups of at most 64 cells grow while the
@@ -346,6 +347,137 @@ void build_wave_tasks(fvx_mesh_s& m)
 	m.d_wgroup.upload(groups);
 	if(!m.wave_order) m.d_wcell.upload(cells);
 	m.d_wslot.upload(slots);
+}
+
+/* Tables of the one-launch residual (residual_patch.hpp). Patches grow like the groups of
+ * build_wave_tasks (consecutive cells in a compact order) while their faces make at most
+ * PATCH_TASKS tasks and patch and halo hold at most PATCH_MAX cells. */
+void build_patches(fvx_mesh_s& m)
+{
+	const int n = m.nelem;
+	std::vector<int> cells, face, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand, entry(n, -1), far(n, -1);
+	std::vector<PatchGroup> groups;
+	std::vector<unsigned short> local;
+	std::vector<unsigned> sides;
+	std::vector<ushort4> slots;
+	int seed = 0, nwmax = 0, nsmax = 192, done = 0; // 192: room for the task results
+	while(done < n) {
+		const int g = (int)groups.size(), first = (int)cells.size();
+		while(grp[seed] >= 0) seed++;
+		cand.assign(1, seed);
+		seen[seed] = g;
+		links[seed] = met[seed] = 0;
+		int ntask = 0, nmet = 1, nown = 0;
+		// listed cells: the patch's and those seen next to it; cells of other groups are seen too
+		while(true) {
+			int best = -1, bl = 0, bo = 0;
+			if(m.wave_order) {                        // the next cell of the order, or none
+				const int c = seed + nown;
+				if(c == n) break;
+				if(seen[c] != g) { seen[c] = g; links[c] = 0; met[c] = nmet++; cand.push_back(c); }
+				if(ntask + m.nnode[c] - links[c] <= PATCH_TASKS
+				   && nmet + m.nnode[c] - links[c] <= PATCH_MAX)
+					best = (int)(std::find(cand.begin(), cand.end(), c) - cand.begin());
+				else if(links[c] == 0) { cand.pop_back(); seen[c] = -1; } // not even halo
+			}
+			else for(int i = 0; i < (int)cand.size(); i++) {
+				const int c = cand[i], l = links[c];
+				if(grp[c] >= 0) continue;              // of another patch: halo only
+				if(ntask + m.nnode[c] - l > PATCH_TASKS || nmet + m.nnode[c] - l > PATCH_MAX) continue;
+				int open = 0;
+				for(int k = 0; k < m.nnode[c]; k++) {
+					const int o = m.esuel[(size_t)c*4 + k];
+					open += o < n && grp[o] < 0;
+				}
+				if(best < 0 || l > bl || (l == bl && (open < bo || (open == bo && met[c] < met[cand[best]])))) {
+					best = i; bl = l; bo = open;
+				}
+			}
+			if(best < 0) break;
+			const int c = cand[best];
+			cand[best] = cand.back();
+			cand.pop_back();
+			grp[c] = g;
+			cells.push_back(c);
+			nown++;
+			ntask += m.nnode[c] - links[c];
+			for(int k = 0; k < m.nnode[c]; k++) {
+				const int o = m.esuel[(size_t)c*4 + k];
+				if(o >= n) continue;
+				if(grp[o] == g) continue;
+				if(seen[o] != g) { seen[o] = g; links[o] = 0; met[o] = nmet++; cand.push_back(o); }
+				links[o]++;
+			}
+		}
+		done += nown;
+		std::sort(cells.begin() + first, cells.end());
+		std::sort(cand.begin(), cand.end());
+		cells.insert(cells.end(), cand.begin(), cand.end());
+		const int nl = (int)cells.size() - first;
+		nsmax = std::max(nsmax, nl);
+		for(int i = 0; i < nl; i++) entry[cells[first + i]] = i;
+		const size_t tb = face.size();
+		face.resize(tb + PATCH_TASKS, -1);
+		sides.resize(tb + PATCH_TASKS, 0u);
+		const size_t lb = local.size();
+		local.resize(lb + 4*(size_t)nl, 0xffff);
+		for(int i = 0; i < nl; i++) {
+			const int c = cells[first + i];
+			for(int k = 0; k < m.nnode[c]; k++) {
+				const int o = m.esuel[(size_t)c*4 + k];
+				unsigned short& e = local[lb + 4*(size_t)i + k];
+				if(o < n && seen[o] == g) e = (unsigned short)entry[o];
+				else if(o < n && far[o] == g) e = (unsigned short)entry[o];
+				else {
+					e = (unsigned short)(cells.size() - first);
+					if(o < n) { far[o] = g; entry[o] = e; }
+					// boundary faces are numbered first
+					cells.push_back(o < n ? o : -1 - m.elemface[(size_t)c*4 + k]);
+				}
+			}
+		}
+		const int nst = (int)cells.size() - first;
+		nwmax = std::max(nwmax, nst);
+		const size_t sb = slots.size();
+		slots.resize(sb + nown, make_ushort4(0xffff, 0xffff, 0xffff, 0xffff));
+		auto set_code = [&](int j, int k, int task, int side) {
+			(&slots[sb + j].x)[k] = (unsigned short)(2*task + side);
+		};
+		int nt = 0;
+		for(int j = 0; j < nown; j++) {
+			const int cc = cells[first + j];
+			for(int k = 0; k < m.nnode[cc]; k++) {
+				const int o = m.esuel[(size_t)cc*4 + k], f = m.elemface[(size_t)cc*4 + k];
+				const bool right = o < n && o < cc;     // cc is the face's right cell
+				if(o < n && grp[o] == g) {
+					if(right) continue;                  // the earlier cell made the task
+					int ko = -1;
+					for(int i = 0; i < m.nnode[o]; i++)
+						if(m.elemface[(size_t)o*4 + i] == f) ko = i;
+					if(ko < 0) throw Error(FVX_ERR_INVALID, "face missing from its right cell");
+					set_code(entry[o], ko, nt, 1);
+				}
+				const unsigned e = local[lb + 4*(size_t)j + k];
+				face[tb + nt] = f;
+				sides[tb + nt] = right ? e | (unsigned)j << 16 : (unsigned)j | e << 16;
+				set_code(j, k, nt, right);
+				nt++;
+			}
+		}
+		if(nt != ntask) throw Error(FVX_ERR_INVALID, "patch task count mismatch");
+		groups.push_back(PatchGroup{first, nown, nl, nst, (int)(lb/4), (int)sb});
+	}
+	// the default limit of a workgroup's LDS (never met with PATCH_MAX cells of ordinary meshes)
+	if((4*(size_t)nwmax + 10*(size_t)nsmax)*sizeof(double) > 65536) return;
+	m.npatch = (int)groups.size();
+	m.patch_nw = nwmax;
+	m.patch_ns = nsmax;
+	m.d_pgroup.upload(groups);
+	m.d_pcell.upload(cells);
+	m.d_plocal.upload(local);
+	m.d_pface.upload(face);
+	m.d_psides.upload(sides);
+	m.d_pslot.upload(slots);
 }
 
 /* Lines of strongly coupled cells (findLines, src/mesh/meshordering.cpp:199-262). Each cell's

@@ -31,6 +31,14 @@ FVX_DECL_FLUX(5) FVX_DECL_FLUX(6)
 FVX_DECL_FLUXW(0) FVX_DECL_FLUXW(1) FVX_DECL_FLUXW(2) FVX_DECL_FLUXW(3) FVX_DECL_FLUXW(4)
 FVX_DECL_FLUXW(5) FVX_DECL_FLUXW(6)
 #undef FVX_DECL_FLUXW
+#define FVX_DECL_PATCH(ID) void launch_residual_patch_##ID(int lim, int mode, bool visc, int ncell, \
+	int npatch, int nw, int ns, const double* u, const PatchTables& pt, const double* soff, \
+	const double* gcoef, const double* eps2, const FaceGeom* fg, const double* centre, \
+	const double* area, const int* bcid, const GasParams* gpa, const BCTable* bta, double* res, \
+	double* dt, int getdt, const BatchArg& ba, int nact, int xcd, hipStream_t s);
+FVX_DECL_PATCH(0) FVX_DECL_PATCH(1) FVX_DECL_PATCH(2) FVX_DECL_PATCH(3) FVX_DECL_PATCH(4)
+FVX_DECL_PATCH(5) FVX_DECL_PATCH(6)
+#undef FVX_DECL_PATCH
 
 /// Ghost states of the boundary faces from their cells' states (the reference's
 /// compute_boundary_states, src/spatial/flow_spatial.cpp:74-82, called at :679 before the
@@ -273,6 +281,11 @@ void Profiler::stop(hipStream_t s)
 	used++;
 }
 
+void Profiler::skip(int k)
+{
+	if(on) count[k]++;
+}
+
 void Profiler::collect()
 {
 	for(size_t i = 0; i < used; i++) {
@@ -349,6 +362,32 @@ void launch_residual(const fvx_disc_s& d, const double* u, double* r, int gettim
 	int mode = 0;
 	const double* rg = nullptr;
 	const double* ug = nullptr;
+	// gradients and fluxes in one launch (residual_patch.hpp) unless a form was selected; not for WENO
+	// weights, which need the neighbours' gradients, nor viscous terms with a limiter, which need
+	// two gradients per cell. Faster than the separate passes from 4,608 cells (9 against 13 us) to
+	// 1,572,864 (176 against 207).
+	if(order2 && d.tune.flux_group && m.npatch > 0 && rec != FVX_RECON_WENO) {
+		const int lim = rec == FVX_RECON_VENKATAKRISHNAN ? 1 : rec == FVX_RECON_BARTHJESPERSEN ? 2 : 0;
+		if(!(visc && lim)) {
+			const PatchTables pt = { m.d_pgroup.p, m.d_pcell.p, m.d_plocal.p, m.d_pface.p, m.d_psides.p,
+			                         m.d_pslot.p };
+			mode = rec == FVX_RECON_VANALBADA ? 2 : 1;
+			d.prof.skip(PROF_GRADIENTS);         // part of the one launch
+			d.prof.start(PROF_FLUX, s);
+			switch(d.nc.conv_numflux) {
+#define FVX_P(ID) case ID: launch_residual_patch_##ID(lim, mode, visc, m.nelem, m.npatch, m.patch_nw, \
+	m.patch_ns, u, pt, m.d_soff.p, d.d_gcoef.p, d.d_eps2.p, m.d_fgeom.p, m.d_centre.p, m.d_area.p, \
+	d.d_bcid.p, ba.gp ? ba.gp : d.d_gas.p, d.d_bct.p, r, dt, gettimesteps, ba, nact, \
+	d.tune.flux_xcd, s); break;
+			FVX_P(0) FVX_P(1) FVX_P(2) FVX_P(3) FVX_P(4) FVX_P(5) FVX_P(6)
+#undef FVX_P
+			default: throw Error(FVX_ERR_INVALID, "unknown flux");
+			}
+			FVX_HIP(hipGetLastError());
+			d.prof.stop(s);
+			return;
+		}
+	}
 	if(order2) {
 		const bool limited = rec == FVX_RECON_VENKATAKRISHNAN || rec == FVX_RECON_BARTHJESPERSEN;
 		if(limited) {
@@ -367,8 +406,8 @@ void launch_residual(const fvx_disc_s& d, const double* u, double* r, int gettim
 	d.prof.start(PROF_FLUX, s);
 	// wave-task form (flux_wave.hpp): each face evaluated once per wave64 cell group. Below 20,000
 	// cells the quad form's shorter chain per wave is as fast or faster (residuals of 15,000 cells,
-	// viscous: 14.4 us, 15.1 in wave tasks; 38,400 cells 19.7 and 18.4).
-	if((d.tune.flux_group && (long)m.nelem*nact >= 20000)
+	// viscous: 14.4 us, 15.1 in wave tasks; 38,400 cells 18.9 and 17.8; first order 9.9 and 9.6).
+	if((d.tune.flux_group && mode != 2 && (long)m.nelem*nact >= 20000)
 	   || (d.tune.flux_wave && flux_wave_apply(d))) {
 		switch(d.nc.conv_numflux) {
 #define FVX_W(ID) case ID: launch_flux_wave_##ID(mode, visc, m.nelem, m.nwgroup, u, rg, ug, \

@@ -97,11 +97,9 @@ void autotune_launch(fvx_disc_s& d, const double* u, int reps, std::vector<fvx_t
 			for(const fvx_tune_row& w : rows)
 				if(w.kernel == FVX_KERNEL_FLUX && w.ms < bq) { bq = w.ms; d.tune.flux_block = w.block; }
 			d.tune.flux_xcd = bx; d.tune.flux_wave = bw;
-			if(!wave) {       // the wave-task form is not a caller's choice here, but the library's
-				d.tune.flux_group = 1;
-				const double t = T.ms([&] { launch_residual(d, u, r.p, 1, dt.p, s); }, reps, s);
-				d.tune.flux_group = t < best;
-			}
+			// the library's own choice of form stays where it beats every form a caller may select
+			d.tune.flux_group = 1;
+			d.tune.flux_group = T.ms([&] { launch_residual(d, u, r.p, 1, dt.p, s); }, reps, s) < best;
 		}
 		else { d.tune.jac_block = bb; d.tune.jac_xcd = bx; }
 	}

@@ -417,10 +417,11 @@ fvx_status fvx_mpnn_train_step(fvx_mpnn n, int ngraph, const float* targets, con
 
 /* Kernel ids for fvx_profile_read and fvx_set_launch / fvx_get_launch. FVX_KERNEL_FLUX_WAVE
  * is the wave-task form of the face-flux pass: each wave64 owns a group of neighbouring cells
- * and evaluates each face touching them once. Without a setting the library chooses between it
- * and the quad-per-cell form by size; setting a launch for it (block 64) selects it always
- * (FVX_ERR_INVALID for a viscous or MUSCL discretisation), setting one for FVX_KERNEL_FLUX
- * selects the quad form. The two forms give bitwise equal residuals and time steps; the wave form's time is read as
+ * and evaluates each face touching them once. Without a setting the library does second-order
+ * residuals in one launch (their time is read as FVX_KERNEL_FLUX, the gradients count with none),
+ * where that does not apply in either form by size; setting a launch for FVX_KERNEL_FLUX_WAVE
+ * (block 64) selects separate gradients and the wave form (FVX_ERR_INVALID for a viscous or MUSCL
+ * discretisation), setting one for FVX_KERNEL_FLUX the quad form. All give bitwise equal residuals and time steps; the wave form's time is read as
  * FVX_KERNEL_FLUX. */
 enum { FVX_KERNEL_GRADIENTS = 0, FVX_KERNEL_FLUX = 1, FVX_KERNEL_JACOBIAN = 2,
        FVX_KERNEL_PC = 3, FVX_KERNEL_FLUX_WAVE = 4 };

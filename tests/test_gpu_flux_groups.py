@@ -1,7 +1,8 @@
-"""The wave-task flux pass where the library chooses it by itself: RCM orders, whose groups are
-grown over neighbouring cells, MUSCL and viscous discretisations, and batches. Both forms evaluate
-a face from the same states in the same way and add a cell's slots in the same order, so the
-results are bitwise equal to the quad-per-cell form's."""
+"""Residuals in the forms the library chooses by itself: second-order ones in one launch over
+patches of cells, first-order, WENO and limited viscous ones with wave tasks from 20,000 cells on,
+in RCM orders, whose groups are grown over neighbouring cells, and in Hilbert order. All forms
+evaluate gradients and faces from the same states in the same way and add a cell's slots in the
+same order, so the results are bitwise equal to the separate passes in quad-per-cell form."""
 import numpy as np
 import pytest
 
@@ -49,6 +50,32 @@ def test_single(torch_cuda, shape, viscous, form):
     for a, b in zip(out[:2], out[2:]):
         assert torch.isfinite(a[0]).all()
         assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+# a patch with one cell, one that is the whole mesh, one task too many, triangles
+@pytest.mark.parametrize("shape", [(1, 1, 0), (10, 10, 0), (11, 11, 0), (45, 21, 2), (40, 33, 33)])
+@pytest.mark.parametrize("order", ["rcm", "hilbert"])
+@pytest.mark.parametrize("viscous", [False, True])
+@pytest.mark.parametrize("form", FORMS[1:4] + [("VANLEER", "GREENGAUSS", "BARTHJESPERSEN")],
+                         ids=lambda f: f[2])
+def test_patches(torch_cuda, shape, order, viscous, form):
+    import torch
+    raw = meshgen.gaussian_bump(*shape)
+    raw = raw.permuted(fvx.rcm_permutation(raw) if order == "rcm" else fvx.hilbert_permutation(raw))
+    extra = dict(Tinf=288.15, Reinf=5000.0, Pr=0.72, viscous=True) if viscous else {}
+    bcs = [(2, "adiabaticwall", (0.0, 0.0)) if viscous else (2, "slipwall"),
+           (3, "inflowoutflow"), (4, "inflowoutflow")]
+    d = fvx.FlowFV(fvx.Mesh(raw), fvx.physics_cfg(Minf=0.5, bcs=bcs, **extra), _num(*form))
+    u = torch.tensor(states.perturbed_freestream(raw, Minf=0.5, L=3.0), device="cuda")
+    out = []
+    for _ in range(2):
+        r = torch.full_like(u, 0.5)
+        dt = torch.zeros(raw.nelem, dtype=torch.float64, device="cuda")
+        d.compute_residual(u, r, True, dt)
+        out.append((r, dt))
+        d.set_launch("flux", 256, True)
+    assert torch.isfinite(out[0][0]).all()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
 @pytest.mark.parametrize("viscous", [False, True])
