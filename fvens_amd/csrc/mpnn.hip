@@ -159,7 +159,8 @@ __device__ __forceinline__ void tile_get_a(const float* t, int lane, int s, floa
 /// fp32 rows (h, Q, da, the gradients) are kept in an order of their own: position 32 s + 16 b +
 /// 4 g + i holds channel 32 s + 8 g + 4 b + i, so that each of the two 16-byte accesses of a lane's
 /// 8 channels makes, with the other lane groups, a full 64-byte segment of every row. In channel
-/// order every access touched twice the segments: k_layer_bwd took 643 us instead of 565.
+/// order every access touched twice the segments: k_layer_bwd took 643 us instead of 565 (at two
+/// waves per SIMD).
 __device__ __forceinline__ void load_row(const float* __restrict__ rows, size_t r, int s, int lane,
                                          float* v)
 {
@@ -188,6 +189,28 @@ __device__ __forceinline__ void tile_mm(const bf16x8* f, int lane, const bf16x8*
 	for(int s = 0; s < S; s++)
 #pragma unroll
 		for(int j = 0; j < 4; j++) acc[j] = mfma(a[s], f[(s*NT + J0 + j)*64 + lane], acc[j]);
+}
+
+template <int CTRL> __device__ __forceinline__ float dpp_f(float v)
+{
+	return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF,
+	                                                          0xF, false));
+}
+/// Sum of v[e] over the 16 rows (lanes of equal lane >> 4), for e = lane & 7. Halves the values in
+/// each exchange: 29 instructions for 8 sums, and one register per sum to keep them over the tiles.
+__device__ __forceinline__ float row_sums8(int lane, const float (&v)[8])
+{
+	const bool h4 = lane & 4, h2 = lane & 2, h1 = lane & 1;
+	float a[8], b[4], c[2];
+#pragma unroll
+	for(int e = 0; e < 8; e++) a[e] = v[e] + dpp_f<0x128>(v[e]);              // row_ror:8
+#pragma unroll
+	for(int e = 0; e < 4; e++)
+		b[e] = (h4 ? a[4 + e] : a[e]) + dpp_f<0x141>(h4 ? a[e] : a[4 + e]);    // row_half_mirror
+#pragma unroll
+	for(int e = 0; e < 2; e++)
+		c[e] = (h2 ? b[2 + e] : b[e]) + dpp_f<0x4E>(h2 ? b[e] : b[2 + e]);     // lane ^ 2
+	return (h1 ? c[1] : c[0]) + dpp_f<0xB1>(h1 ? c[0] : c[1]);               // lane ^ 1
 }
 
 /// Fragments [s][j0 .. j0 + nj) of a packed matrix of NT columns of fragments to LDS.
@@ -319,7 +342,8 @@ __device__ __forceinline__ void update_bwd_tile(const bf16x8* wf, float* t, int 
 /// Bound by HBM and the gathers: per row h 256 + Q about 256 + edges 80 read, h 256 + Q 256
 /// (+ 168 in training) written. P|Q written by a launch of its own and read back took 565 us per
 /// layer on 786,432 rows (117 + 449), this takes 277 (1.1 GB, 77% of the copy rate). Three workgroups a
-/// compute unit; LAST in training holds 69 sums per lane, so two.
+/// compute unit, two (by LDS) for LAST in training, which takes 345 us with the decoder and its
+/// backward pass (in launches of their own 620: 277 + 198 + 152).
 template <bool TRAIN, bool LAST>
 __global__ void __launch_bounds__(RB, TRAIN && LAST ? 2 : 3)
 k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict__ q,
@@ -347,8 +371,7 @@ k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict
 	__syncthreads();
 	const int lane = threadIdx.x & 63, wave = wave_id(), R = g.R;
 	float* t = tile + wave*TILE;
-	float dacc[TRAIN && LAST ? 69 : 1];
-	for(float& v : dacc) v = 0.f;
+	float dsum[2][FO] = {}, dacc[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
 	const Tiles ts = my_tiles(ntile);
 	for(int tt = ts.t; tt < ts.end; tt += ts.step) {
 		const int r = 16*tt + (lane & 15), rc = min(r, R - 1);
@@ -468,8 +491,8 @@ k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict
 				for(int o = 0; o < FO; o++) {
 					const float d = r < R ? yo[o] - tv[o] : 0.f;
 					dy[o] = (float)(2.0*(double)d*inv_count);
-					dacc[64 + o] += dy[o];
-					dacc[68] += d*d;
+					dacc[o] += dy[o];
+					dacc[4] += d*d;
 				}
 #pragma unroll
 				for(int s = 0; s < 2; s++)
@@ -477,8 +500,15 @@ k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict
 					for(int e = 0; e < 8; e++) {
 						const f32x4 d = *reinterpret_cast<const f32x4*>(wd + (32*s + 8*(lane >> 4) + e)*FO);
 						gn[s][e] = dy[0]*d[0] + dy[1]*d[1] + dy[2]*d[2] + dy[3]*d[3];
+					}
 #pragma unroll
-						for(int o = 0; o < FO; o++) dacc[(8*s + e)*FO + o] += hv[s][e]*dy[o];
+				for(int s = 0; s < 2; s++)
+#pragma unroll
+					for(int o = 0; o < FO; o++) {
+						float v[8];
+#pragma unroll
+						for(int e = 0; e < 8; e++) v[e] = hv[s][e]*dy[o];
+						dsum[s][o] += row_sums8(lane, v);
 					}
 				update_bwd_tile(wf + 24*64, t, lane, r, r < R, gn, um, id, dpre, gpart, da);
 			}
@@ -489,16 +519,18 @@ k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict
 		float* red = t;
 		wave_sync();
 #pragma unroll
-		for(int i = 0; i < 69; i++) {
+		for(int s = 0; s < 2; s++)
+#pragma unroll
+			for(int o = 0; o < FO; o++)
+				if((lane & 15) < 8) red[(32*s + 8*(lane >> 4) + (lane & 7))*FO + o] = dsum[s][o];
+#pragma unroll
+		for(int i = 0; i < 5; i++) {
 			float v = dacc[i];
 			v += __shfl_xor(v, 8);
 			v += __shfl_xor(v, 4);
 			v += __shfl_xor(v, 2);
 			v += __shfl_xor(v, 1);
-			if((lane & 15) == 0) {
-				if(i < 64) red[(32*(i >> 5) + 8*(lane >> 4))*FO + (i & 31)] = v;
-				else if(lane == 0) red[256 + i - 64] = v;
-			}
+			if(lane == 0) red[256 + i] = v;
 		}
 		__syncthreads();
 		for(int i = threadIdx.x; i < 261; i += RB) {
@@ -520,11 +552,11 @@ k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict
 ///
 /// Bound by HBM and the gathers of da: per row da 256 + about 256 + masks 64 + edges 80 + gpart 256
 /// read, dP|dQ 256 + dpre 128 + gpart 256 + da 256 written. Three launches that recomputed the
-/// messages from P|Q took 1,148 us per layer on 786,432 rows (790 + 166 + 192), this takes 565
-/// (1.5 GB): the 80 partial sums per lane leave two waves per SIMD, whose waits for the gathers
-/// are the rest.
+/// messages from P|Q took 1,148 us per layer on 786,432 rows (790 + 166 + 192), this takes 403
+/// (1.5 GB, 71% of the copy rate). Three waves per SIMD: with the sums of dWe and dbm kept per lane
+/// and row (80 registers) instead of added over the rows of each tile, two waves took 565.
 template <bool FIRST>
-__global__ void __launch_bounds__(RB, 2) k_layer_bwd(Graph g, int ntile,
+__global__ void __launch_bounds__(RB, 3) k_layer_bwd(Graph g, int ntile,
                                                      const float* __restrict__ da,
                                                      const unsigned* __restrict__ mmask,
                                                      const bf16_t* __restrict__ fbpq,
@@ -543,13 +575,9 @@ __global__ void __launch_bounds__(RB, 2) k_layer_bwd(Graph g, int ntile,
 	__syncthreads();
 	const int lane = threadIdx.x & 63, wave = wave_id(), R = g.R, gl = lane >> 4;
 	float* t = tile + wave*TILE;
-	float wacc[5][2][8];
+	float wsum[5][2];
 #pragma unroll
-	for(int f = 0; f < 5; f++)
-#pragma unroll
-		for(int s = 0; s < 2; s++)
-#pragma unroll
-			for(int e = 0; e < 8; e++) wacc[f][s][e] = 0.f;
+	for(int f = 0; f < 5; f++) wsum[f][0] = wsum[f][1] = 0.f;
 	const Tiles ts = my_tiles(ntile);
 	for(int tt = ts.t; tt < ts.end; tt += ts.step) {
 		const int r = 16*tt + (lane & 15), rc = min(r, R - 1);
@@ -581,6 +609,11 @@ __global__ void __launch_bounds__(RB, 2) k_layer_bwd(Graph g, int ntile,
 			}
 #pragma unroll
 			for(int e = 0; e < 8; e++) { dP[e] = 0.f; dQ[e] = 0.f; }
+			float we[4][8];
+#pragma unroll
+			for(int f = 0; f < 4; f++)
+#pragma unroll
+				for(int e = 0; e < 8; e++) we[f][e] = 0.f;
 #pragma unroll
 			for(int k = 0; k < 4; k++) {
 				const f32x4 ef = *reinterpret_cast<const f32x4*>(g.edge + ((size_t)node*4 + k)*4);
@@ -589,12 +622,13 @@ __global__ void __launch_bounds__(RB, 2) k_layer_bwd(Graph g, int ntile,
 					const float ds = (mo >> (8*k + e)) & 1u ? d[e] : 0.f;
 					dP[e] += ds;
 #pragma unroll
-					for(int f = 0; f < 4; f++) wacc[f][s][e] += ef[f]*ds;
+					for(int f = 0; f < 4; f++) we[f][e] += ef[f]*ds;
 					dQ[e] += (mn[k] >> e) & 1u ? dn[k][e] : 0.f;
 				}
 			}
 #pragma unroll
-			for(int e = 0; e < 8; e++) wacc[4][s][e] += dP[e];
+			for(int f = 0; f < 4; f++) wsum[f][s] += row_sums8(lane, we[f]);
+			wsum[4][s] += row_sums8(lane, dP);
 			a[s] = to_frag(dP);
 			a[2 + s] = to_frag(dQ);
 			if(ok) {
@@ -620,22 +654,13 @@ __global__ void __launch_bounds__(RB, 2) k_layer_bwd(Graph g, int ntile,
 			update_bwd_tile(wf + 16*64, t, lane, r, ok, gn, mk, g.invdeg[node], dpre, gpart, daout);
 		}
 	}
-	// partial layout: We[f][c] (256), bm[c] (64): sum over the 16 rows of a tile by lane
-	// exchanges, then over the waves in order
+	// partial layout: We[f][c] (256), bm[c] (64), added over the waves in order
 	wave_sync();
 #pragma unroll
 	for(int f = 0; f < 5; f++)
 #pragma unroll
 		for(int s = 0; s < 2; s++)
-#pragma unroll
-			for(int e = 0; e < 8; e++) {
-				float v = wacc[f][s][e];
-				v += __shfl_xor(v, 8);
-				v += __shfl_xor(v, 4);
-				v += __shfl_xor(v, 2);
-				v += __shfl_xor(v, 1);
-				if((lane & 15) == 0) t[f*W + 32*s + 8*gl + e] = v;
-			}
+			if((lane & 15) < 8) t[f*W + 32*s + 8*gl + (lane & 7)] = wsum[f][s];
 	__syncthreads();
 	for(int i = threadIdx.x; i < 320; i += RB) {
 		float s = 0.f;
