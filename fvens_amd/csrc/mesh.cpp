@@ -232,6 +232,14 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 	build_patches(m);
 }
 
+static std::vector<int> open_neighbours(const fvx_mesh_s& m)
+{
+	std::vector<int> open(m.nelem, 0);
+	for(int c = 0; c < m.nelem; c++)
+		for(int k = 0; k < m.nnode[c]; k++) open[c] += m.esuel[(size_t)c*4 + k] < m.nelem;
+	return open;
+}
+
 /* Tables of the wave-task flux kernel (flux_wave.hpp). Groups of at most 64 cells grow while the
  * faces touching the group make at most 64 tasks: a cell adds one task per face, less the faces
  * to cells already in the group (those faces' tasks serve both cells).
@@ -266,6 +274,7 @@ void build_wave_tasks(fvx_mesh_s& m)
 	}
 	m.wave_order = n >= 24L*(long)consec.size();
 	std::vector<int> tasks, cells, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand;
+	std::vector<int> open = open_neighbours(m);   // neighbours without a group
 	std::vector<int2> groups;
 	std::vector<unsigned> slots;
 	cells.reserve(n);
@@ -284,14 +293,9 @@ void build_wave_tasks(fvx_mesh_s& m)
 			int best = -1, bl = 0, bo = 0;
 			for(int i = 0; i < (int)cand.size(); i++) {
 				const int c = cand[i], l = links[c];
-				if(ntask + m.nnode[c] - l > 64) continue;
-				int open = 0;
-				for(int k = 0; k < m.nnode[c]; k++) {
-					const int o = m.esuel[(size_t)c*4 + k];
-					open += o < n && grp[o] < 0;
-				}
-				if(best < 0 || l > bl || (l == bl && (open < bo || (open == bo && met[c] < met[cand[best]])))) {
-					best = i; bl = l; bo = open;
+				if(l < bl || ntask + m.nnode[c] - l > 64) continue;
+				if(best < 0 || l > bl || (l == bl && (open[c] < bo || (open[c] == bo && met[c] < met[cand[best]])))) {
+					best = i; bl = l; bo = open[c];
 				}
 			}
 			if(best < 0) break;
@@ -303,7 +307,9 @@ void build_wave_tasks(fvx_mesh_s& m)
 			ntask += m.nnode[c] - links[c];
 			for(int k = 0; k < m.nnode[c]; k++) {
 				const int o = m.esuel[(size_t)c*4 + k];
-				if(o >= n || grp[o] >= 0) continue;
+				if(o >= n) continue;
+				open[o]--;
+				if(grp[o] >= 0) continue;
 				if(seen[o] != g) { seen[o] = g; links[o] = 0; met[o] = nmet++; cand.push_back(o); }
 				links[o]++;
 			}
@@ -355,20 +361,25 @@ void build_wave_tasks(fvx_mesh_s& m)
 void build_patches(fvx_mesh_s& m)
 {
 	const int n = m.nelem;
-	std::vector<int> cells, face, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand, entry(n, -1), far(n, -1);
+	std::vector<int> cells, face, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand, rim, entry(n, -1), far(n, -1);
+	std::vector<int> open = open_neighbours(m);   // neighbours without a patch
 	std::vector<PatchGroup> groups;
 	std::vector<unsigned short> local;
 	std::vector<unsigned> sides;
 	std::vector<ushort4> slots;
+	cells.reserve(2*(size_t)n);
+	local.reserve(6*(size_t)n);
+	slots.reserve(n);
 	int seed = 0, nwmax = 0, nsmax = 192, done = 0; // 192: room for the task results
 	while(done < n) {
 		const int g = (int)groups.size(), first = (int)cells.size();
 		while(grp[seed] >= 0) seed++;
+		// listed cells: the patch's and those next to it, without a patch (cand) or in another (rim)
 		cand.assign(1, seed);
+		rim.clear();
 		seen[seed] = g;
 		links[seed] = met[seed] = 0;
 		int ntask = 0, nmet = 1, nown = 0;
-		// listed cells: the patch's and those seen next to it; cells of other groups are seen too
 		while(true) {
 			int best = -1, bl = 0, bo = 0;
 			if(m.wave_order) {                        // the next cell of the order, or none
@@ -382,15 +393,10 @@ void build_patches(fvx_mesh_s& m)
 			}
 			else for(int i = 0; i < (int)cand.size(); i++) {
 				const int c = cand[i], l = links[c];
-				if(grp[c] >= 0) continue;              // of another patch: halo only
-				if(ntask + m.nnode[c] - l > PATCH_TASKS || nmet + m.nnode[c] - l > PATCH_MAX) continue;
-				int open = 0;
-				for(int k = 0; k < m.nnode[c]; k++) {
-					const int o = m.esuel[(size_t)c*4 + k];
-					open += o < n && grp[o] < 0;
-				}
-				if(best < 0 || l > bl || (l == bl && (open < bo || (open == bo && met[c] < met[cand[best]])))) {
-					best = i; bl = l; bo = open;
+				if(l < bl || ntask + m.nnode[c] - l > PATCH_TASKS || nmet + m.nnode[c] - l > PATCH_MAX)
+					continue;
+				if(best < 0 || l > bl || (l == bl && (open[c] < bo || (open[c] == bo && met[c] < met[cand[best]])))) {
+					best = i; bl = l; bo = open[c];
 				}
 			}
 			if(best < 0) break;
@@ -404,13 +410,18 @@ void build_patches(fvx_mesh_s& m)
 			for(int k = 0; k < m.nnode[c]; k++) {
 				const int o = m.esuel[(size_t)c*4 + k];
 				if(o >= n) continue;
+				open[o]--;
 				if(grp[o] == g) continue;
-				if(seen[o] != g) { seen[o] = g; links[o] = 0; met[o] = nmet++; cand.push_back(o); }
+				if(seen[o] != g) {
+					seen[o] = g; links[o] = 0; met[o] = nmet++;
+					(grp[o] < 0 ? cand : rim).push_back(o);
+				}
 				links[o]++;
 			}
 		}
 		done += nown;
 		std::sort(cells.begin() + first, cells.end());
+		cand.insert(cand.end(), rim.begin(), rim.end());
 		std::sort(cand.begin(), cand.end());
 		cells.insert(cells.end(), cand.begin(), cand.end());
 		const int nl = (int)cells.size() - first;

@@ -38,7 +38,6 @@ namespace fvx {
 
 /// One row of a factor block as the registers hold it. pin() keeps the conversion to FP64 inside
 /// the pass loop: hoisted out of it, the rows would take twice the registers.
-
 template <class VT> struct FacRow;
 template <> struct FacRow<double> {
 	double2 a, b;

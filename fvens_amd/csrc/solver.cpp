@@ -421,7 +421,7 @@ using Op = std::function<void(const double* x, long sx, double* y, long sy, cons
 
 /// Device storage of one FGMRES cycle for up to `cap` instances: bases, per-instance scalar
 /// slots (h column, norms), the least-squares state of the cycle
-/// (k_fgmres_* in linalg.hip), the cycle's instance list and its compacted running list, and
+/// (k_scale_rotate in linalg.hip), the cycle's instance list and its compacted running list, and
 /// pinned host words through which the device reports how many instances still run.
 struct Krylov {
 	long N = 0;
