@@ -22,8 +22,9 @@
  *
  * Host tables (mesh.cpp, build_wave_tasks): tasks[64 g + t] = the face of task t (-1: no task;
  * the face record holds its left cell and its right cell or -1-ib); groups[g] = {first entry in
- * gcells, or first cell where groups are consecutive cells and gcells is null, cells}; cslot[64 g + j] = the slot word of the group's cell j, byte k = 2 task + side for
- * its local face k (side 1: the cell is the face's right cell), 0xff for an unused slot.
+ * gcells, or first cell where groups are consecutive cells and gcells is null, cells};
+ * cslot[64 g + j] = the slot word of the group's cell j, byte k = 2 task + side for its local face
+ * k (side 1: the cell is the face's right cell), 0xff for an unused slot.
  */
 #ifndef FVX_FLUX_WAVE_HPP
 #define FVX_FLUX_WAVE_HPP

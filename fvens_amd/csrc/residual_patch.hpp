@@ -18,10 +18,12 @@
  * than writing and reading them (160 bytes a cell with the second read of the state, of 408) and
  * two more launches: 1,572,864 cells in Hilbert order (HLLC, limited) 207 -> 176 us, 16 instances
  * of 98,304 cells (Roe, limited) 197 -> 153, 262,144 cells viscous MUSCL 78 -> 53, 4,608 cells 20
- * -> 13. Bound by HBM (1,572,864 cells: 660 MB, 77% of the copy rate) and FP64 issue (56% of the time). Four waves per SIMD for Roe, which would
- * spill at five (16 instances 145 against 149 us in a row), five for the other fluxes (HLLC on
- * 1,572,864 cells 175 against 186); viscous three. Larger groups of neighbours list fewer halo
- * cells but pass 256 tasks, one per lane.
+ * -> 13. Bound by HBM (1,572,864 cells: 660 MB, 77% of the copy rate) and FP64 issue (56% of the
+ * time). Four waves per SIMD for Roe, which would spill at five (16 instances 145 against 149 us
+ * in a row), five for the other fluxes (HLLC on 1,572,864 cells 175 against 186); viscous three.
+ * Larger patches would have fewer halo cells, but more than 256 tasks, one per lane. A patch cell's
+ * midpoint offsets from its faces' records instead of the table save 10% of the traffic, but the
+ * gradients then wait for the records: 177 -> 200 us.
  */
 #ifndef FVX_RESIDUAL_PATCH_HPP
 #define FVX_RESIDUAL_PATCH_HPP
