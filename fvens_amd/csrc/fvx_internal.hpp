@@ -237,6 +237,17 @@ struct SgsPatch {
 	DBuf<double> scratch;                  // [ninst][ncell][4] iterate between launches
 	hipStream_t owner = nullptr;           // stream the scratch serves since the last set-up
 	bool claimed = false;
+	/// Back to a new handle's state: tables fit one mesh, precision, colouring and number of instances.
+	void reset()
+	{
+		d_rec.release();
+		d_halo.release();
+		scratch.release();
+		most = cycles = slots = npatch = nhalo = 0;
+		spent = 0;
+		failed = claimed = false;
+		owner = nullptr;
+	}
 };
 }
 

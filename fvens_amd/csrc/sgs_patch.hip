@@ -575,7 +575,11 @@ bool sgs_patch_apply(const fvx_pc_s& p, const VTF* fac, const double* r, long sr
 		switch(t.slots) {
 		FVX_SP(128, 1) FVX_SP(256, 1) FVX_SP(256, 2)
 		default:
-			if constexpr(sizeof(VTF) <= 4) switch(t.slots) { FVX_SP(256, 3) FVX_SP(256, 4) }
+			if constexpr(sizeof(VTF) <= 4) switch(t.slots) {
+			FVX_SP(256, 3) FVX_SP(256, 4)
+			default: throw Error(FVX_ERR_INVALID, "no kernel for this patch size");
+			}
+			else throw Error(FVX_ERR_INVALID, "no kernel for this patch size");
 		}
 #undef FVX_SP
 		zin = zo;

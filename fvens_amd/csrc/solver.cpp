@@ -311,6 +311,7 @@ void pc_init(fvx_pc_s& p, const fvx_mesh_s* m, int type, int prec, int ninst)
 	p.prec = prec;
 	p.ninst = ninst;
 	p.A = nullptr;
+	p.patch.reset();
 	const int n = m->nelem;
 	p.colour.assign(n, 0);
 	p.ncol = 1;
