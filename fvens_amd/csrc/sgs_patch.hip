@@ -23,14 +23,12 @@
 #include "fvx_internal.hpp"
 #include "wave.hpp"
 #include "blocks.hpp"
+#include "threads.hpp"
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <exception>
 #include <new>
 #include <numeric>
-#include <system_error>
-#include <thread>
 
 namespace fvx {
 
@@ -182,24 +180,6 @@ constexpr int SP_CUS = 256;              // compute units: one workgroup each
 inline int capacity(int prec) { return prec == FVX_PREC_F64 ? 512 : 1024; }
 
 inline int threads_for(int n) { return n < 1024 ? 1 : n < 8192 ? 4 : 8; }
-
-/// Runs f(0) .. f(nt - 1), on threads where they can be had; the first exception is rethrown.
-template <class F> void parallel(int nt, F&& f)
-{
-	std::vector<std::thread> th;
-	std::vector<std::exception_ptr> err(nt);
-	auto body = [&](int t) {
-		try { f(t); } catch(...) { err[t] = std::current_exception(); }
-	};
-	th.reserve(nt);
-	int t = 1;
-	try { for(; t < nt; t++) th.emplace_back(body, t); }
-	catch(const std::system_error&) {}
-	body(0);
-	for(; t < nt; t++) body(t);
-	for(std::thread& x : th) x.join();
-	for(const std::exception_ptr& e : err) if(e) std::rethrow_exception(e);
-}
 
 /// The colour of the pass that is e passes before the last one of an application.
 inline int pass_colour(int e, int ncol)
