@@ -348,6 +348,9 @@ void launch_pc_apply(const fvx_pc_s& p, const double* r, long sr, double* z, lon
 template <class VTF>
 bool sgs_patch_apply(const fvx_pc_s& p, const VTF* fac, const double* r, long sr, double* z,
                      long sz, const Inst& L, hipStream_t s);
+/// Makes the patch tables now that the preconditioner's applications would otherwise make once they
+/// have paid for them.
+void sgs_patch_prepare(const fvx_pc_s& p, hipStream_t s);
 int reduction_blocks();
 int max_dots();
 long partial_stride();

@@ -485,52 +485,79 @@ void make_tables(const fvx_pc_s& p, int most, hipStream_t s)
 	t.cycles = cycles;
 }
 
-/// Whether this application runs on the patches. The tables (made on the host: 7 ms for 98,304
-/// cells, 1-2 ms for 4,608) are made once the handle's applications have taken about as long by
+/// Sweeps per launch the tables should allow: at most 4, and their passes must fit a record's bits.
+int most_sweeps(const fvx_pc_s& p)
+{
+	return std::min(std::min(4, p.sweeps), (SP_MAX_PASS - 1)/(2*(p.ncol - 1)));
+}
+
+/// Whether patches can serve the preconditioner on stream s at all.
+bool possible(const fvx_pc_s& p, hipStream_t s)
+{
+	return p.type == FVX_PC_SGS && p.ncol > 1 && 2*(p.ncol - 1) + 1 <= SP_MAX_PASS && !p.patch.failed
+	       && !capturing(s);
+}
+
+/// Runs f, which allocates; false where there is no memory: the colour passes then serve the handle.
+template <class F> bool allocating(SgsPatch& t, F&& f)
+{
+	try {
+		Relaxed relaxed;
+		f();
+		return true;
+	}
+	catch(const std::bad_alloc&) { t.failed = true; }
+	catch(const Error& e) {
+		t.failed = true;
+		if(e.code != FVX_ERR_ALLOC) throw;
+		(void)hipGetLastError();
+	}
+	return false;
+}
+
+void tables(const fvx_pc_s& p, int most, hipStream_t s)
+{
+	SgsPatch& t = p.patch;
+	allocating(t, [&] {
+		make_tables(p, most, s);
+		t.most = most;
+		t.spent = 0;
+		if(!t.cycles) t.failed = true;
+	});
+}
+
+/// Whether this application runs on the patches. The tables (made on the host: 8 ms for 98,304
+/// cells, 2-4 ms for 4,608) are made once the handle's applications have taken about as long by
 /// colour passes as that takes, so that a preconditioner used a few times does not pay for
 /// them; until then, and where the device has no memory for them, the colour passes serve. The
 /// scratch vector of applications of more than one launch serves one stream between two set-ups,
 /// and no recorded graph.
 bool ready(const fvx_pc_s& p, size_t value, int nact, hipStream_t s)
 {
+	if(!possible(p, s)) return false;
 	SgsPatch& t = p.patch;
-	const int C = p.ncol, n = p.m->nelem;
-	if(C < 2 || 2*(C - 1) + 1 > SP_MAX_PASS || t.failed || capturing(s)) return false;
-	const int most = std::min(std::min(4, p.sweeps), (SP_MAX_PASS - 1)/(2*(C - 1)));
-	try {
-		if(t.most < most) {
-			// us of a colour pass: a launch, and its share of the factors at ~7 TB/s
-			t.spent += (2.0*p.sweeps*(C - 1) + 1)*(3.5 + 80.0*n*value*nact/C/7e6);
-			if(t.spent >= 1500 + 0.07*n) {
-				Relaxed relaxed;
-				make_tables(p, most, s);
-				t.most = most;
-				t.spent = 0;
-				if(!t.cycles) t.failed = true;
-			}
-		}
-		if(!t.cycles) return false;
-		if(p.sweeps > t.cycles) {
-			if(t.claimed && t.owner != s) return false;
-			const size_t N = 4*(size_t)n*p.ninst;
-			if(t.scratch.n != N) {
-				Relaxed relaxed;
-				t.scratch.alloc(N);
-			}
-			t.owner = s;
-			t.claimed = true;
-		}
+	const int C = p.ncol, n = p.m->nelem, most = most_sweeps(p);
+	if(t.most < most) {
+		// us of a colour pass: a launch, and its share of the factors at ~7 TB/s
+		t.spent += (2.0*p.sweeps*(C - 1) + 1)*(3.5 + 80.0*n*value*nact/C/7e6);
+		if(t.spent >= 1500 + 0.07*n) tables(p, most, s);
 	}
-	catch(const std::bad_alloc&) { t.failed = true; return false; }
-	catch(const Error& e) {
-		t.failed = true;
-		if(e.code != FVX_ERR_ALLOC) throw;
-		(void)hipGetLastError();
-		return false;
+	if(t.failed || !t.cycles) return false;
+	if(p.sweeps > t.cycles) {
+		if(t.claimed && t.owner != s) return false;
+		const size_t N = 4*(size_t)n*p.ninst;
+		if(t.scratch.n != N && !allocating(t, [&] { t.scratch.alloc(N); })) return false;
+		t.owner = s;
+		t.claimed = true;
 	}
 	return true;
 }
 
+}
+
+void sgs_patch_prepare(const fvx_pc_s& p, hipStream_t s)
+{
+	if(possible(p, s) && p.patch.most < most_sweeps(p)) tables(p, most_sweeps(p), s);
 }
 
 template <class VTF>
@@ -538,7 +565,7 @@ bool sgs_patch_apply(const fvx_pc_s& p, const VTF* fac, const double* r, long sr
                      long sz, const Inst& L, hipStream_t s)
 {
 	const SgsPatch& t = p.patch;
-	if(p.type != FVX_PC_SGS || r == z || !ready(p, sizeof(VTF), L.nact, s)) return false;
+	if(r == z || !ready(p, sizeof(VTF), L.nact, s)) return false;
 	const int steps = (p.sweeps + t.cycles - 1)/t.cycles;
 	const long N = 4L*p.m->nelem;
 	const double* zin = nullptr;

@@ -12,6 +12,8 @@
  * Preconditioner schedule: for the linear system of one pseudo-time step at the given state
  * and CFL number, each preconditioner type and sweep count is timed over set-up plus one
  * FGMRES solve to the given tolerance; candidates whose solve does not reach it are discarded.
+ * Gauss-Seidel is timed with its patch tables in place, as every solve of more than a few steps
+ * runs it: before they were, 16 sweeps on 4,608 cells were timed at 0.85 ms instead of 0.17.
  */
 #include "fvx_internal.hpp"
 #include "wave.hpp"
@@ -134,6 +136,7 @@ void autotune_pc(fvx_disc_s& d, const double* u, double cfl, int restart, double
 			pc_set_sweeps(P, sw);
 			int its = 0;
 			bool ok = true;
+			sgs_patch_prepare(P, s);
 			const double t = T.ms([&] {
 				launch_pc_setup(P, A, Inst(), s);
 				try { its = linear_solve(A, P, r.p, x.p, restart, rtol, s); }
