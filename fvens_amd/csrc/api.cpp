@@ -602,6 +602,10 @@ fvx_status fvx_set_launch(fvx_disc d, int kernel, int block, int xcd)
 			        "first-order or linear reconstruction only");
 			d->tune.flux_xcd = xcd; d->tune.flux_wave = 1; d->tune.flux_group = 0;
 		}
+		else if(kernel == FVX_KERNEL_RESIDUAL) {
+			require(block == 256, "the library's own choice of form is set with block 256");
+			d->tune.flux_xcd = xcd; d->tune.flux_group = 1;
+		}
 		else if(kernel == FVX_KERNEL_JACOBIAN) {
 			require(block <= 256, "the Jacobian kernel takes at most 256 threads per workgroup");
 			d->tune.jac_block = block; d->tune.jac_xcd = xcd;
@@ -618,6 +622,9 @@ fvx_status fvx_get_launch(fvx_disc d, int kernel, int* block, int* xcd)
 		else if(kernel == FVX_KERNEL_FLUX) { *block = d->tune.flux_block; *xcd = d->tune.flux_xcd; }
 		else if(kernel == FVX_KERNEL_FLUX_WAVE) {
 			*block = d->tune.flux_wave ? 64 : 0; *xcd = d->tune.flux_xcd;
+		}
+		else if(kernel == FVX_KERNEL_RESIDUAL) {
+			*block = d->tune.flux_group ? 256 : 0; *xcd = d->tune.flux_xcd;
 		}
 		else if(kernel == FVX_KERNEL_JACOBIAN) { *block = d->tune.jac_block; *xcd = d->tune.jac_xcd; }
 		else require(false, "kernel has no tunable launch shape");

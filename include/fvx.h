@@ -354,11 +354,13 @@ typedef struct {
 } fvx_tune_row;
 
 /* Times every launch shape of the gradient, face-flux and Jacobian kernels at state u and
- * keeps the fastest in d (results are bitwise identical for every shape). rows[cap]. */
+ * keeps the fastest in d (results are bitwise identical for every shape); the library's own choice
+ * of the residual's form stays where none is faster. rows[cap]. */
 fvx_status fvx_autotune(fvx_disc d, const double* u, int reps, fvx_tune_row* rows, int cap,
                         int* nrows, void* stream);
 /* Sets / reads the launch shape of one kernel (block 64, 128, 256 or 512; 256 at most for the
- * Jacobian). */
+ * Jacobian) or, by FVX_KERNEL_FLUX, FVX_KERNEL_FLUX_WAVE and FVX_KERNEL_RESIDUAL, the form of the
+ * residual; see the kernel ids below. */
 fvx_status fvx_set_launch(fvx_disc d, int kernel, int block, int xcd);
 fvx_status fvx_get_launch(fvx_disc d, int kernel, int* block, int* xcd);
 /* Times preconditioner types and sweep counts on the pseudo-time linear system at u and the
@@ -415,16 +417,25 @@ fvx_status fvx_mpnn_train_step(fvx_mpnn n, int ngraph, const float* targets, con
 
 /* ---- timing: the TimingData role of the reference (src/ode/aodesolver.hpp:46-67) ---- */
 
-/* Kernel ids for fvx_profile_read and fvx_set_launch / fvx_get_launch. FVX_KERNEL_FLUX_WAVE
- * is the wave-task form of the face-flux pass: each wave64 owns a group of neighbouring cells
- * and evaluates each face touching them once. Without a setting the library does second-order
- * residuals in one launch (their time is read as FVX_KERNEL_FLUX, the gradients count with none),
- * where that does not apply in either form by size; setting a launch for FVX_KERNEL_FLUX_WAVE
- * (block 64) selects separate gradients and the wave form (FVX_ERR_INVALID for a viscous or MUSCL
- * discretisation), setting one for FVX_KERNEL_FLUX the quad form. All give bitwise equal residuals and time steps; the wave form's time is read as
- * FVX_KERNEL_FLUX. */
+/* Kernel ids for fvx_profile_read and fvx_set_launch / fvx_get_launch. All forms of the residual
+ * give bitwise equal residuals and time steps.
+ * FVX_KERNEL_RESIDUAL stands for the library's own choice of form, which a new discretisation
+ * has: second-order residuals in one launch (read as FVX_KERNEL_FLUX by fvx_profile_read; their
+ * gradients are counted, with no time), the others, WENO reconstruction and limited viscous
+ * flow as separate passes, the flux pass in either form by size. Setting a launch for
+ * FVX_KERNEL_FLUX or FVX_KERNEL_FLUX_WAVE selects separate passes with that form instead;
+ * setting FVX_KERNEL_RESIDUAL (block 256) goes back. fvx_get_launch reads block 256 while the
+ * library chooses, else 0, so that settings read from one discretisation are restored on
+ * another by setting FVX_KERNEL_FLUX, FVX_KERNEL_FLUX_WAVE if its block is 64, and
+ * FVX_KERNEL_RESIDUAL if its block is 256, in this order.
+ * FVX_KERNEL_FLUX_WAVE (block 64) is the wave-task form of the face-flux pass: each wave64 owns a
+ * group of neighbouring cells and evaluates each face touching them once. FVX_ERR_INVALID for a
+ * viscous or MUSCL discretisation; its time is read as FVX_KERNEL_FLUX. fvx_get_launch reads 64
+ * where it is selected, and on a new discretisation where the cell order is compact and it may be.
+ * A setting for FVX_KERNEL_GRADIENTS is that of the separate gradient pass; a residual done in one
+ * launch has none. */
 enum { FVX_KERNEL_GRADIENTS = 0, FVX_KERNEL_FLUX = 1, FVX_KERNEL_JACOBIAN = 2,
-       FVX_KERNEL_PC = 3, FVX_KERNEL_FLUX_WAVE = 4 };
+       FVX_KERNEL_PC = 3, FVX_KERNEL_FLUX_WAVE = 4, FVX_KERNEL_RESIDUAL = 5 };
 
 /* on != 0 resets the counters and starts recording HIP events around every kernel the handle
  * launches (on the launch stream); on == 0 stops recording. */

@@ -124,3 +124,67 @@ def test_preconditioner_tuner_times_what_a_solve_runs(torch_cuda):
             torch.cuda.synchronize()
             t.append(1e3 * (time.perf_counter() - t0))
         assert min(q["sgs", sweeps][3] for q in rows) <= 2 * min(t[100:]), (sweeps, min(t[100:]))
+
+
+def _launches(d, u):
+    """(flux launches, gradient passes, whether the gradients had a pass of their own)"""
+    import torch
+    r = torch.zeros_like(u)
+    d.profile_enable(True)
+    d.compute_residual(u, r)
+    torch.cuda.synchronize()
+    out = d.profile_read("flux")[1], d.profile_read("gradients")[1], d.profile_read("gradients")[0] > 0
+    d.profile_enable(False)
+    return out, r
+
+
+@pytest.mark.parametrize("order", ["rcm", "hilbert"])
+def test_launch_settings_can_be_read_and_set_again(torch_cuda, order):
+    """The residual in one launch, the choice of a new discretisation, given up for a selected form
+    and taken again, also on another discretisation from the settings that were read."""
+    import torch
+    raw = meshgen.airfoil_omesh(128, 32, 16)
+    raw = raw.permuted(fvx.rcm_permutation(raw) if order == "rcm" else fvx.hilbert_permutation(raw))
+    gm = fvx.Mesh(raw)
+
+    def disc():
+        return fvx.FlowFV(gm, fvx.physics_cfg(Minf=0.7, aoa_deg=2.0, bcs=BCS), fvx.numerics_cfg(
+            flux="HLLC", gradient="LEASTSQUARES", recon="VENKATAKRISHNAN"))
+
+    def read(d):
+        return {k: d.get_launch(k) for k in ("gradients", "jacobian", "flux", "flux_wave", "residual")}
+
+    def restore(d, got):
+        for k in ("gradients", "jacobian", "flux"):
+            d.set_launch(k, *got[k])
+        for k, block in (("flux_wave", 64), ("residual", 256)):
+            if got[k][0] == block:
+                d.set_launch(k, *got[k])
+
+    u = torch.tensor(states.perturbed_freestream(raw, Minf=0.7, aoa_deg=2.0), device="cuda")
+    d = disc()
+    new = read(d)
+    assert new["residual"] == (256, True)
+    assert new["flux_wave"][0] == (64 if order == "hilbert" else 0)
+    one, r0 = _launches(d, u)
+    assert one == (1, 1, False)
+    settings = [new]
+    for form, block in (("flux", 128), ("flux_wave", 64)):
+        d.set_launch(form, block, False)
+        assert d.get_launch("residual")[0] == 0 and d.get_launch(form) == (block, False)
+        got, r = _launches(d, u)
+        assert got == (1, 1, True) and torch.equal(r, r0)
+        settings.append(read(d))
+    restore(d, new)
+    assert read(d) == new and _launches(d, u)[0] == one
+    for s in settings:
+        e = disc()
+        restore(e, s)
+        assert read(e) == s
+        got, r = _launches(e, u)
+        assert got == (one if s is new else (1, 1, True)) and torch.equal(r, r0)
+    with pytest.raises(fvx.FvxError):
+        d.set_launch("residual", 64)
+    # the tuner keeps the library's choice or a form of its table, and says which
+    d.autotune(u, reps=3)
+    assert _launches(d, u)[0] == (one if d.get_launch("residual")[0] == 256 else (1, 1, True))
