@@ -148,8 +148,11 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 				m.intfac[(size_t)f*4+2] = m.inpoel[c*4+j];
 				m.intfac[(size_t)f*4+3] = m.inpoel[c*4+(j+1)%nn];
 				m.elemface[(size_t)c*4+j] = f;
+				// by its nodes: two cells may share more than one face
+				const long long key = ekey(m.inpoel[c*4+j], m.inpoel[c*4+(j+1)%nn]);
 				for(int k = 0; k < m.nnode[o]; k++)
-					if(m.esuel[(size_t)o*4+k] == c) m.elemface[(size_t)o*4+k] = f;
+					if(ekey(m.inpoel[o*4+k], m.inpoel[o*4+(k+1)%m.nnode[o]]) == key)
+						m.elemface[(size_t)o*4+k] = f;
 				f++;
 			}
 		}

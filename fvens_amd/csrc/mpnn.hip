@@ -960,7 +960,11 @@ void mpnn_build_graph(const fvx_mesh_s& m, int wall_tag, MpnnGraphHost& gh)
 			const int j = gh.nbr[(size_t)c*4 + k];
 			if(j < 0) continue;
 			for(int kk = 0; kk < 4; kk++)
-				if(gh.nbr[(size_t)j*4 + kk] == c) { gh.rev[(size_t)c*4 + k] = kk; break; }
+				if(gh.nbr[(size_t)j*4 + kk] == c
+				   && m.elemface[(size_t)j*4 + kk] == m.elemface[(size_t)c*4 + k]) {
+					gh.rev[(size_t)c*4 + k] = kk;
+					break;
+				}
 			if(gh.rev[(size_t)c*4 + k] < 0)
 				throw Error(FVX_ERR_INVALID, "mesh neighbour lists are not symmetric");
 		}

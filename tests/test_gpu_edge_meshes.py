@@ -101,3 +101,63 @@ def test_smallest_meshes_jacobian_and_linear_solves(torch_cuda, shape):
         # block Jacobi on the larger meshes: 31 iterations fall short of 4 n unknowns
         if res > 1e-9:
             assert kind == "jacobi" and its == 31 and res < 1e-2, (kind, its, res)
+
+
+def _doublets(nx, ny, cells):
+    """A bump mesh with the given quadrilaterals divided in two along a path through a new node in
+    their middle: the halves share both faces at that node."""
+    raw = meshgen.gaussian_bump(nx, ny, 0)
+    inpoel, coords = raw.inpoel.copy(), [raw.coords]
+    for i, c in enumerate(cells):
+        a, b, cc, d = inpoel[c]
+        x = raw.npoin + i
+        # off the middle, so that the two shared faces differ in length and normal
+        w = np.array([0.4, 0.2, 0.25, 0.15])
+        coords.append(w @ raw.coords[[a, b, cc, d]][None])
+        inpoel[c] = a, b, cc, x
+        inpoel = np.vstack([inpoel, [[a, x, cc, d]]]).astype(np.int32)
+    out = meshgen.RawMesh(np.vstack(coords), inpoel,
+                          np.concatenate([raw.nnode, np.full(len(cells), 4, np.int32)]).astype(np.int32),
+                          raw.bface, raw.btag)
+    assert (out.signed_areas() > 0).all()
+    return out
+
+
+@pytest.mark.parametrize("order", ["natural", "rcm", "hilbert"])
+@pytest.mark.parametrize("cfg", ["first", "gg", "wls"])
+def test_cells_that_share_two_faces(torch_cuda, order, cfg):
+    """Residual and time steps in the library's own form against the oracle (to which every face is
+    one item of a list), and bitwise in the other forms."""
+    import torch
+    raw = _doublets(30, 20, [5, 6, 100, 333, 599])
+    if order != "natural":
+        raw = raw.permuted(fvx.rcm_permutation(raw) if order == "rcm" else fvx.hilbert_permutation(raw))
+    num = dict(CONFIGS, wls=dict(flux="HLLC", gradient="LEASTSQUARES", recon="NONE"))[cfg]
+    phys = dict(Minf=0.5, bcs=BUMP_BCS)
+    u = states.perturbed_freestream(raw, Minf=0.5, L=3.0)
+    od = po.Disc(po.Mesh(raw), po.make_config(**phys, **num))
+    r_ref, dt_ref = od.residual(u)
+    scale = np.maximum(np.abs(r_ref), od.flux_magnitude(u))
+    disc = fvx.FlowFV(fvx.Mesh(raw), fvx.physics_cfg(**phys), fvx.numerics_cfg(**num))
+    ut = torch.tensor(u, device="cuda")
+    out = []
+    for form, block in (("residual", 256), ("flux", 256), ("flux_wave", 64)):
+        disc.set_launch(form, block, True)
+        r = torch.zeros((raw.nelem, 4), dtype=torch.float64, device="cuda")
+        dt = torch.zeros(raw.nelem, dtype=torch.float64, device="cuda")
+        disc.compute_residual(ut, r, True, dt)
+        out.append((r, dt))
+    rel = np.abs(out[0][0].cpu().numpy() - r_ref) / scale
+    assert rel.max() <= 1e-12, rel.max()
+    assert np.allclose(out[0][1].cpu().numpy(), dt_ref, rtol=1e-12, atol=0)
+    for r, dt in out[1:]:
+        assert torch.equal(r, out[0][0]) and torch.equal(dt, out[0][1])
+
+
+def test_reverse_slots_of_cells_that_share_two_faces(torch_cuda):
+    """The warm start's network finds, for every slot, the neighbour's slot of the same face."""
+    raw = _doublets(30, 20, [5, 6, 100, 333, 599])
+    f = fvx.MPNN(fvx.Mesh(raw), 2, 1).features()
+    c, k = np.nonzero(f["nbr"] >= 0)
+    j, kk = f["nbr"][c, k], f["rev"][c, k]
+    assert (f["nbr"][j, kk] == c).all() and (f["rev"][j, kk] == k).all()
