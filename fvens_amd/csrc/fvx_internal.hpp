@@ -306,8 +306,6 @@ void find_lines(const fvx_mesh_desc& d, double threshold, std::vector<std::vecto
                 std::vector<int>& celline);
 void line_order(const fvx_mesh_desc& d, double threshold, int graph_ordering, int* perm);
 void hilbert_order(const fvx_mesh_desc& d, int* perm);
-void build_wave_tasks(fvx_mesh_s& m);
-void build_patches(fvx_mesh_s& m);
 void build_disc(fvx_disc_s& d);
 GasParams make_gas(const fvx_physics_cfg& p);
 

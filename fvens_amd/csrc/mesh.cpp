@@ -10,6 +10,7 @@
  */
 #include "fvx_internal.hpp"
 #include "wave.hpp"
+#include "threads.hpp"
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -88,6 +89,32 @@ std::vector<int> neighbours(const fvx_mesh_desc& d, const std::vector<EdgeRec>& 
 
 }
 
+static void build_geometry(fvx_mesh_s& m, const std::vector<int>& host);
+
+namespace {
+
+/// Host tables of the wave-task flux pass and of the one-launch residual (build_wave_tasks,
+/// build_patches).
+struct WaveTables {
+	std::vector<int> tasks, cells;
+	std::vector<int2> groups;
+	std::vector<unsigned> slots;
+};
+struct PatchHost {
+	std::vector<PatchGroup> groups;
+	std::vector<int> cells, face;
+	std::vector<unsigned short> local;
+	std::vector<unsigned> sides;
+	std::vector<ushort4> slots;
+	int nwmax = 0, nsmax = 0;
+};
+
+}
+
+static std::vector<int> consecutive_groups(const fvx_mesh_s& m);
+static void build_wave_tasks(const fvx_mesh_s& m, const std::vector<int>& consec, WaveTables& T);
+static void build_patches(const fvx_mesh_s& m, PatchHost& T);
+
 void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 {
 	check_desc(d);
@@ -158,6 +185,41 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 		}
 	}
 
+	// The residual's tables need the topology only, so they are made beside the geometry, which this
+	// thread does: 98,304 cells 23 ms instead of 37 one after the other (17 without the patches and
+	// grown groups), 1,572,864 cells in Hilbert order 413 instead of 581 (410).
+	const std::vector<int> consec = consecutive_groups(m);
+	m.wave_order = m.nelem >= 24L*(long)consec.size();
+	WaveTables wt;
+	PatchHost pt;
+	auto piece = [&](int t) {
+		if(t == 0) build_geometry(m, host);
+		else if(t == 1) build_patches(m, pt);
+		else build_wave_tasks(m, consec, wt);
+	};
+	if(m.nelem < 2048) for(int t = 0; t < 3; t++) piece(t);
+	else parallel(3, piece);
+	m.nwgroup = (int)wt.groups.size();
+	m.d_wtask.upload(wt.tasks);
+	m.d_wgroup.upload(wt.groups);
+	if(!m.wave_order) m.d_wcell.upload(wt.cells);
+	m.d_wslot.upload(wt.slots);
+	// the default limit of a workgroup's LDS (never met with PATCH_MAX cells of ordinary meshes)
+	if((4*(size_t)pt.nwmax + 10*(size_t)pt.nsmax)*sizeof(double) > 65536) return;
+	m.npatch = (int)pt.groups.size();
+	m.patch_nw = pt.nwmax;
+	m.patch_ns = pt.nsmax;
+	m.d_pgroup.upload(pt.groups);
+	m.d_pcell.upload(pt.cells);
+	m.d_plocal.upload(pt.local);
+	m.d_pface.upload(pt.face);
+	m.d_psides.upload(pt.sides);
+	m.d_pslot.upload(pt.slots);
+}
+
+/// Geometry from the topology (host: the boundary faces' cells), and the device arrays of both.
+static void build_geometry(fvx_mesh_s& m, const std::vector<int>& host)
+{
 	const double* X = m.coords.data();
 	m.facemetric.assign((size_t)m.naface*3, 0.0);
 	m.gr.assign((size_t)m.naface*2, 0.0);
@@ -231,8 +293,25 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 	m.d_area.upload(m.area);
 	m.d_bhost.upload(host);
 	m.d_btag.upload(m.btag);
-	build_wave_tasks(m);
-	build_patches(m);
+}
+
+/// First cells of the wave-task groups of consecutive cells: at most 64 cells and 64 tasks.
+static std::vector<int> consecutive_groups(const fvx_mesh_s& m)
+{
+	const int n = m.nelem;
+	std::vector<int> consec;
+	for(int c = 0; c < n; ) {
+		const int c0 = c;
+		consec.push_back(c0);
+		for(int nt = 0; c < n && c - c0 < 64; c++) {
+			for(int k = 0; k < m.nnode[c]; k++) {
+				const int o = m.esuel[(size_t)c*4 + k];
+				nt += !(o < n && o >= c0 && o < c);
+			}
+			if(nt > 64) break;
+		}
+	}
+	return consec;
 }
 
 static std::vector<int> open_neighbours(const fvx_mesh_s& m)
@@ -259,34 +338,23 @@ static std::vector<int> open_neighbours(const fvx_mesh_s& m)
  * A task is its face's index (the face record holds the two cells); a cell's slot word holds, in
  * byte k, 2 task + side for its local face k (side 1: the cell is the face's right cell), 0xff when
  * unused. */
-void build_wave_tasks(fvx_mesh_s& m)
+static void build_wave_tasks(const fvx_mesh_s& m, const std::vector<int>& consec, WaveTables& T)
 {
 	const int n = m.nelem;
-	// first cells of the groups of consecutive cells
-	std::vector<int> consec;
-	for(int c = 0; c < n; ) {
-		const int c0 = c;
-		consec.push_back(c0);
-		for(int nt = 0; c < n && c - c0 < 64; c++) {
-			for(int k = 0; k < m.nnode[c]; k++) {
-				const int o = m.esuel[(size_t)c*4 + k];
-				nt += !(o < n && o >= c0 && o < c);
-			}
-			if(nt > 64) break;
-		}
-	}
-	m.wave_order = n >= 24L*(long)consec.size();
-	std::vector<int> tasks, cells, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand;
+	std::vector<int>&tasks = T.tasks, &cells = T.cells;
+	std::vector<int2>& groups = T.groups;
+	std::vector<unsigned>& slots = T.slots;
+	std::vector<int> grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand;
 	std::vector<int> open = open_neighbours(m);   // neighbours without a group
-	std::vector<int2> groups;
-	std::vector<unsigned> slots;
 	cells.reserve(n);
-	consec.push_back(n);
 	int seed = 0;
 	while((int)cells.size() < n) {
 		const int g = (int)groups.size(), first = (int)cells.size();
 		if(m.wave_order)
-			for(int c = consec[g]; c < consec[g + 1]; c++) { grp[c] = g; cells.push_back(c); }
+			for(int c = consec[g]; c < (g + 1 < (int)consec.size() ? consec[g + 1] : n); c++) {
+				grp[c] = g;
+				cells.push_back(c);
+			}
 		else while(grp[seed] >= 0) seed++;
 		cand.assign(1, seed);
 		seen[seed] = g;
@@ -351,25 +419,21 @@ void build_wave_tasks(fvx_mesh_s& m)
 		}
 		if(nt > 64 || (!m.wave_order && nt != ntask)) throw Error(FVX_ERR_INVALID, "wave-task count mismatch");
 	}
-	m.nwgroup = (int)groups.size();
-	m.d_wtask.upload(tasks);
-	m.d_wgroup.upload(groups);
-	if(!m.wave_order) m.d_wcell.upload(cells);
-	m.d_wslot.upload(slots);
 }
 
 /* Tables of the one-launch residual (residual_patch.hpp). Patches grow like the groups of
  * build_wave_tasks (consecutive cells in a compact order) while their faces make at most
  * PATCH_TASKS tasks and patch and halo hold at most PATCH_MAX cells. */
-void build_patches(fvx_mesh_s& m)
+static void build_patches(const fvx_mesh_s& m, PatchHost& T)
 {
 	const int n = m.nelem;
-	std::vector<int> cells, face, grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand, rim, entry(n, -1), far(n, -1);
+	std::vector<int>&cells = T.cells, &face = T.face;
+	std::vector<PatchGroup>& groups = T.groups;
+	std::vector<unsigned short>& local = T.local;
+	std::vector<unsigned>& sides = T.sides;
+	std::vector<ushort4>& slots = T.slots;
+	std::vector<int> grp(n, -1), links(n, 0), met(n, 0), seen(n, -1), cand, rim, entry(n, -1), far(n, -1);
 	std::vector<int> open = open_neighbours(m);   // neighbours without a patch
-	std::vector<PatchGroup> groups;
-	std::vector<unsigned short> local;
-	std::vector<unsigned> sides;
-	std::vector<ushort4> slots;
 	cells.reserve(2*(size_t)n);
 	local.reserve(6*(size_t)n);
 	slots.reserve(n);
@@ -481,17 +545,8 @@ void build_patches(fvx_mesh_s& m)
 		if(nt != ntask) throw Error(FVX_ERR_INVALID, "patch task count mismatch");
 		groups.push_back(PatchGroup{first, nown, nl, nst, (int)(lb/4), (int)sb});
 	}
-	// the default limit of a workgroup's LDS (never met with PATCH_MAX cells of ordinary meshes)
-	if((4*(size_t)nwmax + 10*(size_t)nsmax)*sizeof(double) > 65536) return;
-	m.npatch = (int)groups.size();
-	m.patch_nw = nwmax;
-	m.patch_ns = nsmax;
-	m.d_pgroup.upload(groups);
-	m.d_pcell.upload(cells);
-	m.d_plocal.upload(local);
-	m.d_pface.upload(face);
-	m.d_psides.upload(sides);
-	m.d_pslot.upload(slots);
+	T.nwmax = nwmax;
+	T.nsmax = nsmax;
 }
 
 /* Lines of strongly coupled cells (findLines, src/mesh/meshordering.cpp:199-262). Each cell's
