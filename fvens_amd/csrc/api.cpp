@@ -332,6 +332,16 @@ fvx_status fvx_pc_ordering(fvx_pc p, int* colour, int* ncolours)
 	});
 }
 
+fvx_status fvx_pc_patches(fvx_pc p, int* sweeps, int* npatch, long* served)
+{
+	return guarded([&] {
+		require(p && sweeps && npatch && served, "null argument");
+		*sweeps = p->patch.cycles;
+		*npatch = p->patch.cycles ? p->patch.npatch : 0;
+		*served = p->patch.served;
+	});
+}
+
 fvx_status fvx_pc_set_subdomain_cells(fvx_pc p, int cells)
 {
 	return guarded([&] {

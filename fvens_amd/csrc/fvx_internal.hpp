@@ -232,6 +232,7 @@ struct SgsPatch {
 	bool failed = false;                   // no room for the tables or the scratch vector
 	int cycles = 0;                        // sweeps one launch performs at most (0: no tables)
 	int slots = 0, npatch = 0, nhalo = 0;
+	long served = 0;                       // applications that ran on the patches
 	DBuf<uint4> d_rec;
 	DBuf<int> d_halo;
 	DBuf<double> scratch;                  // [ninst][ncell][4] iterate between launches
@@ -244,6 +245,7 @@ struct SgsPatch {
 		d_halo.release();
 		scratch.release();
 		most = cycles = slots = npatch = nhalo = 0;
+		served = 0;
 		spent = 0;
 		failed = claimed = false;
 		owner = nullptr;

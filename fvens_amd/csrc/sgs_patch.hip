@@ -564,7 +564,7 @@ template <class VTF>
 bool sgs_patch_apply(const fvx_pc_s& p, const VTF* fac, const double* r, long sr, double* z,
                      long sz, const Inst& L, hipStream_t s)
 {
-	const SgsPatch& t = p.patch;
+	SgsPatch& t = p.patch;
 	if(r == z || !ready(p, sizeof(VTF), L.nact, s)) return false;
 	const int steps = (p.sweeps + t.cycles - 1)/t.cycles;
 	const long N = 4L*p.m->nelem;
@@ -592,6 +592,7 @@ bool sgs_patch_apply(const fvx_pc_s& p, const VTF* fac, const double* r, long sr
 		zin = zo;
 		szi = szo;
 	}
+	t.served++;
 	return true;
 }
 

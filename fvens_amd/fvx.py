@@ -474,6 +474,13 @@ class Preconditioner:
         n = self.mesh.nelem
         check(lib().fvx_pc_apply(self.h, _dptr(r, 4 * n), _dptr(z, 4 * n), _stream()))
 
+    def patches(self):
+        """Multicolour SGS: (sweeps per launch on the present patches, 0 without patches; their
+        number; applications that ran on patches)."""
+        s, n, k = C.c_int(), C.c_int(), C.c_long()
+        check(lib().fvx_pc_patches(self.h, C.byref(s), C.byref(n), C.byref(k)))
+        return s.value, n.value, k.value
+
     def ordering(self):
         col = np.zeros(self.mesh.nelem, np.int32)
         nc = C.c_int()

@@ -226,8 +226,17 @@ fvx_status fvx_pc_set_sweeps(fvx_pc p, int sweeps);
 /* PCSetUp: factorises / inverts from the current values of A; later applications use A for
  * the sweeps, so A must stay alive and unchanged until the next set-up. */
 fvx_status fvx_pc_setup(fvx_pc p, fvx_matrix A, void* stream);
-/* PCApply: z = M^-1 r (device vectors [ncell][4]). */
+/* PCApply: z = M^-1 r (device vectors [ncell][4]). Multicolour SGS runs one launch per colour pass
+ * at first and several sweeps per launch, on patches of cells, once its applications have cost
+ * about as much as making the patches does (10 to 25 applications of 16 sweeps). The application
+ * that makes them allocates, waits for the stream and takes longer (2-4 ms on 4,608 cells, 8 on
+ * 98,304, 150-190 on 1,572,864). The bits are the same either way. The patches serve one
+ * stream between two set-ups, no call with r = z and no recorded graph; the colour passes serve
+ * the others, and all where there is no memory for patches. */
 fvx_status fvx_pc_apply(fvx_pc p, const double* r, double* z, void* stream);
+/* Multicolour SGS: how many sweeps a launch performs at most on the present patches (0: there are
+ * none), the number of patches, and how many applications have run on patches so far. */
+fvx_status fvx_pc_patches(fvx_pc p, int* sweeps, int* npatch, long* served);
 /* Host copy of the colour of every cell and the number of colours of the PC's ordering. */
 fvx_status fvx_pc_ordering(fvx_pc p, int* colour, int* ncolours);
 /* FVX_PC_BJACOBI_ILU0: cells per subdomain, in [16, 1024] (default 256); re-partitions the

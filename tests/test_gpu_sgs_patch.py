@@ -3,7 +3,8 @@
 The patches promise the bits of the colour-by-colour passes. Two checks: against a numpy
 restatement of the passes from the exported matrix and the preconditioner's own colours, and
 against the library's colour passes, which still serve an application on a second stream (the
-patches' scratch vector belongs to the first) and one recorded into a graph.
+patches' scratch vector belongs to the first) and one recorded into a graph. fvx_pc_patches says
+which of the two served an application, and every test asserts it.
 """
 import numpy as np
 import pytest
@@ -54,10 +55,19 @@ def _system(name, matrix="f64"):
 
 
 def _warm(P, rhs):
-    """Applies often enough for the patches to serve (they do after a few applications)."""
+    """Applies until the patches serve (they do after a few applications)."""
     z = rhs.clone()
-    for _ in range(150):
+    for _ in range(400):
+        served = P.patches()[2]
         P.apply(rhs, z)
+        if P.patches()[2] > served:
+            return
+    raise AssertionError("no patches")
+
+
+def _same(a, b):
+    """The same values, NaN where the other is NaN (its sign and payload are not promised)."""
+    return bool(((a == b) | (a.isnan() & b.isnan())).all())
 
 
 def _colour_passes(A, colour, rhs, sweeps):
@@ -88,7 +98,9 @@ def test_patches_match_the_restated_colour_passes(torch_cuda, name, sweeps):
     P.setup(A)
     _warm(P, rhs)
     z = torch.full_like(rhs, float("nan"))
+    cycles, patches, served = P.patches()
     P.apply(rhs, z)
+    assert cycles >= 1 and patches >= 1 and P.patches()[2] == served + 1
     want = _colour_passes(A, P.ordering()[0], rhs.cpu().numpy(), sweeps)
     # the same 4x4 products summed in another order: ~1e2 roundings of 1e-16 per value, times the
     # blocks' condition (the bound the other preconditioner tests use)
@@ -111,12 +123,81 @@ def check_sweeps(torch, P, A, rhs, side, sweeps):
     P.setup(A)
     _warm(P, rhs)
     z, zc = torch.full_like(rhs, float("nan")), torch.full_like(rhs, float("nan"))
+    cycles, _, served = P.patches()
+    assert 0 < cycles < sweeps            # more than one launch: the scratch vector is in use
+    P.apply(rhs, z)
+    torch.cuda.synchronize()
+    assert P.patches()[2] == served + 1
+    with torch.cuda.stream(side):
+        P.apply(rhs, zc)
+    torch.cuda.synchronize()
+    assert P.patches()[2] == served + 1   # the second stream's on colour passes
+    assert _same(z, zc), sweeps
+    assert rhs.isfinite().all().item() == z.isfinite().all().item()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16"])
+@pytest.mark.parametrize("name", ["bump", "hybrid", "rcm"])
+def test_non_finite_values_equal_the_colour_passes(torch_cuda, name, prec):
+    """NaN and infinities in the right-hand side and in factor blocks spread to the same cells."""
+    import torch
+    raw, gm, A, rhs = _system(name, "f64" if prec == "f64" else "f32")
+    n = raw.nelem
+    P = fvx.Preconditioner(gm, "sgs", prec, 5)
+    side = torch.cuda.Stream()
+    rhs[n // 3, 1] = float("nan")
+    rhs[n // 2, 0] = float("inf")
+    rhs[2 * n // 3, 3] = -float("inf")
+    for sweeps in (5, 9):
+        check_sweeps(torch, P, A, rhs, side, sweeps)
+    # a state with a NaN cell and one of zero density: blocks that cannot be inverted
+    d = fvx.FlowFV(gm, fvx.physics_cfg(Minf=0.5, bcs=_bcs(raw)), fvx.numerics_cfg(flux="ROE"))
+    u = torch.tensor(states.perturbed_freestream(raw, Minf=0.5), device="cuda")
+    u[n // 4] = float("nan")
+    u[n // 5, 0] = 0.0
+    d.assemble_jacobian(u, A)
+    rhs = torch.ones_like(rhs)
+    P.setup(A)
+    _warm(P, rhs)
+    z, zc = torch.zeros_like(rhs), torch.zeros_like(rhs)
     P.apply(rhs, z)
     torch.cuda.synchronize()
     with torch.cuda.stream(side):
         P.apply(rhs, zc)
     torch.cuda.synchronize()
-    assert torch.equal(z, zc), sweeps
+    assert not z.isfinite().all() and _same(z, zc)
+
+
+def test_batches_equal_single_solves(torch_cuda):
+    """Four instances that need different numbers of Krylov iterations and steps, so that retired
+    ones leave gaps in the launches' lists, against solves of their own on fresh discretisations.
+    Each solve applies 16 sweeps several times as often as the patches need to serve; the batch's
+    launches cover all instances of its list."""
+    import torch
+    raw = meshgen.mesh_k1()
+    raw = raw.permuted(fvx.rcm_permutation(raw))
+    gm = fvx.Mesh(raw)
+    mach, aoa = np.array([0.35, 0.45, 0.55, 0.62]), np.array([0.0, 1.0, -1.0, 2.0])
+    kw = dict(cflinit=50.0, cflfin=500.0, tol=1e-3, maxiter=40, krylov_rtol=1e-3, pc_sweeps=16,
+              pc_precision="f32", jac_precision="f32")
+
+    def disc(m, a):
+        return fvx.FlowFV(gm, fvx.physics_cfg(Minf=m, aoa_deg=a, bcs=BCS),
+                          fvx.numerics_cfg(flux="ROE", gradient="NONE", order2=False))
+
+    d = disc(0.5, 0.0)
+    b = fvx.Batch(d, mach, aoa)
+    fs = torch.tensor(b.freestream(), device="cuda")
+    u = fs[:, None, :].expand(4, raw.nelem, 4).contiguous()
+    st = b.steady_solve(u, **kw)
+    assert len({s["steps"] for s in st}) > 1 and len({s["lin_iters"] for s in st}) > 1, st
+    for i in range(4):
+        di = disc(mach[i], aoa[i])
+        ui = fs[i].expand(raw.nelem, 4).contiguous()
+        si = di.steady_solve(ui, raise_on_failure=False, **kw)
+        assert si["lin_iters"] > 40
+        assert (si["steps"], si["lin_iters"]) == (st[i]["steps"], st[i]["lin_iters"])
+        assert torch.equal(u[i], ui), i
 
 
 def test_recorded_application(torch_cuda):
@@ -128,14 +209,17 @@ def test_recorded_application(torch_cuda):
     z, zg = torch.zeros_like(rhs), torch.zeros_like(rhs)
     P.apply(rhs, z)
     torch.cuda.synchronize()
+    served = P.patches()[2]
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         P.apply(rhs, zg)
-    for _ in range(3):
+    assert P.patches()[2] == served      # recorded as colour passes
+    for i in range(3):
         zg.zero_()
         g.replay()
         P.apply(rhs, z)                  # eager work between the replays
         torch.cuda.synchronize()
+        assert P.patches()[2] == served + i + 1
         assert torch.equal(z, zg)
 
 
@@ -148,6 +232,8 @@ def test_more_sweeps_after_the_setup(torch_cuda):
     _warm(P, rhs)
     fvx.check(fvx.lib().fvx_pc_set_sweeps(P.h, 9))
     z = torch.zeros_like(rhs)
+    cycles, _, served = P.patches()
     P.apply(rhs, z)
+    assert cycles == 2 and P.patches()[2] == served + 1
     want = _colour_passes(A, P.ordering()[0], rhs.cpu().numpy(), 9)
     assert np.abs(z.cpu().numpy() - want).max() <= 1e-11 * np.abs(want).max()
