@@ -78,22 +78,72 @@ def test_patches(torch_cuda, shape, order, viscous, form):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+def _same(a, b):
+    """The same values, NaN where the other is NaN (its sign and payload are not promised)."""
+    return bool(((a == b) | (a.isnan() & b.isnan())).all())
+
+
+# one patch, several, and enough cells for wave tasks
+@pytest.mark.parametrize("shape", [(16, 4, 2), (61, 23, 9), (247, 81, 0)])
+@pytest.mark.parametrize("viscous", [False, True])
+@pytest.mark.parametrize("form", FORMS + [("HLLC", "GREENGAUSS", "BARTHJESPERSEN")],
+                         ids=lambda f: f[2])
+def test_non_finite_states(torch_cuda, shape, viscous, form):
+    """Cells of NaN, infinities, zero density and negative pressure, inside and at boundaries."""
+    import torch
+    raw = meshgen.airfoil_omesh(*shape)
+    raw = raw.permuted(fvx.rcm_permutation(raw))
+    d = fvx.FlowFV(fvx.Mesh(raw), _phys(viscous), _num(*form))
+    u = torch.tensor(states.perturbed_freestream(raw, Minf=0.5, aoa_deg=1.0), device="cuda")
+    n = raw.nelem
+    u[0, 2] = float("nan")
+    u[n // 5, 1] = float("inf")
+    u[n // 4, 3] = -float("inf")
+    u[n // 3, 0] = 0.0
+    u[n // 2, 3] = 0.0
+    u[2 * n // 3] = float("nan")
+    out = []
+    for quad in (False, True):
+        if quad:
+            d.set_launch("flux", 256, True)
+        r = torch.full_like(u, 0.5)
+        dt = torch.zeros(n, dtype=torch.float64, device="cuda")
+        d.compute_residual(u, r, True, dt)
+        out.append((r, dt))
+    assert not out[0][0].isfinite().all()
+    assert _same(out[0][0], out[1][0]) and _same(out[0][1], out[1][1])
+
+
+# what a batch does by size in wave tasks: first order, WENO weights, limited viscous terms
+@pytest.mark.parametrize("viscous,form", [(False, FORMS[0]), (True, FORMS[0]), (False, FORMS[4]),
+                                          (True, FORMS[4]), (True, FORMS[1])],
+                         ids=lambda v: v if isinstance(v, bool) else v[2])
+def test_batch_in_wave_tasks(torch_cuda, viscous, form):
+    _batch(viscous, form)
+
+
 @pytest.mark.parametrize("viscous", [False, True])
 def test_batch(torch_cuda, viscous):
+    _batch(viscous, FORMS[2 if viscous else 1])
+
+
+def _batch(viscous, form):
+    """Instances of one batch in the form the library chooses for their number against single
+    evaluations in the quad form."""
     import torch
     raw = meshgen.airfoil_omesh(61, 23, 9)
     raw = raw.permuted(fvx.rcm_permutation(raw))
     n = 20000 // raw.nelem + 1
     mach, aoa = np.linspace(0.3, 0.6, n), np.linspace(-2.0, 3.0, n)
     gm = fvx.Mesh(raw)
-    d = fvx.FlowFV(gm, _phys(viscous), _num(*FORMS[2 if viscous else 1]))
+    d = fvx.FlowFV(gm, _phys(viscous), _num(*form))
     b = fvx.Batch(d, mach, aoa)
     u = torch.tensor(np.stack([states.perturbed_freestream(raw, Minf=m, aoa_deg=a, seed=i)
                                for i, (m, a) in enumerate(zip(mach, aoa))]), device="cuda")
     r, dt = torch.zeros_like(u), torch.zeros(u.shape[:2], dtype=torch.float64, device="cuda")
     b.compute_residual(u, r, True, dt)
     for i in range(n):
-        di = fvx.FlowFV(gm, _phys(viscous, mach[i], aoa[i]), _num(*FORMS[2 if viscous else 1]))
+        di = fvx.FlowFV(gm, _phys(viscous, mach[i], aoa[i]), _num(*form))
         di.set_launch("flux", 256, True)
         ri, dti = torch.zeros_like(u[i]), torch.zeros_like(dt[i])
         di.compute_residual(u[i].contiguous(), ri, True, dti)

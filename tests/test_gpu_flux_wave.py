@@ -1,6 +1,6 @@
 """The wave-task form of the face-flux pass against the oracle.
 
-Each wave64 owns a group of consecutive cells whose faces make at most 64 tasks and evaluates
+Each wave64 owns a group of neighbouring cells whose faces make at most 64 tasks and evaluates
 every face touching them once (an internal face for both cells); each cell sums its four face
 slots in the quad-per-cell form's order. It applies to inviscid first-order and linear
 reconstruction. Checked against the oracle's residual (per cell within 1e-12 of the local flux
@@ -8,8 +8,9 @@ scale) and time steps: on the bump for every flux (second order with the Venkata
 and first order), on the airfoil in RCM, Hilbert and natural order, for a batch of operating
 points against single evaluations, and bitwise reproducible run to run. Both forms evaluate each
 face flux from the face's left and right states and sum a cell's four slots in the same order,
-so their residuals and time steps are bitwise equal; the library selects the wave form by itself
-where it applies and the cell order packs at least 24 cells per group.
+so their residuals and time steps are bitwise equal. Where a caller may select the wave form and the
+cell order packs at least 24 cells per group, a new discretisation reports it as selected (what
+the library runs of its own choice is tested in test_gpu_flux_groups.py).
 """
 import numpy as np
 import pytest
@@ -129,6 +130,7 @@ def test_wave_and_quad_forms_are_bitwise_equal_on_the_airfoil(torch_cuda):
 
 
 def test_the_form_is_selected_by_the_cell_order(torch_cuda):
+    """What fvx_get_launch reports of the wave form on a new discretisation."""
     raw = meshgen.mesh_k2()
     num = dict(flux="HLLC", gradient="LEASTSQUARES", recon="VENKATAKRISHNAN")
     phys = dict(Minf=0.8, aoa_deg=1.25, bcs=AIRFOIL_BCS)
@@ -157,8 +159,8 @@ def test_the_form_is_selected_by_the_cell_order(torch_cuda):
 def test_full_size_hilbert_workload_matches_the_oracle(torch_cuda):
     """The benchmark's residual workload at its full size: the 2048x512 O-mesh (1,572,864 cells)
     in Hilbert order, HLLC + weighted least squares + Venkatakrishnan K=5 at M0.8, 1.25 deg.
-    The library selects the wave-task form by itself; its residual and time steps match the
-    oracle per cell (1e-12 of the local flux scale), repeat bitwise, and equal the quad form's
+    The library does it in one launch; residual and time steps match the oracle per cell (1e-12
+    of the local flux scale), repeat bitwise, and equal the wave-task form's and the quad form's
     bitwise."""
     import torch
     raw = meshgen.mesh_k2l()
@@ -167,7 +169,7 @@ def test_full_size_hilbert_workload_matches_the_oracle(torch_cuda):
     phys = dict(Minf=0.8, aoa_deg=1.25, bcs=AIRFOIL_BCS)
     num = dict(flux="HLLC", gradient="LEASTSQUARES", recon="VENKATAKRISHNAN", limiter_param=5.0)
     disc = fvx.FlowFV(fvx.Mesh(raw), fvx.physics_cfg(**phys), fvx.numerics_cfg(**num))
-    assert disc.get_launch("flux_wave")[0] == 64
+    assert disc.get_launch("flux_wave")[0] == 64 and disc.get_launch("residual")[0] == 256
     ut = torch.tensor(u, device="cuda")
 
     def evaluate():
@@ -186,6 +188,10 @@ def test_full_size_hilbert_workload_matches_the_oracle(torch_cuda):
     rel = np.abs(r1.cpu().numpy() - r_ref) / scale
     assert rel.max() <= 1e-12, rel.max()
     assert np.allclose(dt1.cpu().numpy(), dt_ref, rtol=1e-12, atol=0)
+    disc.set_launch("flux_wave", 64, True)
+    assert disc.get_launch("residual")[0] == 0
+    rw, dtw = evaluate()
+    assert torch.equal(r1, rw) and torch.equal(dt1, dtw)
     disc.set_launch("flux", 256, True)
     assert disc.get_launch("flux_wave")[0] == 0
     rq, dtq = evaluate()
