@@ -47,6 +47,9 @@ struct BatchArg {
 /// Tables of the one-launch residual (residual_patch.hpp), on the device.
 constexpr int PATCH_TASKS = 256;      ///< face tasks, and threads, per patch
 constexpr int PATCH_MAX = 256;        ///< patch and halo cells
+// LDS of a workgroup: states of the listed cells and of at most four further ones of each, centre
+// and gradient of the listed ones; within the limit of a launch that asks for no more
+static_assert((4*5*PATCH_MAX + 10*PATCH_MAX)*sizeof(double) <= 65536, "patches exceed the LDS");
 struct PatchGroup {
 	int list, nown, nlist, nstate;     ///< first entry in cells; patch cells, those and halo, all entries
 	int local, slots;                  ///< first entries in local and slots

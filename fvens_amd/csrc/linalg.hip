@@ -598,7 +598,7 @@ void k_bj_ilu_apply(const int* __restrict__ bptr, const int* __restrict__ blvptr
 constexpr int RED_BLOCKS = 512;
 constexpr int MAX_DOTS = 32;
 constexpr long PART = (long)RED_BLOCKS*MAX_DOTS;   // per-instance partial-sum stride
-constexpr int FOLD_BLOCKS = 512;                   // see fold()
+constexpr long FOLD_READERS = 4096;                // see fold()
 
 /// Sum over the 256 threads of a block; the result is valid in every thread.
 __device__ __forceinline__ double block_sum(double v, double* sh)
@@ -1186,17 +1186,14 @@ static inline int red_blocks(long N)
 {
 	return (int)std::max(1L, std::min((long)RED_BLOCKS, (N + BLOCK - 1)/BLOCK));
 }
-/// Whether the workgroups that read a reduction's result add its nblk partials themselves (all of
-/// them the same sum) instead of a launch of its own: a launch is ~2.7 us, the partials are
-/// 8 nv nblk bytes for each of `readers` workgroups. With the least squares and the normalisation
-/// in one launch, a pseudo-step's linear algebra takes 320 us instead of 388 on 4,608 cells (6
-/// iterations), 430 instead of 458 on 98,304 (3); up to 64 partials only, 333 and 437. Adding
-/// them in the last workgroup to finish (a fence in each) costs more than it saves from 384
-/// workgroups on.
-static inline bool fold(int nblk, int readers, int nact)
-{
-	return nblk <= FOLD_BLOCKS && (long)readers*nact <= 8L*FOLD_BLOCKS;
-}
+/// Whether the workgroups that read a reduction's result add its partials (at most RED_BLOCKS)
+/// themselves (all of them the same sum) instead of a launch of its own: a launch is ~2.7 us, the
+/// partials are 8 nv nblk bytes for each of `readers` workgroups per instance. With the least squares
+/// and the normalisation in one launch, a pseudo-step's linear algebra takes 320 us instead of 388 on
+/// 4,608 cells (6 iterations), 430 instead of 458 on 98,304 (3); up to 64 partials only, 333 and
+/// 437. Adding them in the last workgroup to finish (a fence in each) costs more than it saves
+/// from 384 workgroups on.
+static inline bool fold(int readers, int nact) { return (long)readers*nact <= FOLD_READERS; }
 
 static void mdot(long N, const double* V, long ldv, long sv, int nv, const double* w, long sw,
                  double* partial, const Inst& L, hipStream_t s)
@@ -1266,7 +1263,7 @@ void launch_arnoldi(long N, const fvx_matrix_s* A, const double* z, long sz, con
 		if(A) launch_spmv(*A, z, sz, w, sw, L, s);
 		mdot(N, V, ldv, sv, nv, w, sw, partial, L, s);
 	}
-	const bool f = fold(nblk, nblk, L.nact);
+	const bool f = fold(nblk, L.nact);
 	if(!f) reduce(nblk, partial, nv, h, sh, L, s);
 	hipLaunchKernelGGL(k_gs_update, dim3(nblk, L.nact), dim3(BLOCK), 0, s, N, L.list, V,
 	                   ldv, sv, nv, partial, f ? nblk : 0, h, sh, w, sw, npart);
@@ -1437,8 +1434,7 @@ void launch_scale_rotate(long N, const double* b, long sb, const double* npart, 
                          hipStream_t s)
 {
 	const int nblk = red_blocks(N), readers = stream_blocks(N);
-	// unlike the dots, a norm's partials are few enough for more workgroups to read
-	const bool f = (long)readers*L.nact <= 8L*FOLD_BLOCKS;
+	const bool f = fold(readers, L.nact);
 	if(!f) {
 		hipLaunchKernelGGL(k_reduce_norm, dim3(1, L.nact), dim3(64), 0, s, nblk, L.list, npart,
 		                   scal + slot, ns);

@@ -204,8 +204,6 @@ void build_mesh(fvx_mesh_s& m, const fvx_mesh_desc& d)
 	m.d_wgroup.upload(wt.groups);
 	if(!m.wave_order) m.d_wcell.upload(wt.cells);
 	m.d_wslot.upload(wt.slots);
-	// the default limit of a workgroup's LDS (never met with PATCH_MAX cells of ordinary meshes)
-	if((4*(size_t)pt.nwmax + 10*(size_t)pt.nsmax)*sizeof(double) > 65536) return;
 	m.npatch = (int)pt.groups.size();
 	m.patch_nw = pt.nwmax;
 	m.patch_ns = pt.nsmax;

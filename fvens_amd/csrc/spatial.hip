@@ -366,7 +366,7 @@ void launch_residual(const fvx_disc_s& d, const double* u, double* r, int gettim
 	// weights, which need the neighbours' gradients, nor viscous terms with a limiter, which need
 	// two gradients per cell. Faster than the separate passes from 4,608 cells (9 against 13 us) to
 	// 1,572,864 (176 against 207).
-	if(order2 && d.tune.flux_group && m.npatch > 0 && rec != FVX_RECON_WENO) {
+	if(order2 && d.tune.flux_group && rec != FVX_RECON_WENO) {
 		const int lim = rec == FVX_RECON_VENKATAKRISHNAN ? 1 : rec == FVX_RECON_BARTHJESPERSEN ? 2 : 0;
 		if(!(visc && lim)) {
 			const PatchTables pt = { m.d_pgroup.p, m.d_pcell.p, m.d_plocal.p, m.d_pface.p, m.d_psides.p,
