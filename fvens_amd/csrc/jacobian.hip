@@ -248,7 +248,8 @@ template <> __device__ __forceinline__ void store_row<float>(float* p, const dou
 /// src/ode/aodesolver.cpp:300-329).
 ///
 /// Bound by FP64 VALU work and its latency: ~1,000 instructions a face and side at two waves per
-/// SIMD (204-228 registers). One lane differentiating both sides in turn, all variables duals,
+/// SIMD (204-228 registers; viscous up to 255, HLL and LLF spill 44 bytes a lane: 60 and 55 us on
+/// 98,304 cells, 75 and 71 with both sides on a lane). One lane differentiating both sides in turn, all variables duals,
 /// needed 290-380 registers and spilled. Assembly on 98,304 cells, FP64, workgroups of 64: Roe
 /// 120 -> 43 us, HLLC 74 -> 44 us; 4,608 cells, workgroups of 256: Roe 25 -> 12 us, HLLC 19 -> 12
 /// us. Held to three waves per SIMD, HLLC spills 140 bytes (48 us). Boundary faces go column by

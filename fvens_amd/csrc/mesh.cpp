@@ -979,8 +979,10 @@ void build_disc(fvx_disc_s& d)
 	// is compact
 	d.tune.flux_wave = flux_wave_apply(d) && m.wave_order;
 	// Jacobian assembly: workgroups of one wave (both sides of a face in turn) where they fill the
-	// chip several times over, else a pair of waves per 16 cells (98,304 cells 43 against 50 us,
-	// 4,608 cells 15 against 12 us; Roe)
+	// chip several times over, else a pair of waves per 16 cells. Roe, FP64, one wave against pairs:
+	// 4,704 cells 10.4 and 9.1 us, 18,816 15.7 and 15.0, 24,576 16.6 and 16.3, 31,104 16.7 and 18.6,
+	// 38,400 20.5 and 20.9, 98,304 36 and 44 (HLLC and FP32 values alike). The mesh decides, also for
+	// batches, whose size the discretisation does not know.
 	d.tune.jac_block = m.nelem >= 32768 ? 64 : 256;
 }
 

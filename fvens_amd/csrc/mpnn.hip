@@ -342,8 +342,10 @@ __device__ __forceinline__ void update_bwd_tile(const bf16x8* wf, float* t, int 
 /// Bound by HBM and the gathers: per row h 256 + Q about 256 + edges 80 read, h 256 + Q 256
 /// (+ 168 in training) written. P|Q written by a launch of its own and read back took 565 us per
 /// layer on 786,432 rows (117 + 449), this takes 277 (1.1 GB, 77% of the copy rate). Three workgroups a
-/// compute unit, two (by LDS) for LAST in training, which takes 345 us with the decoder and its
-/// backward pass (in launches of their own 620: 277 + 198 + 152).
+/// compute unit (168 registers; in inference 52 bytes a lane spill, 56 in LAST), two (by LDS) for LAST
+/// in training, which takes 345 us with the decoder and its backward pass (in launches of their own
+/// 620: 277 + 198 + 152). One graph of 98,304 cells, 34 us a layer: two tiles a wave, too few to hide
+/// the gathers.
 template <bool TRAIN, bool LAST>
 __global__ void __launch_bounds__(RB, TRAIN && LAST ? 2 : 3)
 k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict__ q,
@@ -553,8 +555,9 @@ k_layer(Graph g, int ntile, const float* __restrict__ h, const float* __restrict
 /// Bound by HBM and the gathers of da: per row da 256 + about 256 + masks 64 + edges 80 + gpart 256
 /// read, dP|dQ 256 + dpre 128 + gpart 256 + da 256 written. Three launches that recomputed the
 /// messages from P|Q took 1,148 us per layer on 786,432 rows (790 + 166 + 192), this takes 403
-/// (1.5 GB, 71% of the copy rate). Three waves per SIMD: with the sums of dWe and dbm kept per lane
-/// and row (80 registers) instead of added over the rows of each tile, two waves took 565.
+/// (1.5 GB, 71% of the copy rate). Three waves per SIMD, with 36 bytes a lane of spills (none in
+/// FIRST): with the sums of dWe and dbm kept per lane and row (80 registers) instead of added over the
+/// rows of each tile, two waves took 565.
 template <bool FIRST>
 __global__ void __launch_bounds__(RB, 3) k_layer_bwd(Graph g, int ntile,
                                                      const float* __restrict__ da,

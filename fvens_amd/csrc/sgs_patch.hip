@@ -81,9 +81,14 @@ template <> struct FacRow<bf16> : FacRow<float> {
 /// too). halo[p][h] = the cells only read (-1: none). Slots are in colour order, so that a wave
 /// whose cells are all of another colour skips the pass.
 ///
-/// Bound by FP64 VALU work and LDS reads within a pass (0.3 us at least: barrier, LDS and FMA
-/// latency), between launches by reading the factors once per launch (~7 TB/s). Launches of 3
-/// sweeps take ~18 us on 98,304 cells with FP32 factors (13 colour passes: 58 us).
+/// Bound by the read of the factors of patch and rim (2.04 cells for one of the patch's own on 98,304
+/// cells at three sweeps), beside which nothing runs: a workgroup fills its compute unit, loads its
+/// rows, then makes the passes. A launch of three sweeps moves 55 MB with FP32 factors and takes
+/// 16.9 us, 34 MB and 10.5 us with bfloat16, one of two sweeps 92 MB and 21 us with FP64: 10.6, 6.6
+/// and 18 us of it at the rate of a large copy. The rest is the chain of passes (0.3 us each at
+/// least: barrier, LDS and FMA latency; VALU issue 4 us, LDS 2 us in all) and the launch. 13 colour
+/// passes take 58 us with FP32 factors. Sixteen instances read 503 MB of FP32 factors without any
+/// rim, 98 us at that rate; a launch takes 111.
 template <class VTF, int NQ, int K, bool FIRST>
 __global__ __launch_bounds__(4*NQ)
 void k_sgs_patch(int npass, int ncol, const uint4* __restrict__ rec,
@@ -526,12 +531,12 @@ void tables(const fvx_pc_s& p, int most, hipStream_t s)
 	});
 }
 
-/// Whether this application runs on the patches. The tables (made on the host: 8 ms for 98,304
-/// cells, 2-4 ms for 4,608) are made once the handle's applications have taken about as long by
-/// colour passes as that takes, so that a preconditioner used a few times does not pay for
-/// them; until then, and where the device has no memory for them, the colour passes serve. The
-/// scratch vector of applications of more than one launch serves one stream between two set-ups,
-/// and no recorded graph.
+/// Whether this application runs on the patches. The tables (made on the host: 2-4 ms for 4,608
+/// cells, 8 ms for 98,304, 150-190 ms for 1,572,864) are made once the handle's applications have
+/// taken about as long by colour passes as that takes, so that a preconditioner used a few times
+/// does not pay for them; until then, and where the device has no memory for them, the colour passes
+/// serve. The scratch vector of applications of more than one launch serves one stream between two
+/// set-ups, and no recorded graph.
 bool ready(const fvx_pc_s& p, size_t value, int nact, hipStream_t s)
 {
 	if(!possible(p, s)) return false;

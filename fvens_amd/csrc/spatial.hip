@@ -364,8 +364,8 @@ void launch_residual(const fvx_disc_s& d, const double* u, double* r, int gettim
 	const double* ug = nullptr;
 	// gradients and fluxes in one launch (residual_patch.hpp) unless a form was selected; not for WENO
 	// weights, which need the neighbours' gradients, nor viscous terms with a limiter, which need
-	// two gradients per cell. Faster than the separate passes from 4,608 cells (9 against 13 us) to
-	// 1,572,864 (176 against 207).
+	// two gradients per cell. Faster than the separate passes at every size measured: 192 cells 8
+	// against 15 us, 33,600 9 against 15, 393,216 41 against 51, 1,572,864 176 against 207.
 	if(order2 && d.tune.flux_group && rec != FVX_RECON_WENO) {
 		const int lim = rec == FVX_RECON_VENKATAKRISHNAN ? 1 : rec == FVX_RECON_BARTHJESPERSEN ? 2 : 0;
 		if(!(visc && lim)) {
