@@ -55,11 +55,6 @@ __device__ __forceinline__ bf16x8 to_frag(const float* v)
 	const u32x4 u = { pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]) };
 	return __builtin_bit_cast(bf16x8, u);
 }
-__device__ __forceinline__ bf16x8 zero_frag()
-{
-	const u32x4 u = { 0u, 0u, 0u, 0u };
-	return __builtin_bit_cast(bf16x8, u);
-}
 __device__ __forceinline__ void load8(const float* p, float* v)
 {
 	const f32x4 a = *reinterpret_cast<const f32x4*>(p);
